@@ -1,0 +1,44 @@
+/*
+ * miniep_amd_model.h -- the part of the C ABI that the transformer around the
+ * MoE block calls (the MoE block itself: miniep_amd.h, whose conventions on
+ * pointers, streams, return codes and dtypes hold here too).
+ */
+#ifndef MINIEP_AMD_MODEL_H
+#define MINIEP_AMD_MODEL_H
+
+#include "miniep_amd.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* ------------------------------------------------------------------------
+ * The transformer around the MoE block (modeling.py:55-80,146-197).
+ *
+ * mep_add_norm: h_out = h + round(delta * mult) with each step rounded to
+ * `dtype` (delta NULL: h_out is not written and stands for h), x_out =
+ * weight * (h_out / sqrt(mean(h_out^2) + eps)) in fp32, rounded to `dtype`.
+ * h_out may be h.  (n_rows, hidden) rows, hidden a multiple of 16 bytes, at
+ * most 4096.
+ *
+ * mep_attention: rotate-half RoPE of q and k at positions start .. start+t-1
+ * of the tables cos / sin (n_positions, head_dim) fp32; rotated keys and the
+ * values go into the caches (batch, n_kv_heads, max_len, head_dim) fp32 at
+ * those positions, and query i of each sequence attends positions 0 ..
+ * start+i (scores times `scale`), all in fp32.  q (batch*t, n_heads*head_dim),
+ * k / v (batch*t, n_kv_heads*head_dim), out like q, in `dtype`.
+ * Supported: head_dim 64, n_heads / n_kv_heads in {1, 2, 4}.  One launch for
+ * t = 1, two otherwise.
+ * ---------------------------------------------------------------------- */
+int mep_add_norm(const void* h, const void* delta, float mult, const void* weight, float eps,
+                 int64_t n_rows, int32_t hidden, int32_t dtype, void* h_out, void* x_out, void* stream);
+
+int mep_attention(const void* q, const void* k, const void* v, const float* cos, const float* sin,
+                  int64_t n_positions, int32_t batch, int32_t t, int32_t n_heads, int32_t n_kv_heads,
+                  int32_t head_dim, int64_t start, int64_t max_len, float scale, int32_t dtype,
+                  float* k_cache, float* v_cache, void* out, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* MINIEP_AMD_MODEL_H */

@@ -1,0 +1,574 @@
+// The transformer around the MoE block (gfx950): residual adds and RMSNorm,
+// rotary embedding with the KV cache, causal attention, and the projections of
+// small batches.
+//
+// Replaces, in the reference's model (modeling.py):
+//   RMSNorm                                      :55-63
+//   rotate-half RoPE                             :66-80
+//   GQA attention over the KV cache, fp32        :146-185
+//   the scaled residual adds of Block.forward    :186-197
+//   q/k/v/o projections and the LM head          :160-185, :249-254
+// Activations are bf16 or fp32; scores, softmax and the attention sums are
+// fp32, keys and values are kept in fp32.  Every rounding of the layer-by-layer
+// computation is kept where a tensor of the model's dtype is defined: x after
+// the norm, a projection's output, the scaled residual term, the residual sum.
+#include "../../include/miniep_amd_model.h"
+#include "common.h"
+
+#include <type_traits>
+
+namespace mep {
+namespace {
+
+constexpr float kLog2e = 1.4426950408889634f;
+
+template <int DT>
+__device__ __forceinline__ void unpack_chunk(const u32x4& v, float* f) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  if constexpr (DT == MEP_DTYPE_BF16) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      f[2 * q] = bf16_to_f32(static_cast<uint16_t>(w[q] & 0xffffu));
+      f[2 * q + 1] = bf16_to_f32(static_cast<uint16_t>(w[q] >> 16));
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) f[q] = __uint_as_float(w[q]);
+  }
+}
+
+template <int DT>
+__device__ __forceinline__ u32x4 pack_chunk(const float* f) {
+  u32x4 o;
+  if constexpr (DT == MEP_DTYPE_BF16) {
+    o.x = pack_bf16x2(f[0], f[1]);
+    o.y = pack_bf16x2(f[2], f[3]);
+    o.z = pack_bf16x2(f[4], f[5]);
+    o.w = pack_bf16x2(f[6], f[7]);
+  } else {
+    o.x = __float_as_uint(f[0]);
+    o.y = __float_as_uint(f[1]);
+    o.z = __float_as_uint(f[2]);
+    o.w = __float_as_uint(f[3]);
+  }
+  return o;
+}
+
+// f rounded to the storage type and back
+template <int DT>
+__device__ __forceinline__ float rounded(float f) {
+  if constexpr (DT == MEP_DTYPE_BF16) return bf16_to_f32(f32_to_bf16(f));
+  else return f;
+}
+
+// h + round(delta * mult), the residual step (no contraction: the product is
+// a tensor of its own in the layer-by-layer computation)
+template <int DT>
+__device__ __forceinline__ float residual(float h, float delta, float mult) {
+#pragma clang fp contract(off)
+  const float step = rounded<DT>(delta * mult);
+  return rounded<DT>(h + step);
+}
+
+// ============================================================================
+// Residual add + RMSNorm: h_out = h + round(delta * mult) (delta NULL: h), x =
+// weight * (h_out / sqrt(mean(h_out^2) + eps)).  One wave per row, the row in
+// registers (NCH 16-byte chunks per lane), so h and delta are read once and
+// h_out and x written once.  Bound by those bytes for many rows (2048 rows of
+// 1024 in bf16: 16.8 MB in 5.8 us), by the launch for a few (8 rows: 3.8 us);
+// as torch operations the same step was nine launches.
+// ============================================================================
+constexpr int kNormWaves = 4;
+
+template <int DT, int NCH>
+__global__ __launch_bounds__(kNormWaves * 64) void add_norm_kernel(const typename Elem<DT>::T* __restrict__ h,
+                                                                   const typename Elem<DT>::T* __restrict__ delta,
+                                                                   float mult,
+                                                                   const typename Elem<DT>::T* __restrict__ weight,
+                                                                   float eps, int64_t n, int hidden,
+                                                                   typename Elem<DT>::T* __restrict__ h_out,
+                                                                   typename Elem<DT>::T* __restrict__ x_out) {
+  constexpr int EPC = 16 / Elem<DT>::kBytes;
+  const int lane = lane_id();
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * kNormWaves + (threadIdx.x >> 6);
+  if (row >= n) return;
+  const int64_t base = row * hidden;
+  const int chunks = hidden / EPC;
+  u32x4 hv[NCH], dv[NCH], wv[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int q = c * 64 + lane;
+    if (q >= chunks) continue;
+    hv[c] = *reinterpret_cast<const u32x4*>(h + base + q * EPC);
+    if (delta != nullptr) dv[c] = *reinterpret_cast<const u32x4*>(delta + base + q * EPC);
+    wv[c] = *reinterpret_cast<const u32x4*>(weight + q * EPC);
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int q = c * 64 + lane;
+    if (q >= chunks) continue;
+    float f[EPC];
+    unpack_chunk<DT>(hv[c], f);
+    if (delta != nullptr) {
+      float d[EPC];
+      unpack_chunk<DT>(dv[c], d);
+#pragma unroll
+      for (int i = 0; i < EPC; ++i) f[i] = residual<DT>(f[i], d[i], mult);
+      hv[c] = pack_chunk<DT>(f);
+      *reinterpret_cast<u32x4*>(h_out + base + q * EPC) = hv[c];
+    }
+#pragma unroll
+    for (int i = 0; i < EPC; ++i) ss += f[i] * f[i];
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) ss += __shfl_xor(ss, d, 64);
+  const float r = rsqrtf(ss / static_cast<float>(hidden) + eps);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int q = c * 64 + lane;
+    if (q >= chunks) continue;
+    float f[EPC], w[EPC];
+    unpack_chunk<DT>(hv[c], f);
+    unpack_chunk<DT>(wv[c], w);
+#pragma unroll
+    for (int i = 0; i < EPC; ++i) f[i] = w[i] * (f[i] * r);
+    *reinterpret_cast<u32x4*>(x_out + base + q * EPC) = pack_chunk<DT>(f);
+  }
+}
+
+// ============================================================================
+// Rotary embedding and attention, head size 64.
+// ============================================================================
+constexpr int kHead = 64;
+
+struct AttnParams {
+  const void* q;            // (batch * t, hq * 64) projections, before RoPE
+  const void* k;            // (batch * t, hk * 64)
+  const void* v;            // (batch * t, hk * 64)
+  const float* cos;         // (max positions, 64), the two halves equal
+  const float* sin;
+  float* kc;                // (batch, hk, max_len, 64): keys after RoPE
+  float* vc;                // (batch, hk, max_len, 64)
+  void* out;                // (batch * t, hq * 64)
+  int batch, t, hq, hk;
+  int start;                // positions in the cache before this call; token i is position start + i
+  int64_t max_len;
+  float scale;
+};
+
+// The rotated value of element c of a head whose projections start at `head`:
+// element c pairs with c +- 32, the first half with the negative sign.
+template <int DT>
+__device__ __forceinline__ float rope(const typename Elem<DT>::T* head, int c, const float* cos, const float* sin) {
+  const float x = Elem<DT>::to_f32(head[c]);
+  const float y = Elem<DT>::to_f32(head[c < kHead / 2 ? c + kHead / 2 : c - kHead / 2]);
+  return x * cos[c] + (c < kHead / 2 ? -y : y) * sin[c];
+}
+
+// Keys (rotated) and values of the call's tokens into the cache: one thread
+// per 4 elements of a (token, kv head).
+template <int DT>
+__global__ __launch_bounds__(256) void kv_write_kernel(AttnParams p) {
+  typedef typename Elem<DT>::T T;
+  constexpr int C4 = kHead / 4;
+  const int64_t q = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t total = static_cast<int64_t>(p.batch) * p.t * p.hk * C4;
+  if (q >= total) return;
+  const int c = static_cast<int>(q % C4) * 4;
+  const int64_t th = q / C4;                              // token * hk + head
+  const int head = static_cast<int>(th % p.hk);
+  const int64_t tok = th / p.hk;
+  const int b = static_cast<int>(tok / p.t), i = static_cast<int>(tok % p.t);
+  const int64_t src = th * kHead, pos = p.start + i;
+  const T* const k = static_cast<const T*>(p.k) + src;
+  const T* const v = static_cast<const T*>(p.v) + src;
+  const float* const cs = p.cos + pos * kHead;
+  const float* const sn = p.sin + pos * kHead;
+  f32x4 kr, vr;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    kr[j] = rope<DT>(k, c + j, cs, sn);
+    vr[j] = Elem<DT>::to_f32(v[c + j]);
+  }
+  const int64_t dst = ((static_cast<int64_t>(b) * p.hk + head) * p.max_len + pos) * kHead + c;
+  *reinterpret_cast<f32x4*>(p.kc + dst) = kr;
+  *reinterpret_cast<f32x4*>(p.vc + dst) = vr;
+}
+
+// Attention of more than one query per sequence, causal and aligned to the
+// last key (query i of the call sees keys 0 .. start + i), fp32 on the matrix
+// cores.  A workgroup is 64 queries of one head, 4 waves of 16; keys and
+// values pass through LDS 64 at a time, the next block's loads in flight
+// during a block's MFMAs.  With S^T = K Q^T a lane holds 4 keys of one query
+// (C layout: rows 4 g + i, column r), which is the B operand that O^T =
+// V^T P^T wants when MFMA i takes keys 4 g + i: the probabilities never leave
+// their lane.  LDS rows are padded to 68 floats, which spreads both the
+// 16-byte key reads and the 4-byte value reads over all banks.  Bound by the
+// fp32 MFMAs (32 per wave, 16 keys and 16 queries) and the waits around the
+// two barriers of a block.  8 sequences of 256 tokens, 16 heads: 28.6 us, and
+// 4.6 us for the cache write, against 49 us for torch's fp32 attention after
+// a dozen launches of rotation, cache copy and head repetition.
+constexpr int kFlashQ = 64, kFlashK = 64, kFlashRow = kHead + 4;
+
+template <int DT>
+__global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
+  typedef typename Elem<DT>::T T;
+  __shared__ __attribute__((aligned(16))) float s_k[kFlashK * kFlashRow];
+  __shared__ __attribute__((aligned(16))) float s_v[kFlashK * kFlashRow];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int q0 = (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x)) * kFlashQ;   // longest rows first
+  const int head = static_cast<int>(blockIdx.y) % p.hq, b = static_cast<int>(blockIdx.y) / p.hq;
+  const int kv = head / (p.hq / p.hk);
+  const int S = p.start + p.t;
+  const float* const kc = p.kc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
+  const float* const vc = p.vc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
+
+  // this lane's query: elements 16 j + 4 g .. + 3, rotated and scaled (rows
+  // past the end repeat the last query and are not stored)
+  const int qi = q0 + wave * 16 + r;
+  const int qrow = min(qi, p.t - 1);
+  const int qpos = p.start + qrow;
+  f32x4 q[4];
+  {
+    const T* const src = static_cast<const T*>(p.q) + (static_cast<int64_t>(b) * p.t + qrow) * p.hq * kHead + head * kHead;
+    const float* const cs = p.cos + static_cast<int64_t>(qpos) * kHead;
+    const float* const sn = p.sin + static_cast<int64_t>(qpos) * kHead;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[j][i] = rope<DT>(src, 16 * j + 4 * g + i, cs, sn);
+  }
+  const float sc = p.scale * kLog2e;
+
+  // block of 64 keys: thread moves 16 floats of row tid / 4 (K and V)
+  const int lrow = tid >> 2, lcol = (tid & 3) * 16;
+  f32x4 kr[4], vr[4];
+  auto load = [&](int k0) {
+    const int64_t row = min(k0 + lrow, S - 1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      kr[j] = *reinterpret_cast<const f32x4*>(kc + row * kHead + lcol + 4 * j);
+      vr[j] = *reinterpret_cast<const f32x4*>(vc + row * kHead + lcol + 4 * j);
+    }
+  };
+  const int k_end = min(S, p.start + q0 + kFlashQ);       // keys the workgroup's last query sees
+  float m = -__builtin_inff(), l = 0.0f;
+  f32x4 o[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  load(0);
+  for (int k0 = 0; k0 < k_end; k0 += kFlashK) {
+    __syncthreads();                                      // the previous block's reads are done
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      *reinterpret_cast<f32x4*>(s_k + lrow * kFlashRow + lcol + 4 * j) = kr[j];
+      *reinterpret_cast<f32x4*>(s_v + lrow * kFlashRow + lcol + 4 * j) = vr[j];
+    }
+    __syncthreads();
+    if (k0 + kFlashK < k_end) load(k0 + kFlashK);
+    f32x4 s[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4 kf[4];
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+        kf[kt] = *reinterpret_cast<const f32x4*>(s_k + (16 * kt + r) * kFlashRow + 16 * j + 4 * g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+          s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kt][i], q[j][i], s[kt], 0, 0, 0);
+    }
+    float mb = m;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kt][i] = k0 + 16 * kt + 4 * g + i <= qpos ? s[kt][i] * sc : -__builtin_inff();
+        mb = fmaxf(mb, s[kt][i]);
+      }
+    mb = fmaxf(mb, __shfl_xor(mb, 16, 64));
+    mb = fmaxf(mb, __shfl_xor(mb, 32, 64));               // finite: key 0 is in the first block and seen by all
+    const float alpha = __builtin_amdgcn_exp2f(m - mb);
+    m = mb;
+    l *= alpha;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[d][i] *= alpha;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - m);
+        l += s[kt][i];
+      }
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_v[(16 * kt + 4 * g + i) * kFlashRow + 16 * d + r], s[kt][i], o[d],
+                                                     0, 0, 0);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (qi >= p.t) return;
+  T* const dst = static_cast<T*>(p.out) + (static_cast<int64_t>(b) * p.t + qi) * p.hq * kHead + head * kHead;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const float v[4] = {o[d][0] / l, o[d][1] / l, o[d][2] / l, o[d][3] / l};
+    if constexpr (DT == MEP_DTYPE_BF16)
+      *reinterpret_cast<uint2*>(dst + 16 * d + 4 * g) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    else
+      *reinterpret_cast<f32x4*>(dst + 16 * d + 4 * g) = f32x4{v[0], v[1], v[2], v[3]};
+  }
+}
+
+// Attention of one new token per sequence (decode).  A workgroup of 16 waves
+// is one (sequence, kv head) with its G query heads, so keys and values are
+// read once for the group.  It rotates the new key, writes it and the value
+// to the cache, and walks the cached positions kDecKeys at a time: scores to
+// LDS (16 lanes per key, 16 bytes each, so a wave reads four whole keys per
+// instruction), the chunk's maximum and sum, then the values with the same
+// lane layout.  The sums of the 64 key groups meet in LDS in a fixed order.
+// Bound by one CU's loads and the chunk's barriers: 8 sequences of 513
+// positions, 8 kv heads (16.8 MB of cache): 14.1 us, against 46 us for torch's
+// fp32 attention alone.
+constexpr int kDecWaves = 16, kDecKeys = 2048;
+constexpr int kDecUnroll = 4;
+
+template <int DT, int G>
+__global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnParams p) {
+  typedef typename Elem<DT>::T T;
+  __shared__ __attribute__((aligned(16))) float s_q[G][kHead];
+  __shared__ __attribute__((aligned(16))) float s_new[2][kHead];     // the new token's key and value
+  __shared__ float s_p[G][kDecKeys];
+  __shared__ float s_red[kDecWaves][G];
+  __shared__ __attribute__((aligned(16))) float s_o[kDecWaves][G][kHead];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 15, g = lane >> 4;
+  const int kv = static_cast<int>(blockIdx.x) % p.hk, b = static_cast<int>(blockIdx.x) / p.hk;
+  const int pos = p.start, S = pos + 1;
+  float* const kc = p.kc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
+  float* const vc = p.vc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
+  {
+    const float* const cs = p.cos + static_cast<int64_t>(pos) * kHead;
+    const float* const sn = p.sin + static_cast<int64_t>(pos) * kHead;
+    if (tid < G * kHead) {
+      const T* const src = static_cast<const T*>(p.q) + (static_cast<int64_t>(b) * p.hq + kv * G + tid / kHead) * kHead;
+      s_q[tid / kHead][tid % kHead] = rope<DT>(src, tid % kHead, cs, sn) * (p.scale * kLog2e);
+    } else if (tid < (G + 1) * kHead) {
+      const int e = tid - G * kHead;
+      const float k = rope<DT>(static_cast<const T*>(p.k) + (static_cast<int64_t>(b) * p.hk + kv) * kHead, e, cs, sn);
+      s_new[0][e] = k;
+      kc[static_cast<int64_t>(pos) * kHead + e] = k;
+    } else if (tid < (G + 2) * kHead) {
+      const int e = tid - (G + 1) * kHead;
+      const float v = Elem<DT>::to_f32(static_cast<const T*>(p.v)[(static_cast<int64_t>(b) * p.hk + kv) * kHead + e]);
+      s_new[1][e] = v;
+      vc[static_cast<int64_t>(pos) * kHead + e] = v;
+    }
+  }
+  __syncthreads();
+  f32x4 q[G];
+#pragma unroll
+  for (int h = 0; h < G; ++h) q[h] = *reinterpret_cast<const f32x4*>(&s_q[h][4 * c]);
+  // 16 bytes of position s: from the cache, or the new token's from LDS
+  auto row = [&](const float* cache, int which, int s) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(cache + static_cast<int64_t>(min(s, max(pos - 1, 0))) * kHead + 4 * c);
+    return s == pos ? *reinterpret_cast<const f32x4*>(&s_new[which][4 * c]) : v;
+  };
+  constexpr int kStep = kDecWaves * 4;                     // positions per workgroup step
+  float m[G], l[G];
+  f32x4 o[G];
+#pragma unroll
+  for (int h = 0; h < G; ++h) {
+    m[h] = -__builtin_inff();
+    l[h] = 0.0f;
+    o[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int c0 = 0; c0 < S; c0 += kDecKeys) {
+    const int n = min(kDecKeys, S - c0);
+    float mx[G];
+#pragma unroll
+    for (int h = 0; h < G; ++h) mx[h] = m[h];
+    for (int s0 = wave * 4 + g; s0 < n; s0 += kStep * kDecUnroll) {
+      f32x4 kr[kDecUnroll];
+#pragma unroll
+      for (int u = 0; u < kDecUnroll; ++u) kr[u] = row(kc, 0, c0 + min(s0 + u * kStep, n - 1));
+#pragma unroll
+      for (int u = 0; u < kDecUnroll; ++u) {
+        const int s = s0 + u * kStep;
+#pragma unroll
+        for (int h = 0; h < G; ++h) {
+          float d = kr[u].x * q[h].x + kr[u].y * q[h].y + kr[u].z * q[h].z + kr[u].w * q[h].w;
+#pragma unroll
+          for (int x = 1; x < 16; x <<= 1) d += __shfl_xor(d, x, 64);
+          if (s < n) {
+            mx[h] = fmaxf(mx[h], d);
+            if (c == 0) s_p[h][s] = d;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 16, 64));
+      mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 32, 64));
+      if (lane == 0) s_red[wave][h] = mx[h];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      float v = s_red[0][h];
+#pragma unroll
+      for (int w = 1; w < kDecWaves; ++w) v = fmaxf(v, s_red[w][h]);
+      const float alpha = __builtin_amdgcn_exp2f(m[h] - v);   // 0 in the first chunk
+      m[h] = v;
+      l[h] *= alpha;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[h][i] *= alpha;
+    }
+    for (int s0 = wave * 4 + g; s0 < n; s0 += kStep * kDecUnroll) {
+      f32x4 vr[kDecUnroll];
+#pragma unroll
+      for (int u = 0; u < kDecUnroll; ++u) vr[u] = row(vc, 1, c0 + min(s0 + u * kStep, n - 1));
+#pragma unroll
+      for (int u = 0; u < kDecUnroll; ++u) {
+        const int s = s0 + u * kStep;
+        if (s >= n) continue;
+#pragma unroll
+        for (int h = 0; h < G; ++h) {
+          const float e = __builtin_amdgcn_exp2f(s_p[h][s] - m[h]);
+          l[h] += e;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[h][i] += e * vr[u][i];
+        }
+      }
+    }
+    __syncthreads();                                       // scores and maxima are read before the next chunk's
+  }
+#pragma unroll
+  for (int h = 0; h < G; ++h) {
+#pragma unroll
+    for (int x = 16; x < 64; x <<= 1) {
+      l[h] += __shfl_xor(l[h], x, 64);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[h][i] += __shfl_xor(o[h][i], x, 64);
+    }
+    if (g == 0) *reinterpret_cast<f32x4*>(&s_o[wave][h][4 * c]) = o[h];
+    if (lane == 0) s_red[wave][h] = l[h];
+  }
+  __syncthreads();
+  if (tid < G * kHead) {
+    const int h = tid / kHead, e = tid % kHead;
+    float sum = 0.0f, den = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kDecWaves; ++w) {
+      sum += s_o[w][h][e];
+      den += s_red[w][h];
+    }
+    static_cast<T*>(p.out)[(static_cast<int64_t>(b) * p.hq + kv * G + h) * kHead + e] = Elem<DT>::from_f32(sum / den);
+  }
+}
+
+template <int DT>
+hipError_t launch_attention(const AttnParams& p, hipStream_t stream) {
+  if (p.t == 1) {
+    const dim3 grid(static_cast<unsigned>(p.batch * p.hk));
+    switch (p.hq / p.hk) {
+      case 1: attention_decode_kernel<DT, 1><<<grid, kDecWaves * 64, 0, stream>>>(p); break;
+      case 2: attention_decode_kernel<DT, 2><<<grid, kDecWaves * 64, 0, stream>>>(p); break;
+      default: attention_decode_kernel<DT, 4><<<grid, kDecWaves * 64, 0, stream>>>(p); break;
+    }
+    return hipGetLastError();
+  }
+  const int64_t chunks = static_cast<int64_t>(p.batch) * p.t * p.hk * (kHead / 4);
+  kv_write_kernel<DT><<<dim3(static_cast<unsigned>((chunks + 255) / 256)), 256, 0, stream>>>(p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const dim3 grid(static_cast<unsigned>((p.t + kFlashQ - 1) / kFlashQ), static_cast<unsigned>(p.batch * p.hq));
+  attention_kernel<DT><<<grid, 256, 0, stream>>>(p);
+  return hipGetLastError();
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+}  // namespace mep
+
+using namespace mep;
+
+extern "C" int mep_add_norm(const void* h, const void* delta, float mult, const void* weight, float eps,
+                            int64_t n_rows, int32_t hidden, int32_t dtype, void* h_out, void* x_out, void* stream) {
+  clear_error();
+  const char* fn = "mep_add_norm";
+  MEP_REQUIRE(dtype == MEP_DTYPE_F32 || dtype == MEP_DTYPE_BF16, MEP_ERR_INVALID_ARG, "%s: unknown dtype %d", fn, dtype);
+  MEP_REQUIRE(n_rows >= 0 && n_rows < (int64_t(1) << 31), MEP_ERR_INVALID_ARG, "%s: bad n_rows", fn);
+  const int epc = 16 / dtype_bytes(dtype);
+  MEP_REQUIRE(hidden > 0 && hidden % epc == 0 && hidden <= 4096, MEP_ERR_UNSUPPORTED,
+              "%s: hidden %d must be a positive multiple of %d, at most 4096", fn, hidden, epc);
+  if (n_rows == 0) return MEP_OK;
+  MEP_REQUIRE(h && weight && x_out && (delta == nullptr || h_out != nullptr), MEP_ERR_INVALID_ARG, "%s: null pointer", fn);
+  MEP_REQUIRE(aligned16(h) && aligned16(delta) && aligned16(weight) && aligned16(h_out) && aligned16(x_out),
+              MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
+  const dim3 grid(static_cast<unsigned>((n_rows + kNormWaves - 1) / kNormWaves));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int nch = (hidden / epc + 63) / 64;
+  auto go = [&](auto dt, auto c) {
+    constexpr int DT = decltype(dt)::value, NCH = decltype(c)::value;
+    typedef typename Elem<DT>::T T;
+    add_norm_kernel<DT, NCH><<<grid, kNormWaves * 64, 0, s>>>(static_cast<const T*>(h), static_cast<const T*>(delta), mult,
+                                                              static_cast<const T*>(weight), eps, n_rows, hidden,
+                                                              static_cast<T*>(h_out), static_cast<T*>(x_out));
+  };
+  auto by_width = [&](auto dt) {
+    if (nch <= 2) go(dt, std::integral_constant<int, 2>());
+    else if (nch <= 4) go(dt, std::integral_constant<int, 4>());
+    else if (nch <= 8) go(dt, std::integral_constant<int, 8>());
+    else go(dt, std::integral_constant<int, 16>());
+  };
+  if (dtype == MEP_DTYPE_BF16) by_width(std::integral_constant<int, MEP_DTYPE_BF16>());
+  else by_width(std::integral_constant<int, MEP_DTYPE_F32>());
+  MEP_CHECK_LAUNCH(fn);
+  return MEP_OK;
+}
+
+extern "C" int mep_attention(const void* q, const void* k, const void* v, const float* cos, const float* sin,
+                             int64_t n_positions, int32_t batch, int32_t t, int32_t n_heads, int32_t n_kv_heads,
+                             int32_t head_dim, int64_t start, int64_t max_len, float scale, int32_t dtype,
+                             float* k_cache, float* v_cache, void* out, void* stream) {
+  clear_error();
+  const char* fn = "mep_attention";
+  MEP_REQUIRE(dtype == MEP_DTYPE_F32 || dtype == MEP_DTYPE_BF16, MEP_ERR_INVALID_ARG, "%s: unknown dtype %d", fn, dtype);
+  MEP_REQUIRE(batch >= 0 && t >= 0 && start >= 0 && n_heads >= 1 && n_kv_heads >= 1, MEP_ERR_INVALID_ARG,
+              "%s: bad sizes", fn);
+  MEP_REQUIRE(head_dim == kHead, MEP_ERR_UNSUPPORTED, "%s: head size %d, supported: 64", fn, head_dim);
+  const int group = n_heads / n_kv_heads;
+  MEP_REQUIRE(n_heads % n_kv_heads == 0 && (group == 1 || group == 2 || group == 4), MEP_ERR_UNSUPPORTED,
+              "%s: %d query heads over %d kv heads (1, 2 or 4 each)", fn, n_heads, n_kv_heads);
+  MEP_REQUIRE(start + t <= max_len && start + t <= n_positions, MEP_ERR_INVALID_ARG,
+              "%s: positions up to %lld, the cache holds %lld and the rotary table %lld", fn,
+              static_cast<long long>(start + t), static_cast<long long>(max_len), static_cast<long long>(n_positions));
+  MEP_REQUIRE(max_len < (int64_t(1) << 31) && static_cast<int64_t>(batch) * n_heads <= 65535 &&
+                  static_cast<int64_t>(batch) * t * n_heads * (kHead / 4) < (int64_t(1) << 37),
+              MEP_ERR_UNSUPPORTED, "%s: batch or length too large", fn);
+  if (batch == 0 || t == 0) return MEP_OK;
+  MEP_REQUIRE(q && k && v && cos && sin && k_cache && v_cache && out, MEP_ERR_INVALID_ARG, "%s: null pointer", fn);
+  MEP_REQUIRE(aligned16(k_cache) && aligned16(v_cache) && aligned16(out), MEP_ERR_INVALID_ARG,
+              "%s: the caches and out must be 16-byte aligned", fn);
+  AttnParams p;
+  p.q = q; p.k = k; p.v = v; p.cos = cos; p.sin = sin; p.kc = k_cache; p.vc = v_cache; p.out = out;
+  p.batch = batch; p.t = t; p.hq = n_heads; p.hk = n_kv_heads;
+  p.start = static_cast<int>(start); p.max_len = max_len; p.scale = scale;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const hipError_t e = dtype == MEP_DTYPE_BF16 ? launch_attention<MEP_DTYPE_BF16>(p, s) : launch_attention<MEP_DTYPE_F32>(p, s);
+  MEP_REQUIRE(e == hipSuccess, MEP_ERR_HIP, "%s: launch failed: %s", fn, hipGetErrorString(e));
+  return MEP_OK;
+}

@@ -16,10 +16,16 @@ Weights use the checkpoint's key names (weights.py:17-26), so a loaded
 checkpoint dict drops in.
 
 Choices made here (not fixed by the reference): the KV cache is preallocated per layer and written in
-place (no concatenation per decode step); attention runs in fp32 (batched
-bf16 products with transposed operands are avoided on ROCm); the LM head is
-computed in fp32 for the positions asked for; router logits are fp32 (the
+place (no concatenation per decode step); attention runs in fp32; the LM head
+is computed in fp32 for the positions asked for; router logits are fp32 (the
 router hook decides, see ``backend.route``).
+
+On the GPU a causal forward (no ``positions`` or ``attn_mask`` given) of a model
+with ``fuse_router`` (``build_hip_model``) runs the norms, residual adds, RoPE,
+cache writes and attention on the HIP kernels of ``ops`` (``add_norm``,
+``attention``: head size 64, 1, 2 or 4 query heads per kv head, fp32 cache).
+Everything else, a model with other MoE backends among it, runs the torch
+statement of the same model below.
 """
 from __future__ import annotations
 
@@ -30,6 +36,8 @@ from typing import Callable, Sequence
 
 import torch
 import torch.nn.functional as F
+
+from . import ops
 
 
 @dataclass
@@ -211,14 +219,71 @@ class GraniteMoeModel:
         h = h + self._attention(layer, x, positions, cache, attn_mask) * cfg.residual_multiplier
         x = rms_norm(h, self.w[k_["post_ln"]], cfg.rms_norm_eps)
         B, T, H = x.shape
-        x_flat = x.reshape(B * T, H)
+        moe_out = self._moe_block(layer, x.reshape(B * T, H), moe_valid)
+        return h + moe_out.view(B, T, H) * cfg.residual_multiplier
+
+    def _moe_block(self, layer: int, x: torch.Tensor, moe_valid) -> torch.Tensor:
+        """The MoE block of `layer` on normed rows x (n, H): router hook + backend."""
+        cfg, w_router = self.cfg, self.w[layer_keys(layer)["router"]]
         fused = getattr(self.moe[layer], "route_and_call", None) if self.fuse_router else None
         if fused is not None:
-            moe_out, _, _ = fused(x_flat, self.w[k_["router"]], cfg.num_experts_per_tok, moe_valid)
-        else:
-            topk_idx, topk_gate = self.router(x_flat, self.w[k_["router"]], cfg.num_experts_per_tok)
-            moe_out = self.moe[layer](x_flat, topk_idx, topk_gate, valid_mask=moe_valid)
-        return h + moe_out.view(B, T, H) * cfg.residual_multiplier
+            return fused(x, w_router, cfg.num_experts_per_tok, moe_valid)[0]
+        topk_idx, topk_gate = self.router(x, w_router, cfg.num_experts_per_tok)
+        return self.moe[layer](x, topk_idx, topk_gate, valid_mask=moe_valid)
+
+    def _native(self, input_ids: torch.Tensor, cache: KVCache | None, positions, attn_mask) -> bool:
+        """Whether the HIP kernels cover this forward.  What they do not cover,
+        and what would raise, goes through the torch statement."""
+        cfg, e = self.cfg, self.embed
+        if not self.fuse_router or positions is not None or attn_mask is not None:
+            return False
+        if not e.is_cuda or not input_ids.is_cuda:
+            return False
+        B, T = input_ids.shape
+        hq, hk, d = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+        if e.dtype not in (torch.bfloat16, torch.float32) or d != 64 or hq % hk or hq // hk not in (1, 2, 4):
+            return False
+        if cfg.hidden_size > 4096 or cfg.hidden_size % 8 or B * T == 0 or B * hq > 65535:
+            return False
+        start = 0 if cache is None else cache.length
+        if start + T > self.rope.cos.shape[0]:
+            return False
+        if cache is not None:
+            shape = (B, hk, cache.max_len, d)
+            for c in (*cache.k, *cache.v):
+                if c.dtype != torch.float32 or c.device != e.device or c.shape != shape or not c.is_contiguous():
+                    return False
+            if start + T > cache.max_len:
+                return False
+        return all(w.dtype == e.dtype and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in self.w.values())
+
+    def _forward_native(self, input_ids: torch.Tensor, cache: KVCache | None, moe_valid, logits_at) -> torch.Tensor:
+        """The rows that the head needs, normed: (B, T or 1, H)."""
+        cfg = self.cfg
+        B, T = input_ids.shape
+        H, rm, eps = cfg.hidden_size, cfg.residual_multiplier, cfg.rms_norm_eps
+        start = 0 if cache is None else cache.length
+        h = (self.embed[input_ids] * cfg.embedding_multiplier).view(B * T, H)
+        if cache is None:
+            kc, vc = (torch.empty(B, cfg.num_key_value_heads, T, cfg.head_dim, dtype=torch.float32, device=h.device)
+                      for _ in range(2))
+        moe_out = None
+        for layer in range(cfg.num_hidden_layers):
+            k_ = layer_keys(layer)
+            h, x = ops.add_norm(h, self.w[k_["input_ln"]], eps, moe_out, rm)
+            q, k, v = (F.linear(x, self.w[k_[m]]) for m in ("wq", "wk", "wv"))
+            if cache is not None:
+                kc, vc = cache.k[layer], cache.v[layer]
+            o = ops.attention(q, k, v, self.rope.cos, self.rope.sin, B, start, kc, vc, cfg.attention_multiplier)
+            h, x = ops.add_norm(h, self.w[k_["post_ln"]], eps, F.linear(o, self.w[k_["wo"]]), rm)
+            moe_out = self._moe_block(layer, x, moe_valid).contiguous()
+        if logits_at is not None:
+            at = (torch.arange(B, device=h.device), logits_at)
+            h, moe_out = (None if z is None else z.view(B, T, H)[at] for z in (h, moe_out))
+        norm = self.w["model.norm.weight"]
+        if moe_out is not None and moe_out.dtype != h.dtype:      # a last backend of another dtype
+            return rms_norm(h + moe_out * rm, norm, eps).view(B, -1, H)
+        return ops.add_norm(h, norm, eps, moe_out, rm)[1].view(B, -1, H)
 
     @torch.no_grad()
     def forward(self, input_ids: torch.Tensor, cache: KVCache | None = None, positions=None,
@@ -226,11 +291,16 @@ class GraniteMoeModel:
         """input_ids (B, T) -> fp32 logits (B, T, V), or (B, 1, V) at `logits_at` (B,)."""
         cfg = self.cfg
         B, T = input_ids.shape
+        if moe_valid is not None:
+            moe_valid = moe_valid.reshape(-1)
+        if self._native(input_ids, cache, positions, attn_mask):
+            h = self._forward_native(input_ids, cache, moe_valid, logits_at)
+            if cache is not None:
+                cache.length += T
+            return self._logits(h)
         if positions is None:
             start = cache.length if cache is not None else 0
             positions = torch.arange(start, start + T, device=input_ids.device).expand(B, T)
-        if moe_valid is not None:
-            moe_valid = moe_valid.reshape(-1)
         h = self.embed[input_ids] * cfg.embedding_multiplier
         for layer in range(cfg.num_hidden_layers):
             h = self._block(layer, h, positions, cache, attn_mask, moe_valid)
@@ -238,10 +308,12 @@ class GraniteMoeModel:
             cache.length += T
         if logits_at is not None:
             h = h[torch.arange(B, device=h.device), logits_at][:, None]
-        h = rms_norm(h, self.w["model.norm.weight"], cfg.rms_norm_eps)
+        return self._logits(rms_norm(h, self.w["model.norm.weight"], cfg.rms_norm_eps))
+
+    def _logits(self, h: torch.Tensor) -> torch.Tensor:
         if self._head is None:
             self._head = self.embed.float()            # tied LM head, fp32 copy made once
-        return F.linear(h.float(), self._head) / cfg.logits_scaling
+        return F.linear(h.float(), self._head) / self.cfg.logits_scaling
 
     __call__ = forward
 

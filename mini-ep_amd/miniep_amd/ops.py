@@ -531,3 +531,53 @@ def gather_rows(x: torch.Tensor, perm: torch.Tensor, n_rows: int, top_k: int,
                                     _ptr(flat), _ptr(ids), out.data_ptr(), _stream(dev))
     _lib.check(rc, "mep_gather_rows")
     return out, ids
+
+
+# ----------------------------------------------------------------------------
+# the transformer around the MoE block (modeling.py:55-80,146-197)
+# ----------------------------------------------------------------------------
+def add_norm(h: torch.Tensor, weight: torch.Tensor, eps: float, delta: torch.Tensor | None = None,
+             mult: float = 1.0) -> tuple[torch.Tensor, torch.Tensor]:
+    """(h + delta * mult, rms_norm of that): the residual step and the norm of
+    Block.forward in one launch (without ``delta``: (h, its norm)).  (n, H)
+    rows, H at most 4096."""
+    dev = _require_device(h, weight, delta)
+    for t in (h, weight, delta):
+        if t is not None and (t.dtype != h.dtype or not t.is_contiguous()):
+            raise TypeError("add_norm takes contiguous tensors of one dtype")
+    n, hidden = h.shape
+    if weight.numel() != hidden or (delta is not None and delta.shape != h.shape):
+        raise ValueError(f"weight {tuple(weight.shape)} or delta does not match rows of {hidden}")
+    x = torch.empty_like(h)
+    h_out = h if delta is None else torch.empty_like(h)
+    rc = _lib.lib().mep_add_norm(h.data_ptr(), _ptr(delta), mult, weight.data_ptr(), eps, n, hidden, _dtype_code(h),
+                                 h_out.data_ptr(), x.data_ptr(), _stream(dev))
+    _lib.check(rc, "mep_add_norm")
+    return h_out, x
+
+
+def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, batch: int,
+              start: int, k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float) -> torch.Tensor:
+    """Causal GQA attention of the call's tokens over the cache, with RoPE and
+    the cache write (mep_attention): q (batch*t, hq*64), k / v (batch*t, hk*64)
+    are the projections, the caches (batch, hk, max_len, 64) fp32 hold
+    ``start`` positions and get t more.  Returns (batch*t, hq*64)."""
+    dev = _require_device(q, k, v, cos, sin, k_cache, v_cache)
+    for t in (k, v, q):
+        if t.dtype != q.dtype or not t.is_contiguous():
+            raise TypeError("q, k and v must be contiguous and of one dtype")
+    for t in (cos, sin, k_cache, v_cache):
+        if t.dtype != torch.float32 or not t.is_contiguous():
+            raise TypeError("the rotary tables and the caches must be contiguous fp32 tensors")
+    b, hk, max_len, d = k_cache.shape
+    n, width = q.shape
+    if b != batch or n % batch or v_cache.shape != k_cache.shape or tuple(k.shape) != (n, hk * d) or \
+            v.shape != k.shape or width % d or cos.shape[1] != d or sin.shape != cos.shape:
+        raise ValueError(f"attention shapes do not match: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)} "
+                         f"cache {tuple(k_cache.shape)} batch {batch}")
+    out = torch.empty_like(q)
+    rc = _lib.lib().mep_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+                                  cos.shape[0], batch, n // batch, width // d, hk, d, start, max_len, scale,
+                                  _dtype_code(q), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), _stream(dev))
+    _lib.check(rc, "mep_attention")
+    return out

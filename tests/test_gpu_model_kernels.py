@@ -1,0 +1,101 @@
+"""The kernels around the MoE block (ops.add_norm, ops.attention) against the
+same steps in fp64, and the model's native forward against its torch
+statement."""
+import pytest
+import torch
+
+from miniep_amd import ops
+from miniep_amd.model import KVCache, ModelConfig, RotaryTable, build_hip_model, random_weights
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,H", [(1, 1024), (5, 1000), (33, 2048), (3, 4096), (2, 8), (7, 2056)])
+def test_add_norm(n, H, dtype):
+    """Row widths below, at and above a lane's chunk counts.  h_out's two
+    roundings are torch's own; x is within one rounding of the fp64 norm."""
+    g = torch.Generator().manual_seed(n * H)
+    h, d = (torch.randn(n, H, generator=g).to(dtype).to(DEV) for _ in range(2))
+    w = (1 + 0.1 * torch.randn(H, generator=g)).to(dtype).to(DEV)
+    for delta in (d, None):
+        h2, x = ops.add_norm(h, w, 1e-6, delta, 0.22)
+        want_h = h if delta is None else h + delta * 0.22
+        assert torch.equal(h2, want_h)
+        hd = want_h.double()
+        want = w.double() * hd * torch.rsqrt(hd.pow(2).mean(-1, keepdim=True) + 1e-6)
+        # fp32: the mean of H squares (H/64 + 6 adds), rsqrt and two products; bf16 adds its rounding
+        eps = 2.0 ** -8 if dtype == torch.bfloat16 else (H / 64 + 12) * 2.0 ** -24
+        assert ((x.double() - want).abs() <= eps * want.abs() + 1e-30).all()
+
+
+def _rope64(t, rope, pos):
+    cos, sin = rope.cos[pos].double(), rope.sin[pos].double()       # (t, d)
+    half = t.shape[-1] // 2
+    return t * cos + torch.cat([-t[..., half:], t[..., :half]], -1) * sin
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,start,hq,hk", [
+    (1, 1, 0, 16, 8), (3, 1, 63, 16, 8), (2, 1, 64, 4, 4), (1, 1, 255, 8, 2), (2, 1, 2047, 16, 8), (1, 1, 2500, 8, 2),
+    (2, 2, 0, 16, 8), (1, 17, 0, 4, 4), (2, 64, 5, 8, 2), (1, 65, 0, 16, 8), (2, 130, 70, 16, 8)])
+def test_attention(B, T, start, hq, hk, dtype):
+    """Decode (one token: the new position alone, chunks of 2048 scores and
+    one past them) and prefill (partial and whole blocks of 64 queries and
+    keys, cached positions in front), 1, 2 and 4 query heads per kv head;
+    positions of the cache past the call stay as they are."""
+    d, max_len = 64, start + T + 3
+    cfg = ModelConfig(num_attention_heads=hq, num_key_value_heads=hk, hidden_size=64 * hq)
+    rope = RotaryTable(cfg, DEV)
+    g = torch.Generator().manual_seed(B + T + start)
+    q, k, v = (torch.randn(B * T, h * d, generator=g).to(dtype).to(DEV) for h in (hq, hk, hk))
+    cache = torch.randn(2, B, hk, max_len, d, generator=g).to(DEV)
+    kc, vc = cache[0].clone(), cache[1].clone()
+    out = ops.attention(q, k, v, rope.cos, rope.sin, B, start, kc, vc, 0.05)
+
+    pos = torch.arange(start, start + T, device=DEV)
+    qd, kd, vd = (t.double().view(B, T, -1, d).transpose(1, 2) for t in (q, k, v))
+    qd, kd = _rope64(qd, rope, pos), _rope64(kd, rope, pos)
+    want_k, want_v = cache[0].double(), cache[1].double()
+    want_k[:, :, start:start + T], want_v[:, :, start:start + T] = kd, vd
+    assert torch.equal(vc.double(), want_v)
+    assert (kc.double() - want_k).abs().max() <= 3 * 2.0 ** -24 * want_k.abs().max()
+    S = start + T
+    kk, vv = (t[:, :, :S].repeat_interleave(hq // hk, 1) for t in (want_k, want_v))
+    s = (qd @ kk.transpose(2, 3).contiguous()) * 0.05
+    s = s.masked_fill(torch.arange(S, device=DEV) > pos[:, None], -torch.inf)
+    want = (torch.softmax(s, -1) @ vv).transpose(1, 2).reshape(B * T, hq * d)
+    # a score is a sum of 64 products (error below 64 ulp of the largest), so a
+    # probability is off by that times the score, and the values' sum adds S/64 + 16 roundings
+    tol = (64 * float(s[s.isfinite()].abs().max()) + S / 64 + 32) * 2.0 ** -24 * float(vv.abs().max())
+    err = (out.double() - want).abs()
+    if dtype == torch.bfloat16:
+        err = err - 2.0 ** -8 * want.abs()
+    assert float(err.max()) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_native_forward_equals_torch_statement(dtype):
+    """Prefill, a decode step and a second chunk through one cache, and the
+    cacheless forward, against the same model made to run its torch statement
+    (an explicit causal mask).  One layer of rounding differences in bf16,
+    fp32 sums otherwise."""
+    cfg = ModelConfig(num_hidden_layers=2, vocab_size=997)
+    w = random_weights(cfg, seed=3, dtype=dtype, device=DEV)
+    m = build_hip_model(cfg, w)
+    ids = torch.randint(0, cfg.vocab_size, (3, 45), generator=torch.Generator().manual_seed(1)).to(DEV)
+
+    def causal(t, s):
+        return torch.arange(s, device=DEV) <= torch.arange(s - t, s, device=DEV)[:, None]
+
+    tol = 2e-2 if dtype == torch.bfloat16 else 2e-5
+    a, b = (KVCache(cfg, 3, 50, DEV) for _ in range(2))
+    for lo, hi in ((0, 30), (30, 31), (31, 45)):
+        got = m(ids[:, lo:hi], cache=a)
+        want = m(ids[:, lo:hi], cache=b, attn_mask=causal(hi - lo, hi))
+        assert a.length == b.length == hi and got.shape == want.shape
+        assert float((got - want).norm() / want.norm()) <= tol
+    at = torch.tensor([3, -1, 44], device=DEV)
+    got, want = m(ids, logits_at=at), m(ids, logits_at=at, attn_mask=causal(45, 45))
+    assert got.shape == (3, 1, cfg.vocab_size) and float((got - want).norm() / want.norm()) <= tol
