@@ -38,6 +38,35 @@ int mep_attention(const void* q, const void* k, const void* v, const float* cos,
                   int32_t head_dim, int64_t start, int64_t max_len, float scale, int32_t dtype,
                   float* k_cache, float* v_cache, void* out, void* stream);
 
+/* ------------------------------------------------------------------------
+ * The attention half of Block.forward (modeling.py:186-192) for at most 32
+ * rows (batch * t) of a bf16 model, as one call (4 launches for t = 1):
+ *   h1 = h + round(delta * mult)      (delta NULL: h1 = h)
+ *   q, k, v = rms_norm(h1; norm1) @ {wq, wk, wv}^T
+ *   o = attention of them (mep_attention: RoPE, cache write, causal)
+ *   h_out = h1 + round(round(o @ wo^T) * mult),  x_out = rms_norm(h_out; norm2)
+ * Each projection is rounded to bf16, sums are fp32.  wq (n_heads*head_dim,
+ * hidden), wk / wv (n_kv_heads*head_dim, hidden), wo (hidden,
+ * n_heads*head_dim).  Supported: hidden and n_heads*head_dim in {1024, 2048},
+ * and mep_attention's shapes.  h_out must not be h.
+ *
+ * mep_norm_head: logits (n_rows, vocab) fp32 = rms_norm(h + round(delta *
+ * mult); norm) @ w^T / divisor for at most 32 rows, w (vocab, hidden) bf16,
+ * hidden 1024 or 2048, products and sums in fp32 (modeling.py:249-254).
+ * ---------------------------------------------------------------------- */
+size_t mep_attention_block_workspace(int64_t n_rows, int32_t hidden, int32_t n_heads, int32_t n_kv_heads,
+                                     int32_t head_dim);
+
+int mep_attention_block(const void* h, const void* delta, float mult, const void* norm1, const void* norm2,
+                        float eps, const void* wq, const void* wk, const void* wv, const void* wo,
+                        const float* cos, const float* sin, int64_t n_positions, int32_t batch, int32_t t,
+                        int32_t hidden, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int64_t start,
+                        int64_t max_len, float scale, float* k_cache, float* v_cache, void* workspace,
+                        size_t workspace_bytes, void* h_out, void* x_out, void* stream);
+
+int mep_norm_head(const void* h, const void* delta, float mult, const void* norm, float eps, const void* w,
+                  int64_t n_rows, int32_t hidden, int32_t vocab, float divisor, float* logits, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -23,7 +23,9 @@ router hook decides, see ``backend.route``).
 On the GPU a causal forward (no ``positions`` or ``attn_mask`` given) of a model
 with ``fuse_router`` (``build_hip_model``) runs the norms, residual adds, RoPE,
 cache writes and attention on the HIP kernels of ``ops`` (``add_norm``,
-``attention``: head size 64, 1, 2 or 4 query heads per kv head, fp32 cache).
+``attention``: head size 64, 1, 2 or 4 query heads per kv head, fp32 cache), and
+with at most 32 rows in bf16 the projections and the head (``attention_block``,
+``norm_head``).
 Everything else, a model with other MoE backends among it, runs the torch
 statement of the same model below.
 """
@@ -187,10 +189,11 @@ class GraniteMoeModel:
         self.embed = weights["model.embed_tokens.weight"]
         self.rope = RotaryTable(cfg, self.embed.device)
         self._head: torch.Tensor | None = None
+        self._keys = [layer_keys(layer) for layer in range(cfg.num_hidden_layers)]
 
     def _attention(self, layer: int, x: torch.Tensor, positions: torch.Tensor, cache: KVCache | None,
                    attn_mask: torch.Tensor | None) -> torch.Tensor:
-        cfg, k_ = self.cfg, layer_keys(layer)
+        cfg, k_ = self.cfg, self._keys[layer]
         B, T, H = x.shape
         d, hq, hk = cfg.head_dim, cfg.num_attention_heads, cfg.num_key_value_heads
         x2 = x.reshape(B * T, H)
@@ -214,7 +217,7 @@ class GraniteMoeModel:
         return F.linear(o, self.w[k_["wo"]]).view(B, T, H)
 
     def _block(self, layer: int, h: torch.Tensor, positions, cache, attn_mask, moe_valid) -> torch.Tensor:
-        cfg, k_ = self.cfg, layer_keys(layer)
+        cfg, k_ = self.cfg, self._keys[layer]
         x = rms_norm(h, self.w[k_["input_ln"]], cfg.rms_norm_eps)
         h = h + self._attention(layer, x, positions, cache, attn_mask) * cfg.residual_multiplier
         x = rms_norm(h, self.w[k_["post_ln"]], cfg.rms_norm_eps)
@@ -224,7 +227,7 @@ class GraniteMoeModel:
 
     def _moe_block(self, layer: int, x: torch.Tensor, moe_valid) -> torch.Tensor:
         """The MoE block of `layer` on normed rows x (n, H): router hook + backend."""
-        cfg, w_router = self.cfg, self.w[layer_keys(layer)["router"]]
+        cfg, w_router = self.cfg, self.w[self._keys[layer]["router"]]
         fused = getattr(self.moe[layer], "route_and_call", None) if self.fuse_router else None
         if fused is not None:
             return fused(x, w_router, cfg.num_experts_per_tok, moe_valid)[0]
@@ -255,35 +258,49 @@ class GraniteMoeModel:
                     return False
             if start + T > cache.max_len:
                 return False
-        return all(w.dtype == e.dtype and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in self.w.values())
+        for w in self.w.values():
+            if w.dtype != e.dtype or not w.is_contiguous() or w.data_ptr() % 16:
+                return False
+        return True
 
     def _forward_native(self, input_ids: torch.Tensor, cache: KVCache | None, moe_valid, logits_at) -> torch.Tensor:
-        """The rows that the head needs, normed: (B, T or 1, H)."""
-        cfg = self.cfg
+        """forward on the HIP kernels; at most 32 rows of a bf16 model (decode)
+        run their projections and the head on them as well."""
+        cfg, w = self.cfg, self.w
         B, T = input_ids.shape
-        H, rm, eps = cfg.hidden_size, cfg.residual_multiplier, cfg.rms_norm_eps
+        n, H, rm, eps = B * T, cfg.hidden_size, cfg.residual_multiplier, cfg.rms_norm_eps
+        hq, hk, d = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+        cos, sin, scale = self.rope.cos, self.rope.sin, cfg.attention_multiplier
         start = 0 if cache is None else cache.length
-        h = (self.embed[input_ids] * cfg.embedding_multiplier).view(B * T, H)
+        h = (self.embed[input_ids] * cfg.embedding_multiplier).view(n, H)
+        small = ops.small_rows(n, H, h.dtype) and ops.small_rows(n, hq * d, h.dtype)
+        if small:
+            ws = ops.attention_block_workspace(n, H, hq, hk, d, h.device)
         if cache is None:
-            kc, vc = (torch.empty(B, cfg.num_key_value_heads, T, cfg.head_dim, dtype=torch.float32, device=h.device)
-                      for _ in range(2))
+            kc, vc = (torch.empty(B, hk, T, d, dtype=torch.float32, device=h.device) for _ in range(2))
         moe_out = None
-        for layer in range(cfg.num_hidden_layers):
-            k_ = layer_keys(layer)
-            h, x = ops.add_norm(h, self.w[k_["input_ln"]], eps, moe_out, rm)
-            q, k, v = (F.linear(x, self.w[k_[m]]) for m in ("wq", "wk", "wv"))
+        for layer, k_ in enumerate(self._keys):
+            norm1, norm2 = w[k_["input_ln"]], w[k_["post_ln"]]
             if cache is not None:
                 kc, vc = cache.k[layer], cache.v[layer]
-            o = ops.attention(q, k, v, self.rope.cos, self.rope.sin, B, start, kc, vc, cfg.attention_multiplier)
-            h, x = ops.add_norm(h, self.w[k_["post_ln"]], eps, F.linear(o, self.w[k_["wo"]]), rm)
+            if small:
+                proj = (w[k_["wq"]], w[k_["wk"]], w[k_["wv"]], w[k_["wo"]])
+                h, x = ops.attention_block(h, moe_out, rm, norm1, norm2, eps, proj, cos, sin, B, start, kc, vc, scale, ws)
+            else:
+                h, x = ops.add_norm(h, norm1, eps, moe_out, rm)
+                q, k, v = (F.linear(x, w[k_[m]]) for m in ("wq", "wk", "wv"))
+                o = ops.attention(q, k, v, cos, sin, B, start, kc, vc, scale)
+                h, x = ops.add_norm(h, norm2, eps, F.linear(o, w[k_["wo"]]), rm)
             moe_out = self._moe_block(layer, x, moe_valid).contiguous()
         if logits_at is not None:
             at = (torch.arange(B, device=h.device), logits_at)
             h, moe_out = (None if z is None else z.view(B, T, H)[at] for z in (h, moe_out))
-        norm = self.w["model.norm.weight"]
+        norm = w["model.norm.weight"]
         if moe_out is not None and moe_out.dtype != h.dtype:      # a last backend of another dtype
-            return rms_norm(h + moe_out * rm, norm, eps).view(B, -1, H)
-        return ops.add_norm(h, norm, eps, moe_out, rm)[1].view(B, -1, H)
+            return self._logits(rms_norm(h + moe_out * rm, norm, eps).view(B, -1, H))
+        if ops.small_rows(h.shape[0], H, h.dtype):
+            return ops.norm_head(h, moe_out, rm, norm, eps, self.embed, cfg.logits_scaling).view(B, -1, self.embed.shape[0])
+        return self._logits(ops.add_norm(h, norm, eps, moe_out, rm)[1].view(B, -1, H))
 
     @torch.no_grad()
     def forward(self, input_ids: torch.Tensor, cache: KVCache | None = None, positions=None,
@@ -294,10 +311,10 @@ class GraniteMoeModel:
         if moe_valid is not None:
             moe_valid = moe_valid.reshape(-1)
         if self._native(input_ids, cache, positions, attn_mask):
-            h = self._forward_native(input_ids, cache, moe_valid, logits_at)
+            logits = self._forward_native(input_ids, cache, moe_valid, logits_at)
             if cache is not None:
                 cache.length += T
-            return self._logits(h)
+            return logits
         if positions is None:
             start = cache.length if cache is not None else 0
             positions = torch.arange(start, start + T, device=input_ids.device).expand(B, T)

@@ -581,3 +581,66 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tens
                                   _dtype_code(q), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), _stream(dev))
     _lib.check(rc, "mep_attention")
     return out
+
+
+def small_rows(n_rows: int, hidden: int, dtype: torch.dtype) -> bool:
+    """Whether attention_block / norm_head take n_rows rows of this width."""
+    return n_rows <= 32 and hidden in (1024, 2048) and dtype == torch.bfloat16
+
+
+def attention_block(h: torch.Tensor, delta: torch.Tensor | None, mult: float, norm1: torch.Tensor,
+                    norm2: torch.Tensor, eps: float, weights, cos: torch.Tensor, sin: torch.Tensor, batch: int,
+                    start: int, k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float,
+                    workspace: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """The attention half of Block.forward for at most 32 rows (small_rows) in
+    one call (mep_attention_block): (residual stream after the attention, its
+    norm2).  ``weights`` = (wq, wk, wv, wo); ``workspace`` uint8 of
+    attention_block_workspace bytes, reused by calls on one stream."""
+    dev = _require_device(h, delta, norm1, norm2, *weights, cos, sin, k_cache, v_cache, workspace)
+    for t in (h, norm1, norm2, *weights, h if delta is None else delta):
+        if t.dtype != torch.bfloat16 or not t.is_contiguous():
+            raise TypeError("attention_block takes contiguous bf16 tensors")
+    for t in (cos, sin, k_cache, v_cache):
+        if t.dtype != torch.float32 or not t.is_contiguous():
+            raise TypeError("the rotary tables and the caches must be contiguous fp32 tensors")
+    n, hidden = h.shape
+    b, hk, max_len, d = k_cache.shape
+    wq, wk, wv, wo = weights
+    q_cols = wq.shape[0]
+    if b != batch or n % batch or v_cache.shape != k_cache.shape or q_cols % d or cos.shape[1] != d or \
+            sin.shape != cos.shape or wq.shape != (q_cols, hidden) or wk.shape != (hk * d, hidden) or \
+            wv.shape != wk.shape or wo.shape != (hidden, q_cols) or norm1.shape != (hidden,) or \
+            norm2.shape != (hidden,) or (delta is not None and delta.shape != h.shape):
+        raise ValueError("attention_block: shapes do not match")
+    h_out, x = torch.empty_like(h), torch.empty_like(h)
+    rc = _lib.lib().mep_attention_block(
+        h.data_ptr(), _ptr(delta), mult, norm1.data_ptr(), norm2.data_ptr(), eps, wq.data_ptr(), wk.data_ptr(),
+        wv.data_ptr(), wo.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.shape[0], batch, n // batch, hidden,
+        q_cols // d, hk, d, start, max_len, scale, k_cache.data_ptr(), v_cache.data_ptr(), workspace.data_ptr(),
+        workspace.numel(), h_out.data_ptr(), x.data_ptr(), _stream(dev))
+    _lib.check(rc, "mep_attention_block")
+    return h_out, x
+
+
+def attention_block_workspace(n_rows: int, hidden: int, n_heads: int, n_kv_heads: int, head_dim: int,
+                              device) -> torch.Tensor:
+    nbytes = _lib.lib().mep_attention_block_workspace(n_rows, hidden, n_heads, n_kv_heads, head_dim)
+    return torch.empty(int(nbytes), dtype=torch.uint8, device=device)
+
+
+def norm_head(h: torch.Tensor, delta: torch.Tensor | None, mult: float, norm: torch.Tensor, eps: float,
+              w: torch.Tensor, divisor: float) -> torch.Tensor:
+    """(n, V) fp32 logits rms_norm(h + delta * mult) @ w.T / divisor for at most
+    32 rows (small_rows) of a bf16 model (mep_norm_head)."""
+    dev = _require_device(h, delta, norm, w)
+    for t in (h, norm, w, h if delta is None else delta):
+        if t.dtype != torch.bfloat16 or not t.is_contiguous():
+            raise TypeError("norm_head takes contiguous bf16 tensors")
+    n, hidden = h.shape
+    if norm.shape != (hidden,) or w.dim() != 2 or w.shape[1] != hidden or (delta is not None and delta.shape != h.shape):
+        raise ValueError("norm_head: shapes do not match")
+    logits = torch.empty((n, w.shape[0]), dtype=torch.float32, device=dev)
+    rc = _lib.lib().mep_norm_head(h.data_ptr(), _ptr(delta), mult, norm.data_ptr(), eps, w.data_ptr(), n, hidden,
+                                  w.shape[0], divisor, logits.data_ptr(), _stream(dev))
+    _lib.check(rc, "mep_norm_head")
+    return logits

@@ -99,3 +99,61 @@ def test_native_forward_equals_torch_statement(dtype):
     at = torch.tensor([3, -1, 44], device=DEV)
     got, want = m(ids, logits_at=at), m(ids, logits_at=at, attn_mask=causal(45, 45))
     assert got.shape == (3, 1, cfg.vocab_size) and float((got - want).norm() / want.norm()) <= tol
+
+
+def _norm64(h, w):
+    return w.double() * h.double() * torch.rsqrt(h.double().pow(2).mean(-1, keepdim=True) + 1e-6)
+
+
+@pytest.mark.parametrize("n,H,vocab", [(1, 1024, 16), (16, 1024, 49155), (17, 2048, 1000), (32, 1024, 8193)])
+def test_norm_head(n, H, vocab):
+    """One and two row fragments, partial column tiles, one tile and many per
+    workgroup.  x is bf16 and equal to add_norm's, so the logits are fp32 sums
+    of exact products: H roundings at most, of sums below |x| |w|."""
+    g = torch.Generator().manual_seed(n + vocab)
+    h, d = (torch.randn(n, H, generator=g).bfloat16().to(DEV) for _ in range(2))
+    norm = (1 + 0.1 * torch.randn(H, generator=g)).bfloat16().to(DEV)
+    w = (torch.randn(vocab, H, generator=g) * 0.02).bfloat16().to(DEV)
+    for delta in (d, None):
+        got = ops.norm_head(h, delta, 0.22, norm, 1e-6, w, 6.0)
+        _, x = ops.add_norm(h, norm, 1e-6, delta, 0.22)
+        want = x.double() @ w.double().T.contiguous() / 6.0
+        # the norm's mean is summed in another order than add_norm's: a few x elements round the other way
+        tol = H * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T.contiguous()) / 6.0
+        flip = 2.0 ** -8 * float(x.abs().max()) * float(w.abs().max()) / 6.0
+        assert ((got.double() - want).abs() <= tol + 4 * flip).all()
+
+
+@pytest.mark.parametrize("B,T,start,H,hq,hk", [(1, 1, 0, 1024, 16, 8), (8, 1, 40, 1024, 16, 8), (17, 1, 3, 1024, 16, 16),
+                                               (32, 1, 9, 2048, 16, 4), (3, 7, 5, 1024, 32, 8), (2, 16, 0, 2048, 32, 16)])
+def test_attention_block(B, T, start, H, hq, hk):
+    """mep_attention_block against the same steps as separate calls (add_norm,
+    F.linear, attention): every tensor between the steps is bf16, so the two
+    differ by one bf16 rounding here and there (sums in another order)."""
+    d, n = 64, B * T
+    cfg = ModelConfig(num_attention_heads=hq, num_key_value_heads=hk, hidden_size=64 * hq)
+    rope = RotaryTable(cfg, DEV)
+    g = torch.Generator().manual_seed(B * T + H)
+
+    def mat(*shape, sd=0.02):
+        return (torch.randn(*shape, generator=g) * sd).bfloat16().to(DEV)
+
+    h, moe = mat(n, H, sd=1), mat(n, H, sd=1)
+    n1, n2 = mat(H, sd=1), mat(H, sd=1)
+    wq, wk, wv, wo = mat(hq * d, H), mat(hk * d, H), mat(hk * d, H), mat(H, hq * d)
+    cache = torch.randn(2, B, hk, start + T, d, generator=g).to(DEV)
+    ws = ops.attention_block_workspace(n, H, hq, hk, d, DEV)
+    for delta in (moe, None):
+        kc, vc = cache[0].clone(), cache[1].clone()
+        got_h, got_x = ops.attention_block(h, delta, 0.22, n1, n2, 1e-6, (wq, wk, wv, wo), rope.cos, rope.sin, B, start,
+                                           kc, vc, 0.015625, ws)
+        kr, vr = cache[0].clone(), cache[1].clone()
+        h1, x = ops.add_norm(h, n1, 1e-6, delta, 0.22)
+        q, k, v = (torch.nn.functional.linear(x, w) for w in (wq, wk, wv))
+        o = ops.attention(q, k, v, rope.cos, rope.sin, B, start, kr, vr, 0.015625)
+        want_h, want_x = ops.add_norm(h1, n2, 1e-6, torch.nn.functional.linear(o, wo), 0.22)
+        for a, b, most in ((kc, kr, 2.0 ** -7), (vc, vr, 2.0 ** -7), (got_h, want_h, 2.0 ** -7), (got_x, want_x, 2.0 ** -6)):
+            a, b = a.double(), b.double()
+            # one bf16 step of the element (or of the rotation's other half), seldom
+            assert ((a - b).abs() <= most * b.abs() + 2.0 ** -7 * b.abs().mean()).float().mean() > 0.999
+            assert float((a - b).norm() / b.norm()) <= 2e-3
