@@ -27,7 +27,7 @@
 // 128-byte lines and stores them non-temporally (y_entries is read once, by
 // the combine).  fp32 keeps the simpler two-stage grouped_gemm_kernel.
 //
-// Scheduling (bf16, more than 1024 rows): persistent, one workgroup per CU,
+// Scheduling (bf16, larger batches): persistent, one workgroup per CU,
 // both GEMMs in one launch (kModeBoth; kModeGateUp / kModeDown run one of
 // them).  The row tiles, derived on the device from `offsets` (no host round
 // trip for the counts), are split into one contiguous range per XCD; each
@@ -39,10 +39,11 @@
 // tile's first two stages stream in during the last four steps and the
 // epilogue of the current one.  Within a step, a wave two MFMA groups in runs
 // at raised priority, which keeps the two waves of a SIMD from moving in
-// lockstep.  At most 1024 rows (decode, small batches) run the small-batch
-// kernels below instead: a workgroup per 32-row chunk and column block,
-// weights streamed straight into registers, both GEMMs in one launch.  Every
-// path walks K in the same order, so they give the same bits.
+// lockstep.  Up to some hundred rows per expert run as one launch of
+// moe_gemm_mid_kernel (64- or 128-row chunks, two or three workgroups per CU),
+// and at most 256 rows (decode) as the small-batch kernels: a workgroup per
+// 32-row chunk and column block, weights streamed straight into registers.
+// Every path walks K in the same order, so they give the same bits.
 #include "combine_dev.h"
 #include "common.h"
 #include "router_dev.h"
@@ -84,6 +85,7 @@ struct GemmParams {
   int N;                     // output columns (GEMM-1: I; GEMM-2: H)
   int n_tiles_n;             // column tiles per row tile
   uint32_t a_bytes;          // size of A in bytes (< 4 GiB)
+  uint32_t c_bytes;          // mid-size launch: size of act in bytes (< 4 GiB)
   uint32_t k_magic;          // entry / top_k == umulhi(entry, k_magic) >> k_shift for entry < 2^31
   int k_shift;
   int* flags;                // error flags word of the schedule buffer (sched::kFlags), or NULL
@@ -525,7 +527,9 @@ static_assert(BPW == NF, "one DMA block per MFMA group of an odd step");
 //                    workgroups done, combine workgroups past their wait
 //   line 16 + r      row tile r's GEMM-1 column tiles finished (kModeBoth);
 //                    the small-batch launch of both GEMMs: chunk r's GEMM-1
-//                    counts and GEMM-2 workgroups past their wait (words 0, 1)
+//                    counts and GEMM-2 workgroups past their wait (words 0,
+//                    1); the mid-size one: those of chunks 4 r .. 4 r + 3
+//                    (words 0, 1 of each quarter line)
 // Every launch leaves every word but the flags zero.
 namespace sched {
 constexpr int kLine = 32;                      // ints per 128-byte line
@@ -533,13 +537,14 @@ constexpr int kQueue = 0, kDone = 8 * kLine, kItems = 9 * kLine, kFlags = 10 * k
               kG2Done = 12 * kLine, kCombDone = 13 * kLine, kRowDone = 16 * kLine;
 __host__ __device__ constexpr int queue_word(int q) { return kQueue + q * kLine; }
 __host__ __device__ constexpr int row_word(int r) { return kRowDone + r * kLine; }
+__host__ __device__ constexpr int mid_word(int q) { return row_word(q >> 2) + (q & 3) * (kLine / 4); }
 constexpr int kFlagWait = 1, kFlagDrain = 2, kFlagInput = kFlagInputBit;
 constexpr int kWaitLimit = 1 << 20;            // polls of one row counter (about a second)
 // the small-batch launch of both GEMMs runs up to this many rows
 constexpr int64_t kSmallRows = 1024;
 // row tiles of max_rows rows over n_local experts: each expert adds at most
 // one partial tile; the small-batch launch of both GEMMs keeps a line per
-// 32-row chunk there instead
+// 32-row chunk there instead, the mid-size one a line per four chunks
 inline int64_t words(int64_t max_rows, int n_local) {
   const int64_t tiles = (max_rows + 255) / 256 + n_local;
   const int64_t chunks = max_rows <= kSmallRows ? (max_rows + 31) / 32 + n_local : 0;
@@ -1864,6 +1869,330 @@ hipError_t launch_skinny_both(const GemmParams& p1, const GemmParams& p2, int64_
 }
 
 // ============================================================================
+// bf16 path for some tens to a few hundred rows per expert (a prompt or a
+// large decode batch): one workgroup per (chunk of 16 MFC rows of one local
+// expert, column block of 64 act / 128 output columns), both GEMMs in one
+// launch.
+//
+// The tiled kernel's 256 x 256 tiles leave most of the chip idle there (a few
+// row tiles times 4 column tiles on 256 CUs, each a serial chain of a GEMM-1
+// and a GEMM-2 tile, most of its rows padding); the small-batch kernel reads
+// the weights again for every 32 rows.  Here 4 waves (2 x 2) share a chunk's
+// rows and 128 weight rows through an LDS ring of two blocks of two K-steps
+// (one 128-byte line of every row), filled AHEAD blocks in front through
+// registers.  Two or three workgroups fit on a CU and cover each other's
+// prologues, barriers and epilogues.
+//
+// Threads copy whole lines, 8 lanes per row.  (The weights read straight into
+// the MFMA layout, as the small-batch kernel does, put 16 rows under 16
+// neighbouring lanes: 64 L1 lookups per KiB instead of 8 to 16, which bound
+// the loop once a weight row met more than some 64 rows: 171 us at 4096
+// tokens of the GraniteMoE layer.)  Plain loads and LDS writes, not LDS DMA: the
+// compiler waits for every load in flight before reading LDS that a DMA may
+// have written.  The ring holds MFMA fragments of 1 KiB, lane (lr, lg)'s 16
+// bytes in slot 16 lg + (lr ^ lg ^ 12 (step & 1)); a copying lane group takes
+// rows 4 apart.  That keeps both the fragment reads and the copies' writes
+// (8 lanes of a row to two steps x four lane groups) on distinct banks.
+//
+// Chunks are listed by expert and split into 8 contiguous ranges, one per XCD
+// (workgroup b runs on XCD b mod 8): the column blocks of a chunk share its
+// rows in that XCD's L2, and the chunks of an expert its weights.  GEMM-1's
+// workgroups come first in the grid and are dispatched in order, so every one
+// is resident or done before a GEMM-2 workgroup waits for its chunk (thread 0,
+// bounded, after its first weight loads are out), and every wait ends; a
+// give-up flags the launch and stores NaN.  K is walked in the tiled kernel's
+// order with the same MFMA, so every output has the other kernels' bits.
+namespace mid {
+constexpr int NT = 256;
+constexpr int AHEAD = 2;                      // blocks (two K-steps) of loads in flight
+constexpr int WF = 8;                         // weight fragments of a workgroup: 128 weight rows
+inline int64_t chunks(int64_t max_rows, int n_local, int rows) { return (max_rows + rows - 1) / rows + n_local; }
+}  // namespace mid
+
+// Column block cb of chunk q: rows [row_lo, row_hi) of expert e, at most 16 MFC.
+template <int MFC, bool GEMM1>
+__device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int cb, int n_cb, int row_lo, int row_hi,
+                                          int n_cb_other, int* sched, unsigned char* s_ring, int* s_gave) {
+  typedef uint16_t T;
+  constexpr int AHEAD = mid::AHEAD;
+  constexpr int MF = MFC / 2, NF = 4;                         // row and weight fragments per wave
+  constexpr int AP = MFC / 2, WP = mid::WF / 2;               // copy passes of 32 rows
+  constexpr int STEP = (MFC + mid::WF) * 1024, SLOT = 2 * STEP;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int K = p.K, NB = K / 64, KD = K / 64;                // blocks of two K-steps
+  const int nt = cb / 2;                                      // the tiled kernel's column tile and K rotation
+  const int rot = (!GEMM1 && KD % 4 == 0) ? (nt & 3) * (KD / 4) : 0;
+  const int slot = p.w_slot != nullptr ? p.w_slot[e] : e;
+  const unsigned char* const W =
+      static_cast<const unsigned char*>(p.W) + static_cast<int64_t>(slot) * p.w_expert_stride * 2;
+  const unsigned char* const A = static_cast<const unsigned char*>(p.A);
+
+  // ---- copies: this thread's row of a pass and 16-byte chunk of its line -----------
+  const int c16 = ((tid >> 3) & 3) * 4 + ((tid >> 5) & 3), cf = tid >> 7;   // row 16 cf + c16 of the pass's 32
+  const int cc = tid & 7, clg = cc & 3, cstep = cc >> 2;
+  // weight rows: fragment 4 wn + j.  GEMM-1: j < 2 gate, j >= 2 the up rows of
+  // the same act columns cb*64 + 32 wn ..; GEMM-2: output columns cb*128 +
+  // 64 wn + 32 (j / 2) ..  Row n of the fragment pair's half j & 1 is column
+  // 8 (n / 4) + 4 (j & 1) + n % 4 of the 32, so a lane's results across the
+  // pair are 8 consecutive columns.
+  uint32_t w_off[WP], a_off[AP];                              // byte offsets: x, act and an expert are below 4 GiB
+#pragma unroll
+  for (int i = 0; i < WP; ++i) {
+    const int fr = 2 * i + cf, j = fr & 3;
+    const int in32 = 8 * (c16 >> 2) + 4 * (j & 1) + (c16 & 3);
+    const int row = GEMM1 ? (j >= 2 ? p.N : 0) + cb * 64 + 32 * (fr >> 2) + in32
+                          : cb * 128 + 64 * (fr >> 2) + 32 * (j >> 1) + in32;
+    w_off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K * 2) + cc * 16;
+  }
+  u32x4 wr[AHEAD][WP], ar[AHEAD][AP];
+  auto line = [&](int b) {                                    // byte offset of block b's line of a row
+    int kb = b + rot;
+    if (kb >= NB) kb -= NB;
+    return kb * 128;
+  };
+  auto load_w = [&](int b, u32x4 (&w)[WP]) {
+    const unsigned char* const base = W + line(b);
+#pragma unroll
+    for (int i = 0; i < WP; ++i) w[i] = *reinterpret_cast<const u32x4*>(base + w_off[i]);
+  };
+  auto load_a = [&](int b, u32x4 (&x)[AP]) {
+    const unsigned char* const base = A + line(b);
+#pragma unroll
+    for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const u32x4*>(base + a_off[i]);
+  };
+  unsigned char* const cdst = s_ring + cstep * STEP + cf * 1024 + (16 * clg + (c16 ^ clg ^ (12 * cstep))) * 16;
+  auto write = [&](int b, const u32x4 (&w)[WP], const u32x4 (&x)[AP]) {
+    unsigned char* const dst = cdst + (b & 1) * SLOT;
+#pragma unroll
+    for (int i = 0; i < AP; ++i) *reinterpret_cast<u32x4*>(dst + 2 * i * 1024) = x[i];
+#pragma unroll
+    for (int i = 0; i < WP; ++i) *reinterpret_cast<u32x4*>(dst + (MFC + 2 * i) * 1024) = w[i];
+  };
+  // the weights need neither the row map nor GEMM-1
+#pragma unroll
+  for (int b = 0; b < AHEAD; ++b) load_w(b, wr[b]);
+
+  int* const done1 = sched + sched::mid_word(q);
+  int* const seen2 = done1 + 1;
+  if constexpr (!GEMM1) {
+    if (tid == 0) {
+      const int target = n_cb_other + (q == p.dbg_chunk ? 1 : 0);
+      int polls = 0, gave = 0;
+      while (load_dev_i32(done1) < target) {
+        if (++polls == p.wait_limit) {
+          atomic_or_1(sched + sched::kFlags, sched::kFlagWait);
+          gave = 1;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(4);
+      }
+      *s_gave = gave;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < AP; ++i) {
+    const int r = min(row_lo + 32 * i + 16 * cf + c16, row_hi - 1);
+    uint32_t from = static_cast<uint32_t>(r);
+    if constexpr (GEMM1) {
+      const uint32_t f = static_cast<uint32_t>(p.perm[r]);    // flat entry t*k + s
+      from = p.k_magic ? (__umulhi(f, p.k_magic) >> p.k_shift) : f;
+    }
+    a_off[i] = from * static_cast<uint32_t>(K * 2) + cc * 16;
+  }
+#pragma unroll
+  for (int b = 0; b < AHEAD; ++b) load_a(b, ar[b]);
+
+  // ---- K loop --------------------------------------------------------------------------
+  // Block b (steps 2 b, 2 b + 1), with its first step's fragments in registers:
+  //   write block b + 1 (in registers) to the ring, load block b + 1 + AHEAD;
+  //   step 2 b: MFMAs, each fragment refilled with step 2 b + 1's after its last use;
+  //   barrier (block b + 1 is in the ring); step 2 b + 1 likewise, refilled from
+  //   block b + 1.
+  // Block b + 1's slot held block b - 1, whose last fragments were read before
+  // block b - 1's barrier.  No load is under a run-time condition inside a
+  // round, so the compiler counts the loads in flight exactly; the first
+  // round is peeled so that the loop is entered in its steady state, and the
+  // last one loads nothing.
+  f32x4 acc[MF][NF];
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned char* const frag0 = s_ring + (16 * lg + (lr ^ lg)) * 16;
+  const unsigned char* const frag1 = s_ring + STEP + (16 * lg + (lr ^ lg ^ 12)) * 16;
+  u32x4 a[MF], w[NF];
+  auto read_a = [&](const unsigned char* at, int i) { a[i] = *reinterpret_cast<const u32x4*>(at + (wm * MF + i) * 1024); };
+  auto read_w = [&](const unsigned char* at, int j) {
+    w[j] = *reinterpret_cast<const u32x4*>(at + (MFC + wn * NF + j) * 1024);
+  };
+  constexpr int ROUND = 2;                                    // blocks per round: the ring's slots are immediates
+  static_assert(AHEAD == ROUND, "register sets and ring slots rotate together");
+  auto round = [&](int r, auto last_c) {
+    constexpr bool LAST = decltype(last_c)::value;
+#pragma unroll
+    for (int u = 0; u < ROUND; ++u) {
+      const int b = r * ROUND + u;
+      const bool more = !LAST || u + 1 < ROUND;               // block b + 1 exists
+      constexpr int S = ROUND;
+      if (more) write(b + 1, wr[(u + 1) % S], ar[(u + 1) % S]);
+      if (!LAST) {
+        // past the last block (the round before the last loads one too many) line() wraps: in bounds, unused
+        load_w(b + 1 + AHEAD, wr[(u + 1) % S]);
+        load_a(b + 1 + AHEAD, ar[(u + 1) % S]);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const unsigned char* const next = h == 0 ? frag1 + u * SLOT : frag0 + (u ^ 1) * SLOT;
+        const bool refill = h == 0 || more;
+#pragma unroll
+        for (int j = 0; j < NF; ++j) {
+#pragma unroll
+          for (int i = 0; i < MF; ++i) {
+            mfma_acc(acc[i][j], w[j], a[i]);
+            if (refill && j == NF - 1) read_a(next, i);
+          }
+          if (refill) read_w(next, j);
+          asm volatile("" ::: "memory");
+        }
+        if (h == 0 && more) lds_barrier();
+      }
+    }
+  };
+  write(0, wr[0], ar[0]);
+  load_w(AHEAD, wr[0]);
+  load_a(AHEAD, ar[0]);
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < MF; ++i) read_a(frag0, i);
+#pragma unroll
+  for (int j = 0; j < NF; ++j) read_w(frag0, j);
+  const int rounds = NB / ROUND;                              // K is a multiple of 256
+  round(0, std::integral_constant<bool, false>());
+  for (int r = 1; r < rounds - 1; ++r) round(r, std::integral_constant<bool, false>());
+  round(rounds - 1, std::integral_constant<bool, true>());
+
+  // ---- epilogue: lane (lr, lg) of a fragment pair holds columns 8 lg .. 8 lg + 7 of row lr
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) pin_acc(acc[i][j]);
+  T* const C = static_cast<T*>(p.C);
+  if constexpr (!GEMM1) {
+    if (__builtin_amdgcn_readfirstlane(*s_gave)) {            // the wait for act gave up
+      const float nan = __builtin_nanf("");
+#pragma unroll
+      for (int i = 0; i < MF; ++i)
+#pragma unroll
+        for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{nan, nan, nan, nan};
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MF; ++i) {
+    const int r = row_lo + (wm * MF + i) * 16 + lr;
+    if (r >= row_hi) continue;
+    if constexpr (GEMM1) {
+      u32x4 o;
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const f32x4 g = acc[i][h >> 1], up = acc[i][2 + (h >> 1)];
+        o[h] = pack_bf16x2(silu_f(g[2 * (h & 1)]) * up[2 * (h & 1)], silu_f(g[2 * (h & 1) + 1]) * up[2 * (h & 1) + 1]);
+      }
+      // device scope, so GEMM-2 on any XCD reads the final rows
+      store_dev_16(p.C, p.c_bytes, static_cast<uint32_t>(r * p.N + cb * 64 + 32 * wn + 8 * lg) * 2u, o);
+    } else {
+      T* const dst = C + static_cast<int64_t>(p.perm[r]) * p.N + cb * 128 + 64 * wn + 8 * lg;
+#pragma unroll
+      for (int jp = 0; jp < 2; ++jp) {
+        u32x4 o;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const f32x4 v = acc[i][2 * jp + (h >> 1)];
+          o[h] = pack_bf16x2(v[2 * (h & 1)], v[2 * (h & 1) + 1]);
+        }
+        *reinterpret_cast<u32x4*>(dst + 32 * jp) = o;
+      }
+    }
+  }
+  if constexpr (GEMM1) {
+    // every wave's act stores are complete before the chunk's count goes up
+    __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    __syncthreads();
+    if (tid == 0) atomic_add_1(done1, 1);
+  } else {
+    // the last GEMM-2 workgroup of the chunk takes out what every workgroup
+    // adds, so a count that arrives after a give-up still leaves both at zero
+    if (tid == 0 && atomic_add_1(seen2, 1) == n_cb - 1) {
+      atomic_add_1(done1, -n_cb_other);
+      atomic_add_1(seen2, -n_cb);
+    }
+  }
+}
+
+// Workgroup `unit` of one GEMM: its chunk and column block.
+template <int MFC, bool GEMM1>
+__device__ __forceinline__ void mid_body(const GemmParams& p, int unit, int n_cb_other, int* sched, int* s_pre,
+                                         int* s_off, unsigned char* s_ring, int* s_gave) {
+  constexpr int CH = 16 * MFC;
+  const int tid = threadIdx.x;
+  const int nl = p.n_local;
+  // offsets[nl] < 0: the dispatch gave up; no expert has rows, the call is flagged
+  {
+    const int last = p.offsets[nl];
+    for (int j = tid; j <= nl; j += mid::NT) s_off[j] = last < 0 ? 0 : p.offsets[j];
+    if (last < 0 && unit == 0 && tid == 0 && p.flags != nullptr) atomic_or_1(p.flags, sched::kFlagInput);
+  }
+  __syncthreads();
+  if (tid < 64) scan_units<CH>(s_off, s_pre, nl, 1);
+  __syncthreads();
+  const int n_cb = GEMM1 ? p.N / 64 : p.N / 128;              // column blocks
+  const int n_chunks = s_pre[nl];
+  const int xcd = unit & 7, at = unit >> 3;
+  const int q_lo = static_cast<int>(static_cast<int64_t>(n_chunks) * xcd / 8);
+  const int q_hi = static_cast<int>(static_cast<int64_t>(n_chunks) * (xcd + 1) / 8);
+  const int q = q_lo + at / n_cb, cb = at % n_cb;
+  if (q >= q_hi) return;
+  int lo = 0, hi = nl - 1;                                    // largest j with s_pre[j] <= q
+  while (lo < hi) {
+    const int m = (lo + hi + 1) >> 1;
+    if (s_pre[m] <= q) lo = m; else hi = m - 1;
+  }
+  const int e = __builtin_amdgcn_readfirstlane(lo);
+  const int row_lo = __builtin_amdgcn_readfirstlane(s_off[e] + (q - s_pre[e]) * CH);
+  const int row_hi = __builtin_amdgcn_readfirstlane(min(s_off[e + 1], row_lo + CH));
+  // an expert's last chunk is often short: half the row fragments then
+  if (row_hi - row_lo <= CH / 2)
+    mid_chunk<MFC / 2, GEMM1>(p, e, q, cb, n_cb, row_lo, row_hi, n_cb_other, sched, s_ring, s_gave);
+  else
+    mid_chunk<MFC, GEMM1>(p, e, q, cb, n_cb, row_lo, row_hi, n_cb_other, sched, s_ring, s_gave);
+}
+
+template <int MFC>
+__global__ __launch_bounds__(mid::NT, 2) void moe_gemm_mid_kernel(GemmParams p1, GemmParams p2, int g1_blocks,
+                                                                  int* sched) {
+  __shared__ int s_pre[bfk::NLMAX + 1];
+  __shared__ int s_off[bfk::NLMAX + 1];
+  __shared__ __attribute__((aligned(16))) unsigned char s_ring[4 * (MFC + mid::WF) * 1024];
+  __shared__ int s_gave;
+  const int b = blockIdx.x;
+  if (b < g1_blocks) mid_body<MFC, true>(p1, b, 0, sched, s_pre, s_off, s_ring, &s_gave);
+  else mid_body<MFC, false>(p2, b - g1_blocks, p1.N / 64, sched, s_pre, s_off, s_ring, &s_gave);
+}
+
+template <int MFC>
+hipError_t launch_mid(const GemmParams& p1, const GemmParams& p2, int64_t max_rows, int* sched, hipStream_t stream) {
+  // an XCD's range is at most ceil(chunks / 8) chunks
+  const int64_t per_xcd = (mid::chunks(max_rows, p1.n_local, 16 * MFC) + 7) / 8;
+  const int64_t b1 = 8 * per_xcd * (p1.N / 64), b2 = 8 * per_xcd * (p2.N / 128);
+  moe_gemm_mid_kernel<MFC><<<dim3(static_cast<unsigned>(b1 + b2)), mid::NT, 0, stream>>>(
+      p1, p2, static_cast<int>(b1), sched);
+  return hipGetLastError();
+}
+
+// ============================================================================
 // The decode layer in one launch (mep_moe_layer): router + dispatch, GEMM-1 +
 // SwiGLU, GEMM-2 and the combine, for bf16, 32 experts, top-8 and at most 32
 // tokens (every expert then has at most one 32-row chunk).
@@ -2508,6 +2837,32 @@ bool tiled_down(int dtype, int64_t max_rows, int inter) {
   return dtype == MEP_DTYPE_BF16 && inter % 256 == 0 && max_rows > skinny::kMaxEntries2;
 }
 
+// Row fragments per chunk of the mid-size launch, 0: another kernel runs.
+// (Host side, so by max_rows; us of one call, weights cold, GraniteMoE's
+// experts unless said otherwise, small-batch or tiled kernel -> this one.)
+//  - at most 256 rows: the small-batch launch, which may end with the combine
+//    (32 tokens: 26 with it, 23 + 4 without);
+//  - the tiled kernel where its row tiles are mostly full and its GEMM-1 tiles
+//    fill whole rounds of the CUs: 1500 tokens 67 against 72, 4096 tokens 116
+//    against 143, 2500 tokens 98 against 103;
+//  - this one below (64 tokens 27 -> 23, 128: 43 -> 24, 256: 57 -> 29, 517:
+//    52 -> 37, 1024: 60 -> 50), where an expert's rows fill at most half a
+//    row tile (hidden 2048, 64 experts, 500 tokens: 216 -> 195), and where the
+//    tiled launch's second round would be nearly empty (2048 tokens: 92 -> 82).
+int mid_row_frags(int64_t max_rows, int n_local, int inter) {
+  if (max_rows <= 256) return 0;
+  const int64_t cu = device_cu_count();
+  // row tiles and chunks: an expert's last one is half empty on average
+  const int64_t tiles = (max_rows / bfk::BM + n_local / 2) * (inter / (bfk::BN / 2));
+  const bool sparse = max_rows <= static_cast<int64_t>(n_local) * (bfk::BM / 2);
+  if (!sparse && tiles * 4 > cu * 3 && !(tiles > cu && tiles * 20 <= cu * 27)) return 0;
+  // chunks of 128 rows read the weights half as often as chunks of 64, if the
+  // experts have that many rows and the chip is still full (128 tokens: even;
+  // 384 tokens: 34 -> 30; 10 experts with 120 rows each: 19 with 64, 25 with 128)
+  const int64_t units = (max_rows / 128 + n_local / 2) * (inter / 64);
+  return max_rows >= static_cast<int64_t>(n_local) * 64 && units >= (sparse ? cu : 2 * cu) ? 8 : 4;
+}
+
 // Tile shapes of the generic kernel (fp32, and bf16 GEMM-2 with I % 256 != 0):
 // bf16 256x256 on 8 waves (4 x 2), fp32 128x128 on 4 waves.
 typedef TileCfg<256, 256, 4, 2> CfgBf16;
@@ -2687,6 +3042,26 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
   const size_t need = mep_experts_workspace_size(max_rows, inter, dtype);
   MEP_REQUIRE(workspace_bytes >= need, MEP_ERR_WORKSPACE, "%s: workspace %zu B < required %zu B", fn,
               workspace_bytes, need);
+  const int mid_frags = dtype == MEP_DTYPE_BF16 && inter % 256 == 0 ? mid_row_frags(max_rows, n_local, inter) : 0;
+  if (mid_frags > 0) {
+    MEP_REQUIRE(x && perm && offsets && w_in && w_out && y_entries, MEP_ERR_INVALID_ARG, "%s: null pointer", fn);
+    rc = check_queue(fn, true, tile_queue, tile_queue_ints, max_rows, n_local);
+    if (rc != MEP_OK) return rc;
+    MEP_REQUIRE(aligned16(x) && aligned16(w_in) && aligned16(w_out) && aligned16(workspace) && aligned16(y_entries),
+                MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
+    GemmParams g1 = gemm1_params<MEP_DTYPE_BF16, CfgBf16>(x, n_tokens, top_k, perm, offsets, n_local, w_in, w_slot,
+                                                          hidden, inter, workspace);
+    GemmParams g2 = gemm2_params<MEP_DTYPE_BF16, CfgBf16>(workspace, top_k, perm, offsets, n_local, max_rows, w_out,
+                                                          w_slot, hidden, inter, y_entries);
+    set_sched(g1, tile_queue);
+    set_sched(g2, tile_queue);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    g1.c_bytes = static_cast<uint32_t>(max_rows * inter * 2);
+    const hipError_t e = mid_frags == 4 ? launch_mid<4>(g1, g2, max_rows, tile_queue, s)
+                                        : launch_mid<8>(g1, g2, max_rows, tile_queue, s);
+    MEP_REQUIRE(e == hipSuccess, MEP_ERR_HIP, "%s: %s", fn, hipGetErrorString(e));
+    return MEP_OK;
+  }
   if (tiled_gate_up(dtype, max_rows) && tiled_down(dtype, max_rows, inter)) {
     MEP_REQUIRE(x && perm && offsets && w_in && w_out && y_entries, MEP_ERR_INVALID_ARG, "%s: null pointer", fn);
     rc = check_queue(fn, true, tile_queue, tile_queue_ints, max_rows, n_local);
