@@ -31,6 +31,7 @@ def route(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, return_logits: b
 
 
 def _world1_tables(n_experts: int, device):
+    """(table, n_rep, g2l) of a placement with every expert on rank 0."""
     table = torch.zeros(n_experts, 1, dtype=torch.int32, device=device)
     n_rep = torch.ones(n_experts, dtype=torch.int32, device=device)
     g2l = torch.arange(n_experts, dtype=torch.int32, device=device)
@@ -144,6 +145,11 @@ class HipEPShareBackend:
         for i, e in enumerate(local_experts):
             g2l[e] = i
         self.g2l = g2l.to(self.w_in.device)
+        # constant tables of the send and receive halves, laid out with the placement
+        dev, E = self.w_in.device, self.placement.num_experts
+        self._nobody = torch.full((E,), -1, dtype=torch.int32, device=dev)
+        self._by_rank = _world1_tables(self.placement.world, dev)
+        self._by_expert = _world1_tables(E, dev)
 
     def apply_placement(self, placement: Placement, w_in: torch.Tensor, w_out: torch.Tensor):
         """Swap in a new placement and this rank's re-sliced weights
@@ -178,7 +184,7 @@ class HipEPShareBackend:
                             self.my_rank, self.g2l, len(self.local_experts), seg_tokens=seg,
                             route_counts=rc, want_dest=want_dest, check=self.check)
         if self.stats is not None:
-            self.stats.recv_tokens_per_layer[self.layer] += disp.offsets[-1].to(torch.long)
+            self.stats.recv_tokens_per_layer[self.layer].add_(disp.offsets[-1])
         return disp
 
     def send(self, x_flat, topk_idx, valid_mask=None, rr=None) -> "SendBatch":
@@ -196,12 +202,11 @@ class HipEPShareBackend:
         if has_rep and rr is None:
             rr = torch.zeros(1, E, dtype=torch.long, device=dev)
         rc = self.stats.route_counts[self.layer] if self.stats is not None else None
-        nobody = torch.full((E,), -1, dtype=torch.int32, device=dev)
         d = ops.dispatch(topk_idx, valid_mask, E, table, n_rep, has_rep, rr if has_rep else None, -1,
-                         nobody, 0, route_counts=rc, want_dest=True, check=self.check)
+                         self._nobody, 0, route_counts=rc, want_dest=True, check=self.check)
         # the destination-sorted order is the dispatch itself keyed by destination
         key = d.dest[: n * k].clamp(min=0).view(n, k).to(torch.int64)   # masked entries stay masked
-        t1, r1, ident = _world1_tables(world, dev)
+        t1, r1, ident = self._by_rank if self._by_rank[0].shape[0] == world else _world1_tables(world, dev)
         srt = ops.dispatch(key, valid_mask, world, t1, r1, False, None, 0, ident, world, check=False)
         m = int(srt.offsets[-1])
         send_x, send_ids = ops.gather_rows(x_flat.to(self.w_in.dtype), srt.perm, m, k, topk_idx)
@@ -216,11 +221,11 @@ class HipEPShareBackend:
         if n == 0:
             return torch.empty(0, recv_x.shape[1], dtype=self.w_in.dtype, device=dev)
         E = self.placement.num_experts
-        t1, r1, _ = _world1_tables(E, dev)
+        t1, r1, _ = self._by_expert
         d = ops.dispatch(recv_experts.view(n, 1), None, E, t1, r1, False, None, 0, self.g2l,
                          len(self.local_experts), check=self.check)
         if self.stats is not None:
-            self.stats.recv_tokens_per_layer[self.layer] += d.offsets[-1].to(torch.long)
+            self.stats.recv_tokens_per_layer[self.layer].add_(d.offsets[-1])
         return ops.grouped_swiglu(recv_x.to(self.w_in.dtype), d, self.w_in, self.w_out, w_slot=self.w_slot)
 
     def share(self, x_flat, topk_idx, valid_mask=None, seg_tokens=None, rr=None, y_entries=None,

@@ -285,7 +285,8 @@ class GraniteMoeModel:
                 kc, vc = cache.k[layer], cache.v[layer]
             if small:
                 proj = (w[k_["wq"]], w[k_["wk"]], w[k_["wv"]], w[k_["wo"]])
-                h, x = ops.attention_block(h, moe_out, rm, norm1, norm2, eps, proj, cos, sin, B, start, kc, vc, scale, ws)
+                h, x = ops.attention_block(h, moe_out, rm, norm1, norm2, eps, proj, cos, sin, B, start, kc, vc, scale,
+                                           ws)
             else:
                 h, x = ops.add_norm(h, norm1, eps, moe_out, rm)
                 q, k, v = (F.linear(x, w[k_[m]]) for m in ("wq", "wk", "wv"))
@@ -299,7 +300,8 @@ class GraniteMoeModel:
         if moe_out is not None and moe_out.dtype != h.dtype:      # a last backend of another dtype
             return self._logits(rms_norm(h + moe_out * rm, norm, eps).view(B, -1, H))
         if ops.small_rows(h.shape[0], H, h.dtype):
-            return ops.norm_head(h, moe_out, rm, norm, eps, self.embed, cfg.logits_scaling).view(B, -1, self.embed.shape[0])
+            logits = ops.norm_head(h, moe_out, rm, norm, eps, self.embed, cfg.logits_scaling)
+            return logits.view(B, -1, self.embed.shape[0])
         return self._logits(ops.add_norm(h, norm, eps, moe_out, rm)[1].view(B, -1, H))
 
     @torch.no_grad()

@@ -42,8 +42,18 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def _index(dev: torch.device) -> int:
+    return dev.index if dev.index is not None else torch.cuda.current_device()
+
+
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """Handle of the current stream of ``dev`` (torch.cuda.current_stream builds
+    a Stream object around it: 2 us of a 25 us call, three times)."""
+    return torch._C._cuda_getCurrentRawStream(_index(dev))
+
+
+def _as_dtype(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    return (t if t.dtype == dtype else t.to(dtype)).contiguous()
 
 
 _QUEUES: dict[tuple[int, int], torch.Tensor] = {}
@@ -56,7 +66,7 @@ def _tile_queue(dev: torch.device, max_rows: int, n_local: int) -> torch.Tensor:
     every launch (but for its sticky error word, see ``experts_check``), one
     per stream so that launches on different streams never share it, and
     replaced by a larger zeroed one when a launch needs more words."""
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(dev))
+    key = (_index(dev), _stream(dev))
     need = int(_lib.lib().mep_experts_queue_ints(max_rows, n_local))
     q = _QUEUES.get(key)
     if q is None or q.numel() < need:
@@ -71,7 +81,7 @@ def _dispatch_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     every call on that stream, one per stream so that calls on different
     streams never share it, and replaced by a larger zeroed one when a call
     needs more bytes."""
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(dev))
+    key = (_index(dev), _stream(dev))
     ws = _DISPATCH_WS.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = _DISPATCH_WS[key] = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=dev)
@@ -82,7 +92,7 @@ def dispatch_check(dev: torch.device | None = None) -> None:
     """Synchronise and raise MepError if the last dispatch on the current
     stream of ``dev`` (its workspace) dropped entries or gave up waiting."""
     dev = dev or torch.device("cuda", torch.cuda.current_device())
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(dev))
+    key = (_index(dev), _stream(dev))
     ws = _DISPATCH_WS.get(key)
     if ws is not None:
         _lib.check(_lib.lib().mep_dispatch_check(ws.data_ptr(), _stream(dev)), "mep_dispatch_check")
@@ -93,7 +103,7 @@ def experts_check(dev: torch.device | None = None) -> None:
     stream of ``dev`` flagged its results invalid (a GEMM-2 tile that gave
     up waiting for its GEMM-1 rows, or a tile queue nobody drained)."""
     dev = dev or torch.device("cuda", torch.cuda.current_device())
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(dev))
+    key = (_index(dev), _stream(dev))
     q = _QUEUES.get(key)
     if q is not None:
         _lib.check(_lib.lib().mep_experts_check(q.data_ptr(), _stream(dev)), "mep_experts_check")
@@ -119,7 +129,7 @@ def router_topk(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, return_log
     k selected logits stored in x.dtype (modeling.py:193-195)."""
     dev = _require_device(x_flat, w_router)
     x = x_flat.contiguous()
-    w = w_router.to(x.dtype).contiguous()
+    w = _as_dtype(w_router, x.dtype)
     n, h = x.shape
     e = w.shape[0]
     if w.shape[1] != h:
@@ -136,7 +146,7 @@ def router_topk(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, return_log
 def topk_softmax(logits: torch.Tensor, k: int, gate_dtype: torch.dtype = torch.float32):
     """Top-k + fp32 softmax of precomputed fp32 logits (modeling.py:194-195)."""
     dev = _require_device(logits)
-    lg = logits.to(torch.float32).contiguous()
+    lg = _as_dtype(logits, torch.float32)
     n, e = lg.shape
     idx = torch.empty((n, k), dtype=torch.int64, device=dev)
     gate = torch.empty((n, k), dtype=gate_dtype, device=dev)
@@ -172,6 +182,40 @@ class Dispatch:
         return self.n_tokens * self.top_k
 
 
+_PARTS = {"counts": 0, "offsets": 1, "perm": 2, "row_of_entry": 3}
+
+
+def _part_ptr(disp: Dispatch, name: str) -> int:
+    t = disp.__dict__.get(name)
+    return disp.ptrs[_PARTS[name]] if t is None else t.data_ptr()
+
+
+class _PackedDispatch(Dispatch):
+    """A Dispatch whose index tensors are parts of one allocation, made into
+    tensors of their own when they are first asked for (a decode call asks for
+    none of them; four allocations are 5 us of host time)."""
+
+    def __init__(self, n_tokens: int, top_k: int, n_local: int, dev: torch.device, dest: torch.Tensor | None = None):
+        nk = max(n_tokens * top_k, 1)
+        size = [max(n_local, 1), n_local + 1, nk, nk]
+        start = [0]
+        for v in size:                                      # each part on a 256-byte boundary
+            start.append(start[-1] + (v + 63) // 64 * 64)
+        size[0] = n_local
+        buf = torch.empty(start[-1], dtype=torch.int32, device=dev)
+        base = buf.data_ptr()
+        self.__dict__.update(n_tokens=n_tokens, top_k=top_k, n_local=n_local, dest=dest, _buf=buf, _at=start,
+                             _size=size, ptrs=[base + 4 * v for v in start[:4]])   # counts, offsets, perm, row_of_entry
+
+    def __getattr__(self, name):
+        part = _PARTS.get(name)
+        if part is None:
+            raise AttributeError(name)
+        t = self._buf[self._at[part]:self._at[part] + self._size[part]]
+        self.__dict__[name] = t
+        return t
+
+
 def dispatch(topk_idx: torch.Tensor, valid_mask: torch.Tensor | None, n_experts: int,
              table: torch.Tensor, n_rep: torch.Tensor, has_replicas: bool,
              rr: torch.Tensor | None, my_rank: int, g2l: torch.Tensor, n_local: int,
@@ -182,7 +226,7 @@ def dispatch(topk_idx: torch.Tensor, valid_mask: torch.Tensor | None, n_experts:
     (updated in place when ``has_replicas``); ``seg_tokens`` the S+1 token
     offsets of the source segments (default: one segment)."""
     dev = _require_device(topk_idx, table, n_rep, g2l, rr, route_counts)
-    idx = topk_idx.to(torch.int64).contiguous()
+    idx = _as_dtype(topk_idx, torch.int64)
     n, k = idx.shape
     if seg_tokens is None:
         seg_tokens = [0, n]
@@ -201,21 +245,17 @@ def dispatch(topk_idx: torch.Tensor, valid_mask: torch.Tensor | None, n_experts:
     L = _lib.lib()
     ws = _dispatch_workspace(dev, int(L.mep_dispatch_workspace_size(n, k, n_experts, n_seg, seg_arr)))
     nk = max(n * k, 1)
-    counts = torch.empty(max(n_local, 1), dtype=torch.int32, device=dev)
-    offsets = torch.empty(n_local + 1, dtype=torch.int32, device=dev)
-    perm = torch.empty(nk, dtype=torch.int32, device=dev)
-    row_of_entry = torch.empty(nk, dtype=torch.int32, device=dev)
     dest = torch.empty(nk, dtype=torch.int32, device=dev) if want_dest else None
+    d = _PackedDispatch(n, k, n_local, dev, dest)
     st = _stream(dev)
     rc = L.mep_dispatch(_ptr(idx), _ptr(vm), n, k, n_experts, table.data_ptr(), n_rep.data_ptr(),
                         table.shape[1], 1 if has_replicas else 0, _ptr(rr), seg_arr, n_seg,
-                        my_rank, g2l.data_ptr(), n_local, counts.data_ptr(), offsets.data_ptr(),
-                        perm.data_ptr(), row_of_entry.data_ptr(), _ptr(dest), _ptr(route_counts),
+                        my_rank, g2l.data_ptr(), n_local, *d.ptrs, _ptr(dest), _ptr(route_counts),
                         ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "mep_dispatch")
     if check:
         _lib.check(L.mep_dispatch_check(ws.data_ptr(), st), "mep_dispatch")
-    return Dispatch(counts[:n_local], offsets, perm, row_of_entry, dest, n, k, n_local)
+    return d
 
 
 def route_dispatch(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, valid_mask: torch.Tensor | None = None,
@@ -226,7 +266,7 @@ def route_dispatch(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, valid_m
     those two calls."""
     dev = _require_device(x_flat, w_router, valid_mask, route_counts)
     x = x_flat.contiguous()
-    w = w_router.to(x.dtype).contiguous()
+    w = _as_dtype(w_router, x.dtype)
     n, h = x.shape
     e = w.shape[0]
     if k != 8:
@@ -247,19 +287,13 @@ def route_dispatch(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, valid_m
     gate = torch.empty((n, k), dtype=x.dtype, device=dev)
     logits = torch.empty((n, e), dtype=torch.float32, device=dev) if return_logits else None
     ws = _dispatch_workspace(dev, int(L.mep_route_dispatch_workspace_size(n, e)))
-    nk = max(n * k, 1)
-    counts = torch.empty(e, dtype=torch.int32, device=dev)
-    offsets = torch.empty(e + 1, dtype=torch.int32, device=dev)
-    perm = torch.empty(nk, dtype=torch.int32, device=dev)
-    row_of_entry = torch.empty(nk, dtype=torch.int32, device=dev)
+    d = _PackedDispatch(n, k, e, dev)
     st = _stream(dev)
     rc = L.mep_route_dispatch(x.data_ptr(), w.data_ptr(), _ptr(vm), n, h, e, k, _dtype_code(x), idx.data_ptr(),
-                              gate.data_ptr(), _ptr(logits), counts.data_ptr(), offsets.data_ptr(), perm.data_ptr(),
-                              row_of_entry.data_ptr(), _ptr(route_counts), ws.data_ptr(), ws.numel(), st)
+                              gate.data_ptr(), _ptr(logits), *d.ptrs, _ptr(route_counts), ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "mep_route_dispatch")
     if check:
         _lib.check(L.mep_dispatch_check(ws.data_ptr(), st), "mep_route_dispatch")
-    d = Dispatch(counts, offsets, perm, row_of_entry, None, n, k, e)
     return (idx, gate, d) + ((logits,) if return_logits else ())
 
 
@@ -285,8 +319,8 @@ def grouped_swiglu(x_flat: torch.Tensor, disp: Dispatch, w_in: torch.Tensor, w_o
     if h_in != h or tuple(w_out.shape) != (e_loc, h, inter) or e_loc != n_w:
         raise ValueError(f"weight shapes {tuple(w_in.shape)} / {tuple(w_out.shape)} do not match "
                          f"hidden {h} and {disp.n_local} local experts")
-    wi = w_in.to(x.dtype).contiguous()
-    wo = w_out.to(x.dtype).contiguous()
+    wi = _as_dtype(w_in, x.dtype)
+    wo = _as_dtype(w_out, x.dtype)
     if y_entries is None:
         y_entries = torch.empty((max(n * disp.top_k, 1), h), dtype=x.dtype, device=dev)
     code = _dtype_code(x)
@@ -296,14 +330,14 @@ def grouped_swiglu(x_flat: torch.Tensor, disp: Dispatch, w_in: torch.Tensor, w_o
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
     tq = _tile_queue(dev, max_rows, disp.n_local)
     if w_slot is None:
-        rc = L.mep_grouped_swiglu(x.data_ptr(), n, disp.top_k, disp.perm.data_ptr(), disp.offsets.data_ptr(),
+        rc = L.mep_grouped_swiglu(x.data_ptr(), n, disp.top_k, _part_ptr(disp, "perm"), _part_ptr(disp, "offsets"),
                                   disp.n_local, max_rows, wi.data_ptr(), wo.data_ptr(), h, inter, code,
                                   y_entries.data_ptr(), ws.data_ptr(), ws.numel(), tq.data_ptr(), tq.numel(),
                                   _stream(dev))
         _lib.check(rc, "mep_grouped_swiglu")
     else:
-        rc = L.mep_grouped_swiglu_slots(x.data_ptr(), n, disp.top_k, disp.perm.data_ptr(),
-                                        disp.offsets.data_ptr(), disp.n_local, max_rows, wi.data_ptr(),
+        rc = L.mep_grouped_swiglu_slots(x.data_ptr(), n, disp.top_k, _part_ptr(disp, "perm"),
+                                        _part_ptr(disp, "offsets"), disp.n_local, max_rows, wi.data_ptr(),
                                         wo.data_ptr(), w_slot.contiguous().data_ptr(), h, inter, code,
                                         y_entries.data_ptr(), ws.data_ptr(), ws.numel(),
                                         tq.data_ptr(), tq.numel(), _stream(dev))
@@ -330,9 +364,9 @@ def grouped_swiglu_combine(x_flat: torch.Tensor, disp: Dispatch, w_in: torch.Ten
                          f"hidden {h} and {disp.n_local} local experts")
     if tuple(topk_gate.shape) != (n, disp.top_k):
         raise ValueError(f"topk_gate {tuple(topk_gate.shape)} does not match {n} tokens x top-{disp.top_k}")
-    wi = w_in.to(x.dtype).contiguous()
-    wo = w_out.to(x.dtype).contiguous()
-    gate = topk_gate.to(x.dtype).contiguous()
+    wi = _as_dtype(w_in, x.dtype)
+    wo = _as_dtype(w_out, x.dtype)
+    gate = _as_dtype(topk_gate, x.dtype)
     vm = _mask_u8(valid_mask, n)
     max_rows = n * disp.top_k
     if y_entries is None:
@@ -344,8 +378,8 @@ def grouped_swiglu_combine(x_flat: torch.Tensor, disp: Dispatch, w_in: torch.Ten
     ws_bytes = L.mep_experts_workspace_size(max_rows, inter, code)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
     tq = _tile_queue(dev, max_rows, disp.n_local)
-    rc = L.mep_grouped_swiglu_combine(x.data_ptr(), n, disp.top_k, disp.perm.data_ptr(), disp.offsets.data_ptr(),
-                                      disp.row_of_entry.data_ptr(), gate.data_ptr(), _ptr(vm), disp.n_local,
+    rc = L.mep_grouped_swiglu_combine(x.data_ptr(), n, disp.top_k, _part_ptr(disp, "perm"), _part_ptr(disp, "offsets"),
+                                      _part_ptr(disp, "row_of_entry"), gate.data_ptr(), _ptr(vm), disp.n_local,
                                       max_rows, wi.data_ptr(), wo.data_ptr(), h, inter, code,
                                       y_entries.data_ptr(), ws.data_ptr(), ws.numel(), tq.data_ptr(), tq.numel(),
                                       out.data_ptr(), _stream(dev))
@@ -364,7 +398,7 @@ def moe_layer(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, w_in: torch.
     dev = _require_device(x_flat, w_router, w_in, w_out, valid_mask, route_counts)
     x = x_flat.contiguous()
     n, h = x.shape
-    w = w_router.to(x.dtype).contiguous()
+    w = _as_dtype(w_router, x.dtype)
     e = w.shape[0]
     if w.shape[1] != h or w_in.dim() != 3 or w_out.dim() != 3:
         raise ValueError("w_router must be (E, H), w_in (E, 2I, H) and w_out (E, H, I)")
@@ -375,37 +409,33 @@ def moe_layer(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, w_in: torch.
                          f"hidden {h} and {e} experts")
     if route_counts is not None and (route_counts.dtype != torch.int64 or route_counts.numel() != e):
         raise TypeError("route_counts must be an int64 tensor of n_experts")
-    wi = w_in.to(x.dtype).contiguous()
-    wo = w_out.to(x.dtype).contiguous()
+    wi = _as_dtype(w_in, x.dtype)
+    wo = _as_dtype(w_out, x.dtype)
     vm = _mask_u8(valid_mask, n)
     L = _lib.lib()
     code = _dtype_code(x)
     idx = torch.empty((n, k), dtype=torch.int64, device=dev)
     gate = torch.empty((n, k), dtype=x.dtype, device=dev)
     logits = torch.empty((n, e), dtype=torch.float32, device=dev) if return_logits else None
-    nk = max(n * k, 1)
-    counts = torch.empty(e, dtype=torch.int32, device=dev)
-    offsets = torch.empty(e + 1, dtype=torch.int32, device=dev)
-    perm = torch.empty(nk, dtype=torch.int32, device=dev)
-    row_of_entry = torch.empty(nk, dtype=torch.int32, device=dev)
-    y = torch.empty((nk, h), dtype=x.dtype, device=dev)
+    d = _PackedDispatch(n, k, e, dev)
     out = torch.empty((n, h), dtype=x.dtype, device=dev)
+    st = _stream(dev)
     dws = _dispatch_workspace(dev, int(L.mep_route_dispatch_workspace_size(n, e)))
     max_rows = n * k
-    ews = torch.empty(max(int(L.mep_experts_workspace_size(max_rows, inter, code)), 256), dtype=torch.uint8,
-                      device=dev)
+    # scratch of this call only: the experts' rows, then their workspace (act)
+    y_bytes = (max(max_rows, 1) * h * x.element_size() + 255) // 256 * 256
+    ews_bytes = max(int(L.mep_experts_workspace_size(max_rows, inter, code)), 256)
+    scratch = torch.empty(y_bytes + ews_bytes, dtype=torch.uint8, device=dev)
+    y = scratch.data_ptr()
     need = int(L.mep_moe_layer_queue_ints(n, e, h))
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(dev))
+    key = (_index(dev), st)
     tq = _QUEUES.get(key)
     if tq is None or tq.numel() < need:
         tq = _QUEUES[key] = torch.zeros(max(need, 64), dtype=torch.int32, device=dev)
     rc = L.mep_moe_layer(x.data_ptr(), w.data_ptr(), _ptr(vm), n, h, e, k, code, wi.data_ptr(), wo.data_ptr(), inter,
-                         idx.data_ptr(), gate.data_ptr(), _ptr(logits), counts.data_ptr(), offsets.data_ptr(),
-                         perm.data_ptr(), row_of_entry.data_ptr(), _ptr(route_counts), y.data_ptr(), dws.data_ptr(),
-                         dws.numel(), ews.data_ptr(), ews.numel(), tq.data_ptr(), tq.numel(), out.data_ptr(),
-                         _stream(dev))
+                         idx.data_ptr(), gate.data_ptr(), _ptr(logits), *d.ptrs, _ptr(route_counts), y, dws.data_ptr(),
+                         dws.numel(), y + y_bytes, ews_bytes, tq.data_ptr(), tq.numel(), out.data_ptr(), st)
     _lib.check(rc, "mep_moe_layer")
-    d = Dispatch(counts, offsets, perm, row_of_entry, None, n, k, e)
     return (out, idx, gate, d) + ((logits,) if return_logits else ())
 
 
@@ -453,10 +483,10 @@ def swiglu_gate_up(x_flat: torch.Tensor, disp: Dispatch, w_in: torch.Tensor,
     n, h, inter = _expert_shapes(x, disp, w_in=w_in)
     if act is None:
         act = torch.empty((max(n * disp.top_k, 1), inter), dtype=x.dtype, device=dev)
-    wi = w_in.to(x.dtype).contiguous()
+    wi = _as_dtype(w_in, x.dtype)
     tq = _tile_queue(dev, n * disp.top_k, disp.n_local)
-    rc = _lib.lib().mep_swiglu_gate_up(x.data_ptr(), n, disp.top_k, disp.perm.data_ptr(),
-                                       disp.offsets.data_ptr(), disp.n_local, n * disp.top_k,
+    rc = _lib.lib().mep_swiglu_gate_up(x.data_ptr(), n, disp.top_k, _part_ptr(disp, "perm"),
+                                       _part_ptr(disp, "offsets"), disp.n_local, n * disp.top_k,
                                        wi.data_ptr(), h, inter, _dtype_code(x), act.data_ptr(),
                                        act.numel() * act.element_size(), tq.data_ptr(), tq.numel(),
                                        _stream(dev))
@@ -471,10 +501,10 @@ def swiglu_down(act: torch.Tensor, x_flat: torch.Tensor, disp: Dispatch, w_out: 
     n, h, inter = _expert_shapes(x_flat, disp, w_out=w_out)
     if y_entries is None:
         y_entries = torch.empty((max(n * disp.top_k, 1), h), dtype=act.dtype, device=dev)
-    wo = w_out.to(act.dtype).contiguous()
+    wo = _as_dtype(w_out, act.dtype)
     tq = _tile_queue(dev, n * disp.top_k, disp.n_local)
-    rc = _lib.lib().mep_swiglu_down(act.data_ptr(), n, disp.top_k, disp.perm.data_ptr(),
-                                    disp.offsets.data_ptr(), disp.n_local, n * disp.top_k, wo.data_ptr(),
+    rc = _lib.lib().mep_swiglu_down(act.data_ptr(), n, disp.top_k, _part_ptr(disp, "perm"),
+                                    _part_ptr(disp, "offsets"), disp.n_local, n * disp.top_k, wo.data_ptr(),
                                     h, inter, _dtype_code(act), y_entries.data_ptr(),
                                     tq.data_ptr(), tq.numel(), _stream(dev))
     _lib.check(rc, "mep_swiglu_down")
@@ -487,7 +517,7 @@ def combine(y_entries: torch.Tensor, topk_gate: torch.Tensor, row_of_entry: torc
     dev = _require_device(y_entries, topk_gate, row_of_entry, out)
     n, k = topk_gate.shape
     h = y_entries.shape[1]
-    gate = topk_gate.to(y_entries.dtype).contiguous()
+    gate = _as_dtype(topk_gate, y_entries.dtype)
     vm = _mask_u8(valid_mask, n)
     if out is None:
         out = torch.empty((n, h), dtype=y_entries.dtype, device=dev)
@@ -504,7 +534,7 @@ def combine_rows(y_rows: torch.Tensor, topk_gate: torch.Tensor, row_of_entry: to
     dev = _require_device(y_rows, topk_gate, row_of_entry, out)
     n, k = topk_gate.shape
     h = y_rows.shape[1]
-    gate = topk_gate.to(y_rows.dtype).contiguous()
+    gate = _as_dtype(topk_gate, y_rows.dtype)
     vm = _mask_u8(valid_mask, n)
     if out is None:
         out = torch.empty((n, h), dtype=y_rows.dtype, device=dev)
@@ -525,7 +555,7 @@ def gather_rows(x: torch.Tensor, perm: torch.Tensor, n_rows: int, top_k: int,
     ids = None
     flat = None
     if topk_idx is not None:
-        flat = topk_idx.reshape(-1).to(torch.int64).contiguous()
+        flat = _as_dtype(topk_idx.reshape(-1), torch.int64)
         ids = torch.empty(n_rows, dtype=torch.int64, device=dev)
     rc = _lib.lib().mep_gather_rows(x.data_ptr(), n, top_k, perm.data_ptr(), n_rows, h, _dtype_code(x),
                                     _ptr(flat), _ptr(ids), out.data_ptr(), _stream(dev))
@@ -637,7 +667,8 @@ def norm_head(h: torch.Tensor, delta: torch.Tensor | None, mult: float, norm: to
         if t.dtype != torch.bfloat16 or not t.is_contiguous():
             raise TypeError("norm_head takes contiguous bf16 tensors")
     n, hidden = h.shape
-    if norm.shape != (hidden,) or w.dim() != 2 or w.shape[1] != hidden or (delta is not None and delta.shape != h.shape):
+    if norm.shape != (hidden,) or w.dim() != 2 or w.shape[1] != hidden or \
+            (delta is not None and delta.shape != h.shape):
         raise ValueError("norm_head: shapes do not match")
     logits = torch.empty((n, w.shape[0]), dtype=torch.float32, device=dev)
     rc = _lib.lib().mep_norm_head(h.data_ptr(), _ptr(delta), mult, norm.data_ptr(), eps, w.data_ptr(), n, hidden,
