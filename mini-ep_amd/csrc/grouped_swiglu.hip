@@ -25,7 +25,9 @@
 // columns of one row.  GEMM-1 applies SiLU * up in registers and stores 16 B
 // per lane; GEMM-2 regroups rows through a per-wave LDS slice into whole
 // 128-byte lines and stores them non-temporally (y_entries is read once, by
-// the combine).  fp32 keeps the simpler two-stage grouped_gemm_kernel.
+// the combine).  fp32 runs moe_gemm_mid_kernel; grouped_gemm_kernel, simpler
+// and in two stages, serves the separate GEMM calls in fp32 and GEMM-2 in bf16
+// with an intermediate size that is no multiple of 256.
 //
 // Scheduling (bf16, larger batches): persistent, one workgroup per CU,
 // both GEMMs in one launch (kModeBoth; kModeGateUp / kModeDown run one of
@@ -528,8 +530,8 @@ static_assert(BPW == NF, "one DMA block per MFMA group of an odd step");
 //   line 16 + r      row tile r's GEMM-1 column tiles finished (kModeBoth);
 //                    the small-batch launch of both GEMMs: chunk r's GEMM-1
 //                    counts and GEMM-2 workgroups past their wait (words 0,
-//                    1); the mid-size one: those of chunks 4 r .. 4 r + 3
-//                    (words 0, 1 of each quarter line)
+//                    1); the mid-size one: those of chunks 8 r .. 8 r + 7
+//                    (words 0, 1 of each eighth of the line)
 // Every launch leaves every word but the flags zero.
 namespace sched {
 constexpr int kLine = 32;                      // ints per 128-byte line
@@ -537,14 +539,14 @@ constexpr int kQueue = 0, kDone = 8 * kLine, kItems = 9 * kLine, kFlags = 10 * k
               kG2Done = 12 * kLine, kCombDone = 13 * kLine, kRowDone = 16 * kLine;
 __host__ __device__ constexpr int queue_word(int q) { return kQueue + q * kLine; }
 __host__ __device__ constexpr int row_word(int r) { return kRowDone + r * kLine; }
-__host__ __device__ constexpr int mid_word(int q) { return row_word(q >> 2) + (q & 3) * (kLine / 4); }
+__host__ __device__ constexpr int mid_word(int q) { return row_word(q >> 3) + (q & 7) * (kLine / 8); }
 constexpr int kFlagWait = 1, kFlagDrain = 2, kFlagInput = kFlagInputBit;
 constexpr int kWaitLimit = 1 << 20;            // polls of one row counter (about a second)
 // the small-batch launch of both GEMMs runs up to this many rows
 constexpr int64_t kSmallRows = 1024;
 // row tiles of max_rows rows over n_local experts: each expert adds at most
 // one partial tile; the small-batch launch of both GEMMs keeps a line per
-// 32-row chunk there instead, the mid-size one a line per four chunks
+// 32-row chunk there instead, the mid-size one a line per eight chunks
 inline int64_t words(int64_t max_rows, int n_local) {
   const int64_t tiles = (max_rows + 255) / 256 + n_local;
   const int64_t chunks = max_rows <= kSmallRows ? (max_rows + 31) / 32 + n_local : 0;
@@ -1869,8 +1871,8 @@ hipError_t launch_skinny_both(const GemmParams& p1, const GemmParams& p2, int64_
 }
 
 // ============================================================================
-// bf16 path for some tens to a few hundred rows per expert (a prompt or a
-// large decode batch): one workgroup per (chunk of 16 MFC rows of one local
+// Some tens to a few hundred rows per expert in bf16 (a prompt or a large
+// decode batch), every size in fp32: one workgroup per (chunk of 16 MFC rows of one local
 // expert, column block of 64 act / 128 output columns), both GEMMs in one
 // launch.
 //
@@ -1887,7 +1889,7 @@ hipError_t launch_skinny_both(const GemmParams& p1, const GemmParams& p2, int64_
 // the MFMA layout, as the small-batch kernel does, put 16 rows under 16
 // neighbouring lanes: 64 L1 lookups per KiB instead of 8 to 16, which bound
 // the loop once a weight row met more than some 64 rows: 171 us at 4096
-// tokens of the GraniteMoE layer.)  Plain loads and LDS writes, not LDS DMA: the
+// tokens of the GraniteMoE layer in bf16, 143 so.)  Plain loads and LDS writes, not LDS DMA: the
 // compiler waits for every load in flight before reading LDS that a DMA may
 // have written.  The ring holds MFMA fragments of 1 KiB, lane (lr, lg)'s 16
 // bytes in slot 16 lg + (lr ^ lg ^ 12 (step & 1)); a copying lane group takes
@@ -1909,11 +1911,26 @@ constexpr int WF = 8;                         // weight fragments of a workgroup
 inline int64_t chunks(int64_t max_rows, int n_local, int rows) { return (max_rows + rows - 1) / rows + n_local; }
 }  // namespace mid
 
+// One K-step (64 bytes of every row) of a fragment pair: 32 bf16 in one MFMA,
+// or 16 floats in four, MFMA q on elements 4 lg + q of the lane groups (the
+// order of grouped_gemm_kernel).
+template <int DT>
+__device__ __forceinline__ void mid_mfma(f32x4& acc, const u32x4& w, const u32x4& a) {
+  if constexpr (DT == MEP_DTYPE_BF16) {
+    mfma_acc(acc, w, a);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+v"(acc) : "v"(w[q]), "v"(a[q]));
+  }
+}
+
 // Column block cb of chunk q: rows [row_lo, row_hi) of expert e, at most 16 MFC.
-template <int MFC, bool GEMM1>
+template <int DT, int MFC, bool GEMM1>
 __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int cb, int n_cb, int row_lo, int row_hi,
                                           int n_cb_other, int* sched, unsigned char* s_ring, int* s_gave) {
-  typedef uint16_t T;
+  typedef typename Elem<DT>::T T;
+  constexpr int EB = Elem<DT>::kBytes;
   constexpr int AHEAD = mid::AHEAD;
   constexpr int MF = MFC / 2, NF = 4;                         // row and weight fragments per wave
   constexpr int AP = MFC / 2, WP = mid::WF / 2;               // copy passes of 32 rows
@@ -1921,12 +1938,12 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int lr = lane & 15, lg = lane >> 4;
-  const int K = p.K, NB = K / 64, KD = K / 64;                // blocks of two K-steps
-  const int nt = cb / 2;                                      // the tiled kernel's column tile and K rotation
-  const int rot = (!GEMM1 && KD % 4 == 0) ? (nt & 3) * (KD / 4) : 0;
+  const int row_bytes = p.K * EB, NB = row_bytes / 128;       // blocks of two K-steps
+  // bf16: the tiled kernel's column tile (cb / 2) and its K rotation
+  const int rot = (DT == MEP_DTYPE_BF16 && !GEMM1 && NB % 4 == 0) ? ((cb / 2) & 3) * (NB / 4) : 0;
   const int slot = p.w_slot != nullptr ? p.w_slot[e] : e;
   const unsigned char* const W =
-      static_cast<const unsigned char*>(p.W) + static_cast<int64_t>(slot) * p.w_expert_stride * 2;
+      static_cast<const unsigned char*>(p.W) + static_cast<int64_t>(slot) * p.w_expert_stride * EB;
   const unsigned char* const A = static_cast<const unsigned char*>(p.A);
 
   // ---- copies: this thread's row of a pass and 16-byte chunk of its line -----------
@@ -1944,7 +1961,7 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
     const int in32 = 8 * (c16 >> 2) + 4 * (j & 1) + (c16 & 3);
     const int row = GEMM1 ? (j >= 2 ? p.N : 0) + cb * 64 + 32 * (fr >> 2) + in32
                           : cb * 128 + 64 * (fr >> 2) + 32 * (j >> 1) + in32;
-    w_off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K * 2) + cc * 16;
+    w_off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(row_bytes) + cc * 16;
   }
   u32x4 wr[AHEAD][WP], ar[AHEAD][AP];
   auto line = [&](int b) {                                    // byte offset of block b's line of a row
@@ -2000,7 +2017,7 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
       const uint32_t f = static_cast<uint32_t>(p.perm[r]);    // flat entry t*k + s
       from = p.k_magic ? (__umulhi(f, p.k_magic) >> p.k_shift) : f;
     }
-    a_off[i] = from * static_cast<uint32_t>(K * 2) + cc * 16;
+    a_off[i] = from * static_cast<uint32_t>(row_bytes) + cc * 16;
   }
 #pragma unroll
   for (int b = 0; b < AHEAD; ++b) load_a(b, ar[b]);
@@ -2051,7 +2068,7 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
         for (int j = 0; j < NF; ++j) {
 #pragma unroll
           for (int i = 0; i < MF; ++i) {
-            mfma_acc(acc[i][j], w[j], a[i]);
+            mid_mfma<DT>(acc[i][j], w[j], a[i]);
             if (refill && j == NF - 1) read_a(next, i);
           }
           if (refill) read_w(next, j);
@@ -2069,7 +2086,7 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
   for (int i = 0; i < MF; ++i) read_a(frag0, i);
 #pragma unroll
   for (int j = 0; j < NF; ++j) read_w(frag0, j);
-  const int rounds = NB / ROUND;                              // K is a multiple of 256
+  const int rounds = NB / ROUND;                              // NB is even and at least 4 (the host checks)
   round(0, std::integral_constant<bool, false>());
   for (int r = 1; r < rounds - 1; ++r) round(r, std::integral_constant<bool, false>());
   round(rounds - 1, std::integral_constant<bool, true>());
@@ -2095,25 +2112,26 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
     const int r = row_lo + (wm * MF + i) * 16 + lr;
     if (r >= row_hi) continue;
     if constexpr (GEMM1) {
-      u32x4 o;
+      float v[8];
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const f32x4 g = acc[i][h >> 1], up = acc[i][2 + (h >> 1)];
-        o[h] = pack_bf16x2(silu_f(g[2 * (h & 1)]) * up[2 * (h & 1)], silu_f(g[2 * (h & 1) + 1]) * up[2 * (h & 1) + 1]);
-      }
+      for (int c = 0; c < 8; ++c) v[c] = silu_f(acc[i][c >> 2][c & 3]) * acc[i][2 + (c >> 2)][c & 3];
       // device scope, so GEMM-2 on any XCD reads the final rows
-      store_dev_16(p.C, p.c_bytes, static_cast<uint32_t>(r * p.N + cb * 64 + 32 * wn + 8 * lg) * 2u, o);
+      const uint32_t at = static_cast<uint32_t>(r * p.N + cb * 64 + 32 * wn + 8 * lg) * static_cast<uint32_t>(EB);
+      if constexpr (DT == MEP_DTYPE_BF16) {
+        store_dev_16(p.C, p.c_bytes, at, pack_row_chunk<DT>(v));
+      } else {
+        store_dev_16(p.C, p.c_bytes, at, pack_row_chunk<DT>(v));
+        store_dev_16(p.C, p.c_bytes, at + 16, pack_row_chunk<DT>(v + 4));
+      }
     } else {
       T* const dst = C + static_cast<int64_t>(p.perm[r]) * p.N + cb * 128 + 64 * wn + 8 * lg;
 #pragma unroll
       for (int jp = 0; jp < 2; ++jp) {
-        u32x4 o;
+        float v[8];
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const f32x4 v = acc[i][2 * jp + (h >> 1)];
-          o[h] = pack_bf16x2(v[2 * (h & 1)], v[2 * (h & 1) + 1]);
-        }
-        *reinterpret_cast<u32x4*>(dst + 32 * jp) = o;
+        for (int c = 0; c < 8; ++c) v[c] = acc[i][2 * jp + (c >> 2)][c & 3];
+        *reinterpret_cast<u32x4*>(dst + 32 * jp) = pack_row_chunk<DT>(v);
+        if constexpr (DT == MEP_DTYPE_F32) *reinterpret_cast<u32x4*>(dst + 32 * jp + 4) = pack_row_chunk<DT>(v + 4);
       }
     }
   }
@@ -2133,7 +2151,7 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
 }
 
 // Workgroup `unit` of one GEMM: its chunk and column block.
-template <int MFC, bool GEMM1>
+template <int DT, int MFC, bool GEMM1>
 __device__ __forceinline__ void mid_body(const GemmParams& p, int unit, int n_cb_other, int* sched, int* s_pre,
                                          int* s_off, unsigned char* s_ring, int* s_gave) {
   constexpr int CH = 16 * MFC;
@@ -2164,13 +2182,14 @@ __device__ __forceinline__ void mid_body(const GemmParams& p, int unit, int n_cb
   const int row_lo = __builtin_amdgcn_readfirstlane(s_off[e] + (q - s_pre[e]) * CH);
   const int row_hi = __builtin_amdgcn_readfirstlane(min(s_off[e + 1], row_lo + CH));
   // an expert's last chunk is often short: half the row fragments then
-  if (row_hi - row_lo <= CH / 2)
-    mid_chunk<MFC / 2, GEMM1>(p, e, q, cb, n_cb, row_lo, row_hi, n_cb_other, sched, s_ring, s_gave);
-  else
-    mid_chunk<MFC, GEMM1>(p, e, q, cb, n_cb, row_lo, row_hi, n_cb_other, sched, s_ring, s_gave);
+  if constexpr (MFC > 2) {
+    if (row_hi - row_lo <= CH / 2)
+      return mid_chunk<DT, MFC / 2, GEMM1>(p, e, q, cb, n_cb, row_lo, row_hi, n_cb_other, sched, s_ring, s_gave);
+  }
+  mid_chunk<DT, MFC, GEMM1>(p, e, q, cb, n_cb, row_lo, row_hi, n_cb_other, sched, s_ring, s_gave);
 }
 
-template <int MFC>
+template <int DT, int MFC>
 __global__ __launch_bounds__(mid::NT, 2) void moe_gemm_mid_kernel(GemmParams p1, GemmParams p2, int g1_blocks,
                                                                   int* sched) {
   __shared__ int s_pre[bfk::NLMAX + 1];
@@ -2178,16 +2197,16 @@ __global__ __launch_bounds__(mid::NT, 2) void moe_gemm_mid_kernel(GemmParams p1,
   __shared__ __attribute__((aligned(16))) unsigned char s_ring[4 * (MFC + mid::WF) * 1024];
   __shared__ int s_gave;
   const int b = blockIdx.x;
-  if (b < g1_blocks) mid_body<MFC, true>(p1, b, 0, sched, s_pre, s_off, s_ring, &s_gave);
-  else mid_body<MFC, false>(p2, b - g1_blocks, p1.N / 64, sched, s_pre, s_off, s_ring, &s_gave);
+  if (b < g1_blocks) mid_body<DT, MFC, true>(p1, b, 0, sched, s_pre, s_off, s_ring, &s_gave);
+  else mid_body<DT, MFC, false>(p2, b - g1_blocks, p1.N / 64, sched, s_pre, s_off, s_ring, &s_gave);
 }
 
-template <int MFC>
+template <int DT, int MFC>
 hipError_t launch_mid(const GemmParams& p1, const GemmParams& p2, int64_t max_rows, int* sched, hipStream_t stream) {
   // an XCD's range is at most ceil(chunks / 8) chunks
   const int64_t per_xcd = (mid::chunks(max_rows, p1.n_local, 16 * MFC) + 7) / 8;
   const int64_t b1 = 8 * per_xcd * (p1.N / 64), b2 = 8 * per_xcd * (p2.N / 128);
-  moe_gemm_mid_kernel<MFC><<<dim3(static_cast<unsigned>(b1 + b2)), mid::NT, 0, stream>>>(
+  moe_gemm_mid_kernel<DT, MFC><<<dim3(static_cast<unsigned>(b1 + b2)), mid::NT, 0, stream>>>(
       p1, p2, static_cast<int>(b1), sched);
   return hipGetLastError();
 }
@@ -2863,6 +2882,17 @@ int mid_row_frags(int64_t max_rows, int n_local, int inter) {
   return max_rows >= static_cast<int64_t>(n_local) * 64 && units >= (sparse ? cu : 2 * cu) ? 8 : 4;
 }
 
+// fp32, every size: chunks of 64 rows, or of 32 while those of 64 are too few
+// to fill the chip twice (an fp32 MFMA is 8 times slower than a bf16 one, so
+// padding rows cost more than reading the weights again).  us of one call
+// against the two launches of 128 x 128 tiles, GraniteMoE's experts: 1 token
+// 109 -> 40, 32: 116 -> 53, 128: 114 -> 70 (64-row chunks: 107), 256: 217 ->
+// 91, 512: 216 -> 140, 1500: 424 -> 325 (32-row chunks: 350), 4096: 946 -> 802.
+int mid_row_frags_f32(int64_t max_rows, int n_local, int inter) {
+  const int64_t units = (max_rows / 64 + n_local / 2) * (inter / 64);
+  return units >= 2 * device_cu_count() ? 4 : 2;
+}
+
 // Tile shapes of the generic kernel (fp32, and bf16 GEMM-2 with I % 256 != 0):
 // bf16 256x256 on 8 waves (4 x 2), fp32 128x128 on 4 waves.
 typedef TileCfg<256, 256, 4, 2> CfgBf16;
@@ -3042,23 +3072,33 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
   const size_t need = mep_experts_workspace_size(max_rows, inter, dtype);
   MEP_REQUIRE(workspace_bytes >= need, MEP_ERR_WORKSPACE, "%s: workspace %zu B < required %zu B", fn,
               workspace_bytes, need);
-  const int mid_frags = dtype == MEP_DTYPE_BF16 && inter % 256 == 0 ? mid_row_frags(max_rows, n_local, inter) : 0;
+  int mid_frags = 0;
+  if (dtype == MEP_DTYPE_BF16 && inter % 256 == 0) mid_frags = mid_row_frags(max_rows, n_local, inter);
+  // (fp32's two launches take any schedule buffer: a smaller one keeps them)
+  else if (dtype == MEP_DTYPE_F32 && static_cast<int64_t>(tile_queue_ints) >= sched::words(max_rows, n_local))
+    mid_frags = mid_row_frags_f32(max_rows, n_local, inter);
   if (mid_frags > 0) {
     MEP_REQUIRE(x && perm && offsets && w_in && w_out && y_entries, MEP_ERR_INVALID_ARG, "%s: null pointer", fn);
     rc = check_queue(fn, true, tile_queue, tile_queue_ints, max_rows, n_local);
     if (rc != MEP_OK) return rc;
     MEP_REQUIRE(aligned16(x) && aligned16(w_in) && aligned16(w_out) && aligned16(workspace) && aligned16(y_entries),
                 MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
-    GemmParams g1 = gemm1_params<MEP_DTYPE_BF16, CfgBf16>(x, n_tokens, top_k, perm, offsets, n_local, w_in, w_slot,
-                                                          hidden, inter, workspace);
-    GemmParams g2 = gemm2_params<MEP_DTYPE_BF16, CfgBf16>(workspace, top_k, perm, offsets, n_local, max_rows, w_out,
-                                                          w_slot, hidden, inter, y_entries);
-    set_sched(g1, tile_queue);
-    set_sched(g2, tile_queue);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    g1.c_bytes = static_cast<uint32_t>(max_rows * inter * 2);
-    const hipError_t e = mid_frags == 4 ? launch_mid<4>(g1, g2, max_rows, tile_queue, s)
-                                        : launch_mid<8>(g1, g2, max_rows, tile_queue, s);
+    auto run = [&](auto dt) {
+      constexpr int DT = decltype(dt)::value;
+      GemmParams g1 = gemm1_params<DT, CfgBf16>(x, n_tokens, top_k, perm, offsets, n_local, w_in, w_slot, hidden, inter,
+                                                workspace);
+      GemmParams g2 = gemm2_params<DT, CfgBf16>(workspace, top_k, perm, offsets, n_local, max_rows, w_out, w_slot, hidden,
+                                                inter, y_entries);
+      set_sched(g1, tile_queue);
+      set_sched(g2, tile_queue);
+      g1.c_bytes = static_cast<uint32_t>(max_rows * inter * dtype_bytes(DT));
+      hipStream_t s = static_cast<hipStream_t>(stream);
+      constexpr int LOW = DT == MEP_DTYPE_F32 ? 2 : 4, HIGH = 2 * LOW;   // the row fragments the rules choose from
+      return mid_frags == LOW ? launch_mid<DT, LOW>(g1, g2, max_rows, tile_queue, s)
+                              : launch_mid<DT, HIGH>(g1, g2, max_rows, tile_queue, s);
+    };
+    const hipError_t e = dtype == MEP_DTYPE_BF16 ? run(std::integral_constant<int, MEP_DTYPE_BF16>())
+                                                 : run(std::integral_constant<int, MEP_DTYPE_F32>());
     MEP_REQUIRE(e == hipSuccess, MEP_ERR_HIP, "%s: %s", fn, hipGetErrorString(e));
     return MEP_OK;
   }

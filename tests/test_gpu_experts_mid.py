@@ -1,5 +1,5 @@
-"""The mid-size experts launch (some tens to a few hundred rows per expert,
-both GEMMs in one launch): the bits of the two separate launches on every
+"""The mid-size experts launch (some tens to a few hundred rows per expert in
+bf16, any in fp32; both GEMMs in one launch): the bits of the two separate launches on every
 row, at row counts around the edges of its 16-row fragments, half chunks and
 chunks, with few and many experts, and a wait that gives up."""
 import numpy as np
@@ -16,18 +16,22 @@ DEV = "cuda"
 BF = torch.bfloat16
 
 
-def _case(counts, k, H, I, seed):
+def _case(counts, k, H, I, seed, dtype=BF):
     E, n = len(counts), sum(counts) // k
     topk = _topk_with_counts(counts, k, n, seed)
     g = torch.Generator().manual_seed(seed)
-    x = torch.randn(n, H, generator=g).to(BF).to(DEV)
+    x = torch.randn(n, H, generator=g).to(dtype).to(DEV)
     w_in, w_out = workloads.expert_weights(g, E, H, I)
     table, n_rep, g2l = _world1(E)
     d = ops.dispatch(topk.to(DEV), None, E, table, n_rep, False, None, 0, g2l, E)
-    return x, d, w_in.to(BF).to(DEV), w_out.to(BF).to(DEV)
+    return x, d, w_in.to(dtype).to(DEV), w_out.to(dtype).to(DEV)
 
 
 @pytest.mark.parametrize("name,counts,k,H,I", [
+    # fp32 (names "f32..."): 32-row chunks, the shortest K loop (128 floats); 64-row chunks with short last ones
+    ("f32_edges32", [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 3], 2, 256, 128),
+    ("f32_one_row", [1], 1, 1024, 512),
+    ("f32_edges64", [64, 1, 127, 128, 129, 63, 65, 16, 33, 31, 96, 97] * 2, 2, 512, 2048),
     # 64-row chunks: empty experts, 1 row, around fragments, halves and chunks
     ("edges64", [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 13], 4, 1024, 512),
     # 128-row chunks: an average of 64 rows and more, enough column blocks
@@ -39,13 +43,14 @@ def _case(counts, k, H, I, seed):
 ])
 def test_mid_launch_equals_two_launches(name, counts, k, H, I):
     banner(f"mid-size experts launch: {name}")
-    x, d, wi, wo = _case(counts, k, H, I, len(counts))
+    f32 = name.startswith("f32")
+    x, d, wi, wo = _case(counts, k, H, I, len(counts), torch.float32 if f32 else BF)
     n = x.shape[0]
-    assert n * k > 256
+    assert f32 or n * k > 256
     results = []
     for rep in range(2):                                            # a second input through the same buffers
-        xr = x if rep == 0 else x.flip(0).contiguous()
-        y1 = torch.full((n * k, H), 7.0, dtype=BF, device=DEV)
+        xr = x if rep == 0 else -x.flip(0).contiguous()
+        y1 = torch.full((n * k, H), 7.0, dtype=x.dtype, device=DEV)
         y2 = y1.clone()
         ops.grouped_swiglu(xr, d, wi, wo, y1)
         _two_launches(xr, d, wi, wo, y2)
@@ -102,3 +107,20 @@ def test_mid_launch_giveup():
     ops.grouped_swiglu(x, d, wi, wo, y2)
     ops.experts_check()
     assert torch.equal(y2, y0)
+
+
+def test_f32_small_schedule_buffer():
+    """fp32 calls with a schedule buffer below mep_experts_queue_ints keep the
+    two launches, which take any: same bits."""
+    banner("experts fp32: small schedule buffer")
+    x, d, wi, wo = _case([40, 3, 0, 21], 1, 256, 128, 9, torch.float32)
+    L = _lib.lib()
+    n, H, I = x.shape[0], 256, 128
+    want = ops.grouped_swiglu(x, d, wi, wo)
+    got = torch.empty_like(want)
+    ws = torch.empty(L.mep_experts_workspace_size(n, I, _lib.DTYPE_F32), dtype=torch.uint8, device=DEV)
+    tq = torch.zeros(64, dtype=torch.int32, device=DEV)
+    rc = L.mep_grouped_swiglu(x.data_ptr(), n, 1, d.perm.data_ptr(), d.offsets.data_ptr(), 4, n, wi.data_ptr(),
+                              wo.data_ptr(), H, I, _lib.DTYPE_F32, got.data_ptr(), ws.data_ptr(), ws.numel(),
+                              tq.data_ptr(), tq.numel(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(got, want) and int(tq.abs().sum()) == 0
