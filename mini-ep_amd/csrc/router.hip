@@ -132,6 +132,124 @@ __global__ __launch_bounds__(kWaves * 64) void router_kernel(const typename Elem
                          topk_idx, gate, logits, hist);
 }
 
+// The router with 16 tokens per workgroup, for the shapes without a kernel of
+// their own and batches that give the 64-token kernels too few workgroups.
+//
+// A batch of some hundred tokens is bound by latency: router_kernel runs it on
+// a few CUs, each walking K in segments whose loads are waited for before the
+// next segment's go out, and reads x in the MFMA layout (16 rows under 16
+// neighbouring lanes: 64 L1 lookups per KiB).  Here the workgroup's 16 + E rows
+// go through LDS 512 bytes of each at a time, copied in whole lines with
+// AHEAD blocks of loads in flight in registers, and the waves split the
+// experts (wave w the 16 of fragment w), which also shortens the fp32 MFMA
+// chain.  LDS rows are 128 bytes, chunk c of row r at c ^ (r & 7): conflict-
+// free.  K order, MFMA and operands are router_kernel's, so the logits have its
+// bits.
+constexpr int kAhead16 = 4;
+
+template <int DT, int NF, int KC>
+__global__ __launch_bounds__(kWaves * 64, 1) void router16_kernel(const typename Elem<DT>::T* __restrict__ x,
+                                                                  const typename Elem<DT>::T* __restrict__ w,
+                                                                  int64_t n_tokens, int hidden, int k,
+                                                                  int64_t* __restrict__ topk_idx,
+                                                                  typename Elem<DT>::T* __restrict__ gate,
+                                                                  float* __restrict__ logits) {
+  constexpr int E = NF * 16, R = kRowsPerWave + E;            // rows in LDS: tokens, then experts
+  constexpr int EB = Elem<DT>::kBytes, kBlock = 512;          // bytes of a row per block
+  constexpr int kLineRows = R * 128;                          // one line of every row
+  constexpr int kPasses = R * 4 / 32;                         // copies of a thread per block: 8 lanes per line
+  __shared__ __attribute__((aligned(16))) unsigned char s_ring[2][4 * kLineRows];
+  __shared__ float lg[kRowsPerWave][E + 1];
+  __shared__ __attribute__((aligned(16))) uint64_t keys[kRowsPerWave * (E + 2)];
+  __shared__ __attribute__((aligned(16))) float sel_val[kRowsPerWave * 64];
+  __shared__ int sel_idx[kRowsPerWave * 64];
+  __shared__ float rsum[kRowsPerWave];
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kRowsPerWave;
+  const int row_bytes = hidden * EB, NB = row_bytes / kBlock;
+
+  // copy i of this thread: 16-byte chunk tid % 8 of line `item` % 4 of row
+  // `item` / 4, item = 32 i + tid / 8, so neighbouring lane groups read one row on
+  const unsigned char* src[kPasses];
+  int dst[kPasses];
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) {
+    const int item = 32 * i + (tid >> 3), row = item >> 2, line = item & 3, c = tid & 7;
+    const int64_t tok = t0 + row < n_tokens ? t0 + row : n_tokens - 1;      // in-bounds read, result discarded
+    src[i] = (row < kRowsPerWave ? reinterpret_cast<const unsigned char*>(x) + tok * row_bytes
+                                 : reinterpret_cast<const unsigned char*>(w) +
+                                       static_cast<int64_t>(row - kRowsPerWave) * row_bytes) +
+             line * 128 + c * 16;
+    dst[i] = line * kLineRows + row * 128 + ((c ^ (row & 7)) << 4);
+  }
+  u32x4 v[kAhead16][kPasses];
+  auto load = [&](int b, u32x4 (&to)[kPasses]) {
+    const int64_t off = static_cast<int64_t>(b < NB ? b : NB - 1) * kBlock;   // past the end: in bounds, unused
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) to[i] = *reinterpret_cast<const u32x4*>(src[i] + off);
+  };
+#pragma unroll
+  for (int b = 0; b < kAhead16; ++b) load(b, v[b]);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int nf = wave < NF ? wave : NF - 1;                    // (a wave past the fragments repeats the last one's)
+  // One barrier a block: the other slot's readers are past the barrier before
+  // it is written again.
+  for (int b0 = 0; b0 < NB; b0 += kAhead16) {
+#pragma unroll
+    for (int u = 0; u < kAhead16; ++u) {
+      const int b = b0 + u;
+      if (b >= NB) break;
+      unsigned char* const ring = s_ring[u & 1];
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) *reinterpret_cast<u32x4*>(ring + dst[i]) = v[u][i];
+      load(b + kAhead16, v[u]);
+      __builtin_amdgcn_s_waitcnt(0xC07F);                      // lgkmcnt(0): this wave's copies are in LDS
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const unsigned char* const line = ring + (j >> 1) * kLineRows;
+        const int c = ((4 * (j & 1) + g) ^ (r & 7)) << 4;      // rows r and 16 + 16 nf + r share r & 7
+        const u32x4 xv = *reinterpret_cast<const u32x4*>(line + r * 128 + c);
+        const u32x4 wv = *reinterpret_cast<const u32x4*>(line + (kRowsPerWave + nf * 16 + r) * 128 + c);
+        if constexpr (DT == MEP_DTYPE_BF16) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xv), __builtin_bit_cast(bf16x8, wv),
+                                                        acc, 0, 0, 0);
+        } else {
+          const float* xf = reinterpret_cast<const float*>(&xv);
+          const float* wf = reinterpret_cast<const float*>(&wv);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[q], wf[q], acc, 0, 0, 0);
+        }
+      }
+      asm volatile("" ::: "memory");
+    }
+  }
+  if (wave < NF)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lg[4 * g + i][nf * 16 + r] = acc[i];
+  __syncthreads();
+  if (logits != nullptr) {
+    for (int p = tid; p < kRowsPerWave * E; p += kWaves * 64) {
+      const int t = p / E;
+      if (t0 + t < n_tokens) logits[(t0 + t) * E + (p - t * E)] = lg[t][p - t * E];
+    }
+  }
+  if constexpr (KC == 8 && E == 32) {
+    // one wave selects for the 16 tokens in registers (four lanes each)
+    if (wave == 0)
+      select_topk_wave<DT, E, KC>(&lg[0][0], E + 1, t0, n_tokens, sel_val, sel_idx, topk_idx, gate, keys, E + 2,
+                                  RouterHist{}, nullptr, nullptr);
+  } else {
+    // four tokens per wave (64 experts, top-8 by one wave: 4 us longer)
+    constexpr int TW = kRowsPerWave / kWaves;
+    const int f = wave * TW;
+    select_topk_from_lds<DT, E, KC>(&lg[f][0], E + 1, TW, E, k, t0 + f, n_tokens, sel_val + f * 64, sel_idx + f * 64,
+                                   rsum + f, topk_idx, gate, keys + f * (E + 2), E + 2);
+  }
+}
+
 template <int NSEG>
 __global__ __launch_bounds__(kWaves * 64) void router32_kernel(const uint16_t* __restrict__ x,
                                                                const uint16_t* __restrict__ w, int64_t n_tokens,
@@ -444,6 +562,32 @@ hipError_t launch_router(const void* x, const void* w, int64_t n, int hidden, in
   const T* xp = static_cast<const T*>(x);
   const T* wp = static_cast<const T*>(w);
   T* gp = static_cast<T*>(gate);
+  // fp32 and 64 experts, while 16 tokens per workgroup are at most one round
+  // of the CUs (us, 1000 tokens: fp32 hidden 1024, 32 experts 20.7 -> 10.2;
+  // bf16 hidden 2048, 64 experts, top-8 24.9 -> 12.9, top-6 of hidden 768
+  // 22.1 -> 10.2).  Past that the 64-token workgroups read W_r less often
+  // (16384 tokens, 64 experts in bf16: 30 against 67), and bf16 with 16 or 32
+  // experts is even (7.8 against 8.1).
+  if (hist.bc == nullptr && (DT == MEP_DTYPE_F32 || E == 64) &&
+      n <= static_cast<int64_t>(kRowsPerWave) * device_cu_count()) {
+    const dim3 grid16(static_cast<unsigned>((n + kRowsPerWave - 1) / kRowsPerWave));
+#define MEP_ROUTER16_CASE(NF_)                                                                                \
+  if (k == 8) router16_kernel<DT, NF_, 8><<<grid16, kWaves * 64, 0, stream>>>(xp, wp, n, hidden, k, idx, gp, logits); \
+  else router16_kernel<DT, NF_, 0><<<grid16, kWaves * 64, 0, stream>>>(xp, wp, n, hidden, k, idx, gp, logits);
+    if (E == 64) {
+      MEP_ROUTER16_CASE(4)
+    } else if constexpr (DT == MEP_DTYPE_F32) {
+      if (E == 32) {
+        MEP_ROUTER16_CASE(2)
+      } else if (E == 16) {
+        MEP_ROUTER16_CASE(1)
+      } else {
+        return hipErrorInvalidValue;
+      }
+    }
+#undef MEP_ROUTER16_CASE
+    return hipGetLastError();
+  }
   if constexpr (DT == MEP_DTYPE_BF16) {
     // GraniteMoE's shape: the specialised kernel
     if (E == 32 && k == 8 && (hidden == 1024 || hidden == 2048 || hidden == 4096)) {
