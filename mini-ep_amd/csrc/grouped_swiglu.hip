@@ -2345,7 +2345,7 @@ __device__ void decode_route(const DecodeParams& p, unsigned char* lds) {
   if (tid < E) s_mask[tid] = 0u;
   const int64_t t0 = static_cast<int64_t>(wave) * kRowsPerWave;
   f32x4 acc[2];
-  router32_logits<NSEG>(p.x, p.w_router, p.n_tokens, t0, ws, acc);
+  router32_logits<NSEG>(p.x, p.w_router, p.n_tokens, t0, ws, reinterpret_cast<unsigned char*>(lg[wave]), acc);
   RouterHist hist{};
   hist.valid = p.valid;
   int sel[2];                                     // experts of this lane's two slots, -1: not dispatched

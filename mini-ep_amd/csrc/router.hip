@@ -258,13 +258,13 @@ __global__ __launch_bounds__(kWaves * 64) void router32_kernel(const uint16_t* _
                                                                float* __restrict__ logits, RouterHist hist) {
   constexpr int E = 32, KC = 8;
   __shared__ __attribute__((aligned(16))) unsigned char ws[E * kRowStride32];
-  __shared__ float lg[kWaves][kRowsPerWave][E + 1];
+  __shared__ __attribute__((aligned(16))) float lg[kWaves][kRowsPerWave][E + 1];   // 2112 B a wave
   __shared__ int s_cnt[E];
   const int tid = threadIdx.x, wave = tid >> 6;
   if (tid < E) s_cnt[tid] = 0;                    // published by the first barrier of router32_logits
   const int64_t t0 = (static_cast<int64_t>(blockIdx.x) * kWaves + wave) * kRowsPerWave;
   f32x4 acc[2];
-  router32_logits<NSEG>(x, w, n_tokens, t0, ws, acc);
+  router32_logits<NSEG>(x, w, n_tokens, t0, ws, reinterpret_cast<unsigned char*>(lg[wave]), acc);
   // the E = 32, top-8 selection runs in registers: no key / selection scratch
   router_tail<MEP_DTYPE_BF16, E, KC>(acc, lg[wave], nullptr, nullptr, nullptr, nullptr, s_cnt, t0, n_tokens, KC,
                                       topk_idx, gate, logits, hist);
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(kWaves * 64) void route_dispatch32_kernel(const uin
   constexpr int E = 32, KC = 8;
   constexpr int kParts = kWaves * 64 / E;         // 8 threads per expert sum the histogram rows
   __shared__ __attribute__((aligned(16))) unsigned char ws[E * kRowStride32];
-  __shared__ float lg[kWaves][kRowsPerWave][E + 1];
+  __shared__ __attribute__((aligned(16))) float lg[kWaves][kRowsPerWave][E + 1];   // 2112 B a wave
   __shared__ int s_wcnt[kWaves][E];               // entries of expert e in wave w of this block
   __shared__ int s_part[kParts][2][E];            // per part: entries in earlier blocks / in all blocks
   __shared__ int s_base[E];                       // first row of expert e's entries of this block
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(kWaves * 64) void route_dispatch32_kernel(const uin
   const uint64_t tag = static_cast<uint64_t>(0x80000000u | epoch) << 32;
   asm volatile("" ::: "memory");
   f32x4 acc[2];
-  router32_logits<NSEG>(x, w, n_tokens, t0, ws, acc);
+  router32_logits<NSEG>(x, w, n_tokens, t0, ws, reinterpret_cast<unsigned char*>(lg[wave]), acc);
   RouterHist hist{};
   hist.valid = o.valid;
   int sel[2];                                     // experts of this lane's two slots, -1: not dispatched

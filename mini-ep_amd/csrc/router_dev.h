@@ -369,17 +369,32 @@ constexpr int kSegBytes = 64 * 1024;
 // and multiply interleaved one by one, the LDS latency is paid 64 times).
 // One wave's 16 x 32 logit tile of the GraniteMoE router shape (bf16, 32
 // experts, hidden 1024 * NSEG); `ws` is the workgroup's LDS copy of one W_r
-// segment.  Called by every thread of the workgroup (it contains barriers).
+// segment, `xs` 2 KiB of the wave's own (which may be its logit rows).  x is
+// read in whole lines, 8 lanes per row, and put into the MFMA layout through
+// `xs`, chunk c of row r at c ^ (r & 7): read in that layout, 16 rows under 16
+// neighbouring lanes, each KiB took 64 L1 lookups instead of 16 (router +
+// dispatch of 100 tokens 11.6 -> 10.7 us, of 4096 13.0 -> 12.4; of 16384 16.0 ->
+// 16.4, LDS then bounds the phase).  Called by every thread of the workgroup (it contains
+// barriers).
 template <int NSEG>
 __device__ __forceinline__ void router32_logits(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                int64_t n_tokens, int64_t t0, unsigned char* ws, f32x4 (&acc)[2]) {
+                                                int64_t n_tokens, int64_t t0, unsigned char* ws, unsigned char* xs,
+                                                f32x4 (&acc)[2]) {
   constexpr int NF = 2, H = 1024 * NSEG;
   constexpr int kRowStride = 1024 * 2 + 16;        // bytes of one W_r row segment in LDS (16 B pad: conflict-free)
   const int tid = threadIdx.x, lane = lane_id();
   const int r = lane & 15, g = lane >> 4;
-  int64_t tok = t0 + r;
-  if (tok >= n_tokens) tok = n_tokens - 1;        // in-bounds read, result discarded
-  const uint16_t* xrow = x + tok * H + g * 8;
+  // copy i of a line of the 16 rows: row 8 i + lane / 8, chunk lane % 8
+  const uint16_t* xrow[2];
+  unsigned char* xdst[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    const int64_t tok = t0 + row < n_tokens ? t0 + row : n_tokens - 1;    // in-bounds read, result discarded
+    xrow[i] = x + tok * H + (lane & 7) * 8;
+    xdst[i] = xs + row * 128 + (((lane & 7) ^ (row & 7)) << 4);
+  }
+  const unsigned char* const xsrc = xs + r * 128;
   // W_r chunk i of this thread: row (tid >> 7) + 2 i, 16 bytes at column (tid & 127) * 8
   const uint16_t* wrow = w + static_cast<int64_t>(tid >> 7) * H + (tid & 127) * 8;
   const int wlds = (tid >> 7) * kRowStride + (tid & 127) * 16;
@@ -391,17 +406,32 @@ __device__ __forceinline__ void router32_logits(const uint16_t* __restrict__ x, 
 #pragma unroll
     for (int i = 0; i < 16; ++i) wt[i] = *reinterpret_cast<const u32x4*>(wrow + 2 * i * H + seg * 1024);
     asm volatile("" ::: "memory");               // the weight loads go out first
-    u32x4 xa[4][8];
+    u32x4 xa[4][4][2];                            // blocks of 4 lines, two copies each
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) xa[b][j] = *reinterpret_cast<const u32x4*>(xrow + seg * 1024 + b * 256 + j * 32);
+      for (int l = 0; l < 4; ++l)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          xa[b][l][i] = *reinterpret_cast<const u32x4*>(xrow[i] + seg * 1024 + b * 256 + l * 64);
     if (seg > 0) __syncthreads();                 // the previous segment's fragment reads are done
 #pragma unroll
     for (int i = 0; i < 16; ++i) *reinterpret_cast<u32x4*>(ws + wlds + 2 * i * kRowStride) = wt[i];
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
+      // the block's row fragments through the wave's 2 KiB (a wave's LDS
+      // accesses complete in order, so each line's writes follow the reads of
+      // the line before)
+      u32x4 xb[8];
+#pragma unroll
+      for (int l = 0; l < 4; ++l) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(xdst[i]) = xa[b][l][i];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          xb[2 * l + h] = *reinterpret_cast<const u32x4*>(xsrc + (((4 * h + g) ^ (r & 7)) << 4));
+      }
       u32x4 wb[8][NF];
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -413,7 +443,7 @@ __device__ __forceinline__ void router32_logits(const uint16_t* __restrict__ x, 
       for (int j = 0; j < 8; ++j)
 #pragma unroll
         for (int nf = 0; nf < NF; ++nf)
-          acc[nf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[b][j]),
+          acc[nf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xb[j]),
                                                             __builtin_bit_cast(bf16x8, wb[j][nf]), acc[nf], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
