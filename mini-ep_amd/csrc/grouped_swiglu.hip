@@ -1930,8 +1930,7 @@ template <int DT, int MFC, bool GEMM1>
 __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int cb, int n_cb, int row_lo, int row_hi,
                                           int n_cb_other, int* sched, unsigned char* s_ring, int* s_gave) {
   typedef typename Elem<DT>::T T;
-  constexpr int EB = Elem<DT>::kBytes;
-  constexpr int AHEAD = mid::AHEAD;
+  constexpr int EB = Elem<DT>::kBytes, AHEAD = mid::AHEAD;
   constexpr int MF = MFC / 2, NF = 4;                         // row and weight fragments per wave
   constexpr int AP = MFC / 2, WP = mid::WF / 2;               // copy passes of 32 rows
   constexpr int STEP = (MFC + mid::WF) * 1024, SLOT = 2 * STEP;
@@ -2041,12 +2040,14 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
   const unsigned char* const frag0 = s_ring + (16 * lg + (lr ^ lg)) * 16;
   const unsigned char* const frag1 = s_ring + STEP + (16 * lg + (lr ^ lg ^ 12)) * 16;
   u32x4 a[MF], w[NF];
-  auto read_a = [&](const unsigned char* at, int i) { a[i] = *reinterpret_cast<const u32x4*>(at + (wm * MF + i) * 1024); };
+  auto read_a = [&](const unsigned char* at, int i) {
+    a[i] = *reinterpret_cast<const u32x4*>(at + (wm * MF + i) * 1024);
+  };
   auto read_w = [&](const unsigned char* at, int j) {
     w[j] = *reinterpret_cast<const u32x4*>(at + (MFC + wn * NF + j) * 1024);
   };
-  constexpr int ROUND = 2;                                    // blocks per round: the ring's slots are immediates
-  static_assert(AHEAD == ROUND, "register sets and ring slots rotate together");
+  constexpr int ROUND = AHEAD;                                // blocks per round: sets and slots are immediates
+  static_assert(ROUND == 2, "register sets and ring slots alternate together");
   auto round = [&](int r, auto last_c) {
     constexpr bool LAST = decltype(last_c)::value;
 #pragma unroll
@@ -2087,8 +2088,10 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
 #pragma unroll
   for (int j = 0; j < NF; ++j) read_w(frag0, j);
   const int rounds = NB / ROUND;                              // NB is even and at least 4 (the host checks)
-  round(0, std::integral_constant<bool, false>());
-  for (int r = 1; r < rounds - 1; ++r) round(r, std::integral_constant<bool, false>());
+  if (rounds > 1) {
+    round(0, std::integral_constant<bool, false>());
+    for (int r = 1; r < rounds - 1; ++r) round(r, std::integral_constant<bool, false>());
+  }
   round(rounds - 1, std::integral_constant<bool, true>());
 
   // ---- epilogue: lane (lr, lg) of a fragment pair holds columns 8 lg .. 8 lg + 7 of row lr
@@ -2877,9 +2880,10 @@ int mid_row_frags(int64_t max_rows, int n_local, int inter) {
   if (!sparse && tiles * 4 > cu * 3 && !(tiles > cu && tiles * 20 <= cu * 27)) return 0;
   // chunks of 128 rows read the weights half as often as chunks of 64, if the
   // experts have that many rows and the chip is still full (128 tokens: even;
-  // 384 tokens: 34 -> 30; 10 experts with 120 rows each: 19 with 64, 25 with 128)
+  // 384 tokens: 34 -> 30, 700: 47 -> 42; 10 experts with 120 rows each: 19 with
+  // 64, 25 with 128)
   const int64_t units = (max_rows / 128 + n_local / 2) * (inter / 64);
-  return max_rows >= static_cast<int64_t>(n_local) * 64 && units >= (sparse ? cu : 2 * cu) ? 8 : 4;
+  return max_rows >= static_cast<int64_t>(n_local) * 64 && units * 4 >= cu * (sparse ? 4 : 7) ? 8 : 4;
 }
 
 // fp32, every size: chunks of 64 rows, or of 32 while those of 64 are too few
@@ -3087,8 +3091,8 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
       constexpr int DT = decltype(dt)::value;
       GemmParams g1 = gemm1_params<DT, CfgBf16>(x, n_tokens, top_k, perm, offsets, n_local, w_in, w_slot, hidden, inter,
                                                 workspace);
-      GemmParams g2 = gemm2_params<DT, CfgBf16>(workspace, top_k, perm, offsets, n_local, max_rows, w_out, w_slot, hidden,
-                                                inter, y_entries);
+      GemmParams g2 = gemm2_params<DT, CfgBf16>(workspace, top_k, perm, offsets, n_local, max_rows, w_out, w_slot,
+                                                hidden, inter, y_entries);
       set_sched(g1, tile_queue);
       set_sched(g2, tile_queue);
       g1.c_bytes = static_cast<uint32_t>(max_rows * inter * dtype_bytes(DT));
