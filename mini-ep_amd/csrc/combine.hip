@@ -95,9 +95,12 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const typename Elem<D
   *reinterpret_cast<u32x4*>(out + t * hidden + c * EPC) = pack_row_chunk<DT>(acc);
 }
 
-// k = 8, (token, slot) layout: combine8_chunk (combine_dev.h), the same
-// slot-order sum as combine_kernel, with y read by non-temporal loads.
-template <int DT>
+// k = 8: combine8_chunk and, INDEXED, combine8_rows_chunk (combine_dev.h), the
+// same slot-order sum as combine_kernel with a token's cells read together (one
+// after the other, as there, a cell's row and the cell itself are a chain of
+// eight times two round trips: 1024 tokens of 1024 in bf16, indexed, 13.1 ->
+// MEASURE us), y by non-temporal loads.
+template <int DT, bool INDEXED>
 __global__ __launch_bounds__(kCombine8Threads) void combine8_kernel(const typename Elem<DT>::T* __restrict__ y,
                                                             const typename Elem<DT>::T* __restrict__ gate,
                                                             const int32_t* __restrict__ row_of_entry,
@@ -111,9 +114,9 @@ __global__ __launch_bounds__(kCombine8Threads) void combine8_kernel(const typena
   if (!chunk_of_thread<kCombine8Threads>(n_tokens, hidden / EPC, t, c)) return;
   // y is read exactly once: non-temporal loads keep these 268 MB (T=16384)
   // from evicting x and the weights from the 256 MB MALL before the next layer
-  combine8_chunk<DT>(y, gate, row_of_entry, valid, t, c, hidden, out, [](const T* p) {
-    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-  });
+  auto load = [](const T* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); };
+  if constexpr (INDEXED) combine8_rows_chunk<DT>(y, gate, row_of_entry, valid, t, c, hidden, out, load);
+  else combine8_chunk<DT>(y, gate, row_of_entry, valid, t, c, hidden, out, load);
 }
 
 // out[i, :] = x[perm[i] / top_k, :] (and ids_out[i] = topk_flat[perm[i]]):
@@ -159,14 +162,14 @@ int combine_entry(const char* fn, const void* y, const void* topk_gate, const in
               MEP_ERR_INVALID_ARG, "%s: y / out must be 16-byte aligned", fn);
   const dim3 grid(static_cast<unsigned>((n_tokens * cpr + kThreads - 1) / kThreads));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!INDEXED && top_k == 8) {
+  if (top_k == 8) {
     const dim3 grid8(static_cast<unsigned>((n_tokens * cpr + kCombine8Threads - 1) / kCombine8Threads));
     if (dtype == MEP_DTYPE_BF16)
-      combine8_kernel<MEP_DTYPE_BF16><<<grid8, kCombine8Threads, 0, s>>>(
+      combine8_kernel<MEP_DTYPE_BF16, INDEXED><<<grid8, kCombine8Threads, 0, s>>>(
           static_cast<const uint16_t*>(y), static_cast<const uint16_t*>(topk_gate), row_of_entry, valid_mask,
           n_tokens, hidden, static_cast<uint16_t*>(out));
     else
-      combine8_kernel<MEP_DTYPE_F32><<<grid8, kCombine8Threads, 0, s>>>(
+      combine8_kernel<MEP_DTYPE_F32, INDEXED><<<grid8, kCombine8Threads, 0, s>>>(
           static_cast<const float*>(y), static_cast<const float*>(topk_gate), row_of_entry, valid_mask,
           n_tokens, hidden, static_cast<float*>(out));
   } else if (dtype == MEP_DTYPE_BF16)

@@ -34,6 +34,44 @@ __device__ __forceinline__ u32x4 pack_row_chunk(const float* acc) {
   return o;
 }
 
+// The sum of one chunk of the token's k = 8 cells, given the chunks, the row of
+// each cell (< 0: absent) and the gates.
+template <int DT>
+__device__ __forceinline__ void combine8_sum(const u32x4 (&v)[8], const int32_t (&row)[8], const float (&g)[8],
+                                             bool tok_ok, bool poison, typename Elem<DT>::T* __restrict__ dst) {
+  constexpr int EPC = 16 / Elem<DT>::kBytes;
+  float acc[EPC];
+#pragma unroll
+  for (int q = 0; q < EPC; ++q) acc[q] = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const bool here = tok_ok && row[s] >= 0;
+    poison |= row[s] == kPoisonRow;
+    float yv[EPC];
+    if constexpr (DT == MEP_DTYPE_BF16) {
+      const uint32_t w[4] = {v[s].x, v[s].y, v[s].z, v[s].w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        yv[2 * q] = bf16_to_f32(static_cast<uint16_t>(w[q] & 0xffffu));
+        yv[2 * q + 1] = bf16_to_f32(static_cast<uint16_t>(w[q] >> 16));
+      }
+    } else {
+      yv[0] = __uint_as_float(v[s].x);
+      yv[1] = __uint_as_float(v[s].y);
+      yv[2] = __uint_as_float(v[s].z);
+      yv[3] = __uint_as_float(v[s].w);
+    }
+#pragma unroll
+    for (int q = 0; q < EPC; ++q) {
+      const float sum = acc[q] + g[s] * yv[q];
+      acc[q] = here ? sum : acc[q];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < EPC; ++q) acc[q] = poison ? __builtin_nanf("") : acc[q];
+  *reinterpret_cast<u32x4*>(dst) = pack_row_chunk<DT>(acc);
+}
+
 // DEV: the token's row_of_entry entries and gates are read with device-scope
 // loads (written earlier in the same launch, possibly on another XCD), and so
 // is `poison` if given: nonzero there makes the chunk NaN, as a poisoned
@@ -46,8 +84,7 @@ __device__ __forceinline__ void combine8_chunk(const typename Elem<DT>::T* __res
                                                typename Elem<DT>::T* __restrict__ out, LoadY load_y,
                                                const int32_t* poison_word = nullptr) {
   typedef typename Elem<DT>::T T;
-  constexpr int K = 8;
-  constexpr int EPC = 16 / Elem<DT>::kBytes;
+  constexpr int K = 8, EPC = 16 / Elem<DT>::kBytes;
   const T* ybase = y + (t * K) * hidden + c * EPC;
   u32x4 v[K];
 #pragma unroll
@@ -80,37 +117,36 @@ __device__ __forceinline__ void combine8_chunk(const typename Elem<DT>::T* __res
     }
   }
   const bool tok_ok = valid == nullptr || valid[t] != 0;
-  bool poison = pw != 0;
-  float acc[EPC];
-#pragma unroll
-  for (int q = 0; q < EPC; ++q) acc[q] = 0.0f;
+  combine8_sum<DT>(v, row, g, tok_ok, pw != 0, out + t * hidden + c * EPC);
+}
+
+// The same sum with cell (t, s) in row row_of_entry[t*8 + s] of y (the
+// expert-parallel return path).  The rows are read first, then the 8 cells
+// together; an absent cell is not read.
+template <int DT, class LoadY>
+__device__ __forceinline__ void combine8_rows_chunk(const typename Elem<DT>::T* __restrict__ y,
+                                                    const typename Elem<DT>::T* __restrict__ gate,
+                                                    const int32_t* __restrict__ row_of_entry,
+                                                    const uint8_t* __restrict__ valid, int64_t t, int c, int hidden,
+                                                    typename Elem<DT>::T* __restrict__ out, LoadY load_y) {
+  constexpr int K = 8, EPC = 16 / Elem<DT>::kBytes;
+  int32_t row[K];
+  float g[K];
+  const bool tok_ok = valid == nullptr || valid[t] != 0;
 #pragma unroll
   for (int s = 0; s < K; ++s) {
-    const bool here = tok_ok && row[s] >= 0;
-    poison |= row[s] == kPoisonRow;
-    float yv[EPC];
-    if constexpr (DT == MEP_DTYPE_BF16) {
-      const uint32_t w[4] = {v[s].x, v[s].y, v[s].z, v[s].w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        yv[2 * q] = bf16_to_f32(static_cast<uint16_t>(w[q] & 0xffffu));
-        yv[2 * q + 1] = bf16_to_f32(static_cast<uint16_t>(w[q] >> 16));
-      }
-    } else {
-      yv[0] = __uint_as_float(v[s].x);
-      yv[1] = __uint_as_float(v[s].y);
-      yv[2] = __uint_as_float(v[s].z);
-      yv[3] = __uint_as_float(v[s].w);
-    }
-#pragma unroll
-    for (int q = 0; q < EPC; ++q) {
-      const float sum = acc[q] + g[s] * yv[q];
-      acc[q] = here ? sum : acc[q];
-    }
+    row[s] = row_of_entry[t * K + s];
+    g[s] = Elem<DT>::to_f32(gate[t * K + s]);
   }
 #pragma unroll
-  for (int q = 0; q < EPC; ++q) acc[q] = poison ? __builtin_nanf("") : acc[q];
-  *reinterpret_cast<u32x4*>(out + t * hidden + c * EPC) = pack_row_chunk<DT>(acc);
+  for (int s = 0; s < K; ++s) row[s] = tok_ok ? row[s] : -1;   // a masked token is 0, poisoned or not
+  u32x4 v[K];
+#pragma unroll
+  for (int s = 0; s < K; ++s) {
+    v[s] = u32x4{0u, 0u, 0u, 0u};
+    if (row[s] >= 0) v[s] = load_y(y + static_cast<int64_t>(row[s]) * hidden + c * EPC);
+  }
+  combine8_sum<DT>(v, row, g, tok_ok, false, out + t * hidden + c * EPC);
 }
 
 }  // namespace mep

@@ -64,3 +64,36 @@ def test_combine_rows_indexed(dtype, H):
     cells[present.numpy()] = y.float().numpy()[rows.numpy()[present.numpy()]]
     ref = O.combine(cells, gate.float().numpy(), present.numpy(), n, k)
     assert rel_err(out, ref) <= (TOL_BF16 if dtype == torch.bfloat16 else TOL_F32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,H", [(1, 8), (7, 520), (129, 1024)])
+def test_combine_rows_k8_masks_and_poison(dtype, n, H):
+    """k = 8 through indices: masked tokens are 0 whatever their cells hold, a
+    poisoned cell (-2) makes its token NaN, a token without cells is 0, and
+    rows that nothing names (NaN here) do not reach an output.  Bar as above."""
+    banner(f"combine_rows k=8 {dtype} n={n} H={H}")
+    k = 8
+    g = torch.Generator().manual_seed(n)
+    y = torch.randn(n * k + 3, H, generator=g).to(dtype)
+    y[n * k:] = float("nan")
+    gate = torch.softmax(torch.randn(n, k, generator=g), -1).to(dtype)
+    rows = torch.randperm(n * k, generator=g).to(torch.int32).reshape(n, k)
+    rows[torch.rand(n, k, generator=g) < 0.3] = -1
+    valid = torch.rand(n, generator=g) < 0.7
+    rows[n // 2] = -1
+    poisoned = torch.zeros(n, dtype=torch.bool)
+    if n > 4:
+        poisoned[1] = poisoned[4] = True
+        valid[1], valid[4] = True, False
+        rows[1, 3] = rows[4, 7] = -2
+    out = ops.combine_rows(y.to(DEV), gate.to(DEV), rows.reshape(-1).to(DEV), valid.to(DEV)).float().cpu()
+    nan = poisoned & valid
+    assert bool(torch.isnan(out[nan]).all()) and bool(torch.isfinite(out[~nan]).all())
+    present = (rows >= 0) & valid[:, None]
+    cells = torch.where(present[..., None], y[rows.clamp(min=0).long()].float(), torch.zeros(()))
+    ref = O.combine(cells.reshape(n * k, H).numpy(), gate.float().numpy(), present.reshape(-1).numpy(), n, k)
+    assert not out[~valid].any() and not out[n // 2].nan_to_num().any()
+    keep = ~nan.numpy()
+    tol = TOL_BF16 if dtype == torch.bfloat16 else TOL_F32
+    assert np.abs(out.numpy()[keep] - ref[keep]).max() <= tol * max(np.abs(ref[keep]).max(), 1e-30)
