@@ -170,6 +170,19 @@ inline int dtype_bytes(int dtype) {
   return dtype == MEP_DTYPE_F32 ? 4 : (dtype == MEP_DTYPE_BF16 ? 2 : 0);
 }
 
+// Workgroup barrier that orders LDS only: this wave's LDS reads and writes
+// complete (lgkmcnt(0)) before it arrives.  __syncthreads() also waits for
+// every outstanding global access (vmcnt(0)): for stores nobody waits for, and
+// for loads that a pipeline keeps in flight.  The empty asm statements keep
+// the compiler from moving memory accesses across.
+constexpr int kLgkmcnt0 = 0xC07F;   // s_waitcnt lgkmcnt(0) alone (vmcnt 63, expcnt 7)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(kLgkmcnt0);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 }  // namespace mep
 
 // Report a failed precondition from a C-ABI entry point.

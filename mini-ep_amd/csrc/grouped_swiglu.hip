@@ -141,19 +141,6 @@ constexpr int kFlagInputBit = 4;
 
 constexpr int pow2_floor(int v) { int r = 1; while (r * 2 <= v) r *= 2; return r; }
 
-// Workgroup barrier that orders LDS only: this wave's LDS reads and writes
-// complete (lgkmcnt(0)) before it arrives.  __syncthreads() also waits for
-// every outstanding global access (vmcnt(0)); in the epilogue that would wait
-// for the previous pass's stores and the next tile's first DMA stage.  The
-// empty asm statements keep the compiler from moving memory accesses across.
-constexpr int kLgkmcnt0 = 0xC07F;   // s_waitcnt lgkmcnt(0) alone (vmcnt 63, expcnt 7)
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(kLgkmcnt0);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 template <int DT, class Cfg, bool GEMM1>
 __global__ __launch_bounds__(Cfg::NT) void grouped_gemm_kernel(GemmParams p) {
   typedef typename Elem<DT>::T T;

@@ -156,6 +156,7 @@ struct AttnParams {
   int start;                // positions in the cache before this call; token i is position start + i
   int64_t max_len;
   float scale;
+  int n_cu;                 // compute units of the device
 };
 
 // The rotated value of element c of a head whose projections start at `head`:
@@ -165,6 +166,18 @@ __device__ __forceinline__ float rope(const typename Elem<DT>::T* head, int c, c
   const float x = Elem<DT>::to_f32(head[c]);
   const float y = Elem<DT>::to_f32(head[c < kHead / 2 ? c + kHead / 2 : c - kHead / 2]);
   return x * cos[c] + (c < kHead / 2 ? -y : y) * sin[c];
+}
+
+// Four elements of a head from an address that is a multiple of them.
+template <int DT>
+__device__ __forceinline__ f32x4 load4(const typename Elem<DT>::T* src) {
+  if constexpr (DT == MEP_DTYPE_BF16) {
+    const uint2 w = *reinterpret_cast<const uint2*>(src);
+    return f32x4{bf16_to_f32(static_cast<uint16_t>(w.x & 0xffffu)), bf16_to_f32(static_cast<uint16_t>(w.x >> 16)),
+                 bf16_to_f32(static_cast<uint16_t>(w.y & 0xffffu)), bf16_to_f32(static_cast<uint16_t>(w.y >> 16))};
+  } else {
+    return *reinterpret_cast<const f32x4*>(src);
+  }
 }
 
 // Keys (rotated) and values of the call's tokens into the cache: one thread
@@ -184,14 +197,13 @@ __global__ __launch_bounds__(256) void kv_write_kernel(AttnParams p) {
   const int64_t src = th * kHead, pos = p.start + i;
   const T* const k = static_cast<const T*>(p.k) + src;
   const T* const v = static_cast<const T*>(p.v) + src;
-  const float* const cs = p.cos + pos * kHead;
-  const float* const sn = p.sin + pos * kHead;
-  f32x4 kr, vr;
+  const f32x4 cs = *reinterpret_cast<const f32x4*>(p.cos + pos * kHead + c);
+  const f32x4 sn = *reinterpret_cast<const f32x4*>(p.sin + pos * kHead + c);
+  const f32x4 x = load4<DT>(k + c), y = load4<DT>(k + (c < kHead / 2 ? c + kHead / 2 : c - kHead / 2));
+  const f32x4 vr = load4<DT>(v + c);
+  f32x4 kr;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    kr[j] = rope<DT>(k, c + j, cs, sn);
-    vr[j] = Elem<DT>::to_f32(v[c + j]);
-  }
+  for (int j = 0; j < 4; ++j) kr[j] = x[j] * cs[j] + (c < kHead / 2 ? -y[j] : y[j]) * sn[j];
   const int64_t dst = ((static_cast<int64_t>(b) * p.hk + head) * p.max_len + pos) * kHead + c;
   *reinterpret_cast<f32x4*>(p.kc + dst) = kr;
   *reinterpret_cast<f32x4*>(p.vc + dst) = vr;
@@ -207,9 +219,11 @@ __global__ __launch_bounds__(256) void kv_write_kernel(AttnParams p) {
 // their lane.  LDS rows are padded to 68 floats, which spreads both the
 // 16-byte key reads and the 4-byte value reads over all banks.  Bound by the
 // fp32 MFMAs (32 per wave, 16 keys and 16 queries) and the waits around the
-// two barriers of a block.  8 sequences of 256 tokens, 16 heads: 28.6 us, and
-// 4.6 us for the cache write, against 49 us for torch's fp32 attention after
-// a dozen launches of rotation, cache copy and head repetition.
+// two barriers of a block.  8 sequences of 256 tokens, 16 heads: 20.3 us (512
+// tokens: 56), and 4.6 us for the cache write, against 49 us for torch's fp32
+// attention after a dozen launches of rotation, cache copy and head
+// repetition.  (With the query tile as the fastest grid index the longest
+// tiles all fall on two XCDs: 27 and 90 us.)
 constexpr int kFlashQ = 64, kFlashK = 64, kFlashRow = kHead + 4;
 
 template <int DT>
@@ -219,9 +233,22 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) float s_v[kFlashK * kFlashRow];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int q0 = (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x)) * kFlashQ;   // longest rows first
-  const int head = static_cast<int>(blockIdx.y) % p.hq, b = static_cast<int>(blockIdx.y) / p.hq;
-  const int kv = head / (p.hq / p.hk);
+  // workgroup -> (query tile, sequence, head of the group, kv head), kv head
+  // fastest: the heads and tiles of a kv head share an XCD's L2, and the tiles
+  // with the most keys come first on every XCD
+  int id = static_cast<int>(blockIdx.x);
+  const int kv = id % p.hk;
+  id /= p.hk;
+  const int G = p.hq / p.hk;
+  const int head = kv * G + id % G;
+  id /= G;
+  // (tile, sequence) pairs of one round of the CUs; the second round, which
+  // joins the first on the same CUs, is taken backwards: a CU gets a long and
+  // a short tile
+  const int per = p.n_cu / p.hq, pairs = (p.t + kFlashQ - 1) / kFlashQ * p.batch;
+  if (id >= per && id < 2 * per) id = per + min(2 * per, pairs) - 1 - id;
+  const int b = id % p.batch;
+  const int q0 = ((p.t + kFlashQ - 1) / kFlashQ - 1 - id / p.batch) * kFlashQ;
   const int S = p.start + p.t;
   const float* const kc = p.kc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
   const float* const vc = p.vc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
@@ -236,10 +263,16 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
     const T* const src = static_cast<const T*>(p.q) + (static_cast<int64_t>(b) * p.t + qrow) * p.hq * kHead + head * kHead;
     const float* const cs = p.cos + static_cast<int64_t>(qpos) * kHead;
     const float* const sn = p.sin + static_cast<int64_t>(qpos) * kHead;
+    f32x4 x[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) x[j] = load4<DT>(src + 16 * j + 4 * g);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) q[j][i] = rope<DT>(src, 16 * j + 4 * g + i, cs, sn);
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 c = *reinterpret_cast<const f32x4*>(cs + 16 * j + 4 * g);
+      const f32x4 s = *reinterpret_cast<const f32x4*>(sn + 16 * j + 4 * g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[j][i] = x[j][i] * c[i] + (j < 2 ? -x[j + 2][i] : x[j - 2][i]) * s[i];
+    }
   }
   const float sc = p.scale * kLog2e;
 
@@ -338,11 +371,22 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
 // LDS (16 lanes per key, 16 bytes each, so a wave reads four whole keys per
 // instruction), the chunk's maximum and sum, then the values with the same
 // lane layout.  The sums of the 64 key groups meet in LDS in a fixed order.
-// Bound by one CU's loads and the chunk's barriers: 8 sequences of 513
-// positions, 8 kv heads (16.8 MB of cache): 14.1 us, against 46 us for torch's
-// fp32 attention alone.
+// Two batches of loads are kept in flight, from the first keys (before the
+// rotation) through the softmax's barrier to the last values.  Bound by one
+// CU's loads: 8 sequences of 513 positions, 8 kv heads (16.8 MB of cache):
+// 11.0 us (14.1 with one batch at a time and the sums of 16 lanes through
+// LDS), against 46 us for torch's fp32 attention alone.
 constexpr int kDecWaves = 16, kDecKeys = 2048;
-constexpr int kDecUnroll = 4;
+
+// The sum over a row of 16 lanes, in every lane: the tree of xor 1, 2, 4, 8 (a
+// mirrored lane holds what the xor partner holds once the steps before agree).
+__device__ __forceinline__ float sum16(float v) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));    // quad_perm 1 0 3 2
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));    // quad_perm 2 3 0 1
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true));   // row_half_mirror
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xF, 0xF, true));   // row_mirror
+  return v;
+}
 
 template <int DT, int G>
 __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnParams p) {
@@ -358,6 +402,21 @@ __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnPa
   const int pos = p.start, S = pos + 1;
   float* const kc = p.kc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
   float* const vc = p.vc + (static_cast<int64_t>(b) * p.hk + kv) * p.max_len * kHead;
+  // a batch: kDecUnroll cached positions per lane group, 16 bytes of each per
+  // lane (past the end, and in place of the new token: the last one again)
+  constexpr int kDecUnroll = G == 4 ? 2 : 4;               // G = 4 has no registers for more
+  constexpr int kStep = kDecWaves * 4, kBatch = kStep * kDecUnroll;
+  f32x4 ra[kDecUnroll], rb[kDecUnroll];
+  auto fetch = [&](f32x4 (&r)[kDecUnroll], const float* cache, int c0, int s0) {   // positions c0 + s0 ..
+    const char* const base = reinterpret_cast<const char*>(cache + static_cast<int64_t>(c0) * kHead);
+    const int last = max(pos - 1 - c0, 0);
+#pragma unroll
+    for (int u = 0; u < kDecUnroll; ++u) {
+      const int s = min(s0 + u * kStep + wave * 4 + g, last);
+      r[u] = *reinterpret_cast<const f32x4*>(base + static_cast<uint32_t>(s * (kHead * 4) + 16 * c));
+    }
+  };
+  fetch(ra, kc, 0, 0);
   {
     const float* const cs = p.cos + static_cast<int64_t>(pos) * kHead;
     const float* const sn = p.sin + static_cast<int64_t>(pos) * kHead;
@@ -376,84 +435,91 @@ __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnPa
       vc[static_cast<int64_t>(pos) * kHead + e] = v;
     }
   }
-  __syncthreads();
-  f32x4 q[G];
+  lds_barrier();
+  f32x4 q[G], fresh[2];                                    // the queries; the new token's key and value
 #pragma unroll
   for (int h = 0; h < G; ++h) q[h] = *reinterpret_cast<const f32x4*>(&s_q[h][4 * c]);
-  // 16 bytes of position s: from the cache, or the new token's from LDS
-  auto row = [&](const float* cache, int which, int s) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(cache + static_cast<int64_t>(min(s, max(pos - 1, 0))) * kHead + 4 * c);
-    return s == pos ? *reinterpret_cast<const f32x4*>(&s_new[which][4 * c]) : v;
-  };
-  constexpr int kStep = kDecWaves * 4;                     // positions per workgroup step
-  float m[G], l[G];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) fresh[i] = *reinterpret_cast<const f32x4*>(&s_new[i][4 * c]);
+  float m[G], l[G], mx[G];
   f32x4 o[G];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
-    m[h] = -__builtin_inff();
+    m[h] = mx[h] = -__builtin_inff();
     l[h] = 0.0f;
     o[h] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   for (int c0 = 0; c0 < S; c0 += kDecKeys) {
     const int n = min(kDecKeys, S - c0);
-    float mx[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) mx[h] = m[h];
-    for (int s0 = wave * 4 + g; s0 < n; s0 += kStep * kDecUnroll) {
-      f32x4 kr[kDecUnroll];
-#pragma unroll
-      for (int u = 0; u < kDecUnroll; ++u) kr[u] = row(kc, 0, c0 + min(s0 + u * kStep, n - 1));
+    const int nb = (n + kBatch - 1) / kBatch, pairs = (nb + 1) / 2;
+    if (c0 != 0) fetch(ra, kc, c0, 0);
+    auto scores = [&](const f32x4 (&kr)[kDecUnroll], int bt) {
+      if (bt >= nb) return;
 #pragma unroll
       for (int u = 0; u < kDecUnroll; ++u) {
-        const int s = s0 + u * kStep;
+        const int s = bt * kBatch + u * kStep + wave * 4 + g;
+        const f32x4 k = c0 + s == pos ? fresh[0] : kr[u];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-          float d = kr[u].x * q[h].x + kr[u].y * q[h].y + kr[u].z * q[h].z + kr[u].w * q[h].w;
-#pragma unroll
-          for (int x = 1; x < 16; x <<= 1) d += __shfl_xor(d, x, 64);
+          const float d = sum16(k.x * q[h].x + k.y * q[h].y + k.z * q[h].z + k.w * q[h].w);
           if (s < n) {
             mx[h] = fmaxf(mx[h], d);
             if (c == 0) s_p[h][s] = d;
           }
         }
       }
+    };
+    for (int i = 0; i < pairs; ++i) {
+      fetch(rb, kc, c0, (2 * i + 1) * kBatch);
+      scores(ra, 2 * i);
+      // after the last keys, the first values
+      fetch(ra, i + 1 < pairs ? kc : vc, c0, i + 1 < pairs ? (2 * i + 2) * kBatch : 0);
+      scores(rb, 2 * i + 1);
     }
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 16, 64));
-      mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 32, 64));
-      if (lane == 0) s_red[wave][h] = mx[h];
+      float v = mx[h];
+      v = fmaxf(v, __shfl_xor(v, 16, 64));
+      v = fmaxf(v, __shfl_xor(v, 32, 64));
+      if (lane == 0) s_red[wave][h] = v;
     }
-    __syncthreads();
+    lds_barrier();                                         // the values' loads stay in flight
 #pragma unroll
     for (int h = 0; h < G; ++h) {
       float v = s_red[0][h];
 #pragma unroll
       for (int w = 1; w < kDecWaves; ++w) v = fmaxf(v, s_red[w][h]);
       const float alpha = __builtin_amdgcn_exp2f(m[h] - v);   // 0 in the first chunk
-      m[h] = v;
+      m[h] = mx[h] = v;
       l[h] *= alpha;
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[h][i] *= alpha;
     }
-    for (int s0 = wave * 4 + g; s0 < n; s0 += kStep * kDecUnroll) {
-      f32x4 vr[kDecUnroll];
-#pragma unroll
-      for (int u = 0; u < kDecUnroll; ++u) vr[u] = row(vc, 1, c0 + min(s0 + u * kStep, n - 1));
+    auto values = [&](const f32x4 (&vr)[kDecUnroll], int bt) {
+      if (bt >= nb) return;
 #pragma unroll
       for (int u = 0; u < kDecUnroll; ++u) {
-        const int s = s0 + u * kStep;
+        const int s = bt * kBatch + u * kStep + wave * 4 + g;
         if (s >= n) continue;
+        const f32x4 v = c0 + s == pos ? fresh[1] : vr[u];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
           const float e = __builtin_amdgcn_exp2f(s_p[h][s] - m[h]);
           l[h] += e;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[h][i] += e * vr[u][i];
+          for (int i = 0; i < 4; ++i) o[h][i] += e * v[i];
         }
       }
+    };
+    for (int i = 0; i < pairs; ++i) {
+      fetch(rb, vc, c0, (2 * i + 1) * kBatch);
+      values(ra, 2 * i);
+      if (i + 1 == pairs) break;
+      fetch(ra, vc, c0, (2 * i + 2) * kBatch);
+      values(rb, 2 * i + 1);
     }
-    __syncthreads();                                       // scores and maxima are read before the next chunk's
+    values(rb, 2 * pairs - 1);
+    lds_barrier();                                         // scores and maxima are read before the next chunk's
   }
 #pragma unroll
   for (int h = 0; h < G; ++h) {
@@ -494,8 +560,10 @@ hipError_t launch_attention(const AttnParams& p, hipStream_t stream) {
   kv_write_kernel<DT><<<dim3(static_cast<unsigned>((chunks + 255) / 256)), 256, 0, stream>>>(p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const dim3 grid(static_cast<unsigned>((p.t + kFlashQ - 1) / kFlashQ), static_cast<unsigned>(p.batch * p.hq));
-  attention_kernel<DT><<<grid, 256, 0, stream>>>(p);
+  const dim3 grid(static_cast<unsigned>((p.t + kFlashQ - 1) / kFlashQ) * static_cast<unsigned>(p.batch * p.hq));
+  AttnParams pf = p;
+  pf.n_cu = device_cu_count();
+  attention_kernel<DT><<<grid, 256, 0, stream>>>(pf);
   return hipGetLastError();
 }
 
@@ -759,8 +827,10 @@ extern "C" int mep_attention(const void* q, const void* k, const void* v, const 
   if (rc != MEP_OK) return rc;
   if (batch == 0 || t == 0) return MEP_OK;
   MEP_REQUIRE(q && k && v && cos && sin && k_cache && v_cache && out, MEP_ERR_INVALID_ARG, "%s: null pointer", fn);
-  MEP_REQUIRE(aligned16(k_cache) && aligned16(v_cache) && aligned16(out), MEP_ERR_INVALID_ARG,
-              "%s: the caches and out must be 16-byte aligned", fn);
+  for (const void* ptr : {q, k, v, static_cast<const void*>(cos), static_cast<const void*>(sin),
+                          static_cast<const void*>(k_cache), static_cast<const void*>(v_cache),
+                          static_cast<const void*>(out)})
+    MEP_REQUIRE(aligned16(ptr), MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
   AttnParams p;
   p.q = q; p.k = k; p.v = v; p.cos = cos; p.sin = sin; p.kc = k_cache; p.vc = v_cache; p.out = out;
   p.batch = batch; p.t = t; p.hq = n_heads; p.hk = n_kv_heads;
@@ -798,7 +868,8 @@ extern "C" int mep_attention_block(const void* h, const void* delta, float mult,
               MEP_ERR_INVALID_ARG, "%s: null pointer", fn);
   const size_t need = mep_attention_block_workspace(n, hidden, n_heads, n_kv_heads, head_dim);
   MEP_REQUIRE(workspace_bytes >= need, MEP_ERR_WORKSPACE, "%s: workspace %zu B < required %zu B", fn, workspace_bytes, need);
-  for (const void* ptr : {h, delta, norm1, norm2, wq, wk, wv, wo, static_cast<const void*>(k_cache),
+  for (const void* ptr : {h, delta, norm1, norm2, wq, wk, wv, wo, static_cast<const void*>(cos),
+                          static_cast<const void*>(sin), static_cast<const void*>(k_cache),
                           static_cast<const void*>(v_cache), static_cast<const void*>(workspace),
                           static_cast<const void*>(h_out), static_cast<const void*>(x_out)})
     MEP_REQUIRE(aligned16(ptr), MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
