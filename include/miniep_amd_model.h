@@ -67,6 +67,16 @@ int mep_attention_block(const void* h, const void* delta, float mult, const void
 int mep_norm_head(const void* h, const void* delta, float mult, const void* norm, float eps, const void* w,
                   int64_t n_rows, int32_t hidden, int32_t vocab, float divisor, float* logits, void* stream);
 
+/* ------------------------------------------------------------------------
+ * Projections of a bf16 model (modeling.py:160-185): out[i] (n_rows, cols[i])
+ * = x (n_rows, k) @ w[i]^T for 1 to 3 matrices w[i] (cols[i], k) in one launch
+ * (w, cols and out are host arrays of n_mats), fp32 sums rounded to bf16.
+ * Supported: k a multiple of 128,
+ * at least 256; cols multiples of 128; x and each matrix below 4 GiB.
+ * ---------------------------------------------------------------------- */
+int mep_linear(const void* x, int64_t n_rows, int32_t k, const void* const* w, const int32_t* cols,
+               int32_t n_mats, void* const* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

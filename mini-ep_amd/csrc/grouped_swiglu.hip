@@ -48,6 +48,7 @@
 // Every path walks K in the same order, so they give the same bits.
 #include "combine_dev.h"
 #include "common.h"
+#include "ring_gemm.h"
 #include "router_dev.h"
 
 #include <type_traits>
@@ -561,19 +562,6 @@ struct MoeParams {
   int dbg_row;               // row tile whose GEMM-2 tiles wait for one count more (test hook; -1: none)
 };
 
-// 16x16x32 bf16 MFMA with the accumulator in VGPRs; src0 = weight
-// fragment, src1 = row fragment, so the result is C^T (lane: one row, 4
-// consecutive columns).  mfma_first starts a new accumulation (C operand 0).
-__device__ __forceinline__ void mfma_acc(f32x4& acc, const u32x4& w, const u32x4& a) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(w), "v"(a));
-}
-__device__ __forceinline__ void mfma_first(f32x4& acc, const u32x4& w, const u32x4& a) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=v"(acc) : "v"(w), "v"(a));
-}
-// Orders later reads of `acc` after every earlier volatile asm (an empty asm
-// that claims to rewrite it).  AMDGPU register constraints live in device
-// functions only: in a kernel body the host pass parses them as x86 ones.
-__device__ __forceinline__ void pin_acc(f32x4& acc) { asm volatile("" : "+v"(acc)); }
 // buffer_load_dwordx4 ... lds of one 1 KiB block: lane L's 16 bytes from
 // base + voff + soff land at lds + 16 L; an offset at or past `bytes` reads
 // zeros instead of faulting.  (A plain device function: inside the kernel
@@ -1878,10 +1866,7 @@ hipError_t launch_skinny_both(const GemmParams& p1, const GemmParams& p2, int64_
 // the loop once a weight row met more than some 64 rows: 171 us at 4096
 // tokens of the GraniteMoE layer in bf16, 143 so.)  Plain loads and LDS writes, not LDS DMA: the
 // compiler waits for every load in flight before reading LDS that a DMA may
-// have written.  The ring holds MFMA fragments of 1 KiB, lane (lr, lg)'s 16
-// bytes in slot 16 lg + (lr ^ lg ^ 12 (step & 1)); a copying lane group takes
-// rows 4 apart.  That keeps both the fragment reads and the copies' writes
-// (8 lanes of a row to two steps x four lane groups) on distinct banks.
+// have written.)  The K loop is ring_loop (ring_gemm.h).
 //
 // Chunks are listed by expert and split into 8 contiguous ranges, one per XCD
 // (workgroup b runs on XCD b mod 8): the column blocks of a chunk share its
@@ -1892,35 +1877,17 @@ hipError_t launch_skinny_both(const GemmParams& p1, const GemmParams& p2, int64_
 // give-up flags the launch and stores NaN.  K is walked in the tiled kernel's
 // order with the same MFMA, so every output has the other kernels' bits.
 namespace mid {
-constexpr int NT = 256;
-constexpr int AHEAD = 2;                      // blocks (two K-steps) of loads in flight
-constexpr int WF = 8;                         // weight fragments of a workgroup: 128 weight rows
 inline int64_t chunks(int64_t max_rows, int n_local, int rows) { return (max_rows + rows - 1) / rows + n_local; }
 }  // namespace mid
-
-// One K-step (64 bytes of every row) of a fragment pair: 32 bf16 in one MFMA,
-// or 16 floats in four, MFMA q on elements 4 lg + q of the lane groups (the
-// order of grouped_gemm_kernel).
-template <int DT>
-__device__ __forceinline__ void mid_mfma(f32x4& acc, const u32x4& w, const u32x4& a) {
-  if constexpr (DT == MEP_DTYPE_BF16) {
-    mfma_acc(acc, w, a);
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+v"(acc) : "v"(w[q]), "v"(a[q]));
-  }
-}
 
 // Column block cb of chunk q: rows [row_lo, row_hi) of expert e, at most 16 MFC.
 template <int DT, int MFC, bool GEMM1>
 __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int cb, int n_cb, int row_lo, int row_hi,
                                           int n_cb_other, int* sched, unsigned char* s_ring, int* s_gave) {
   typedef typename Elem<DT>::T T;
-  constexpr int EB = Elem<DT>::kBytes, AHEAD = mid::AHEAD;
+  constexpr int EB = Elem<DT>::kBytes, AHEAD = ring::AHEAD;
   constexpr int MF = MFC / 2, NF = 4;                         // row and weight fragments per wave
-  constexpr int AP = MFC / 2, WP = mid::WF / 2;               // copy passes of 32 rows
-  constexpr int STEP = (MFC + mid::WF) * 1024, SLOT = 2 * STEP;
+  constexpr int AP = MFC / 2, WP = ring::WP;                  // copy passes of 32 rows
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int lr = lane & 15, lg = lane >> 4;
@@ -1933,8 +1900,8 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
   const unsigned char* const A = static_cast<const unsigned char*>(p.A);
 
   // ---- copies: this thread's row of a pass and 16-byte chunk of its line -----------
-  const int c16 = ((tid >> 3) & 3) * 4 + ((tid >> 5) & 3), cf = tid >> 7;   // row 16 cf + c16 of the pass's 32
-  const int cc = tid & 7, clg = cc & 3, cstep = cc >> 2;
+  const ring::Copy cp;
+  const int c16 = cp.row16, cf = cp.half, cc = cp.chunk;
   // weight rows: fragment 4 wn + j.  GEMM-1: j < 2 gate, j >= 2 the up rows of
   // the same act columns cb*64 + 32 wn ..; GEMM-2: output columns cb*128 +
   // 64 wn + 32 (j / 2) ..  Row n of the fragment pair's half j & 1 is column
@@ -1964,14 +1931,6 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
     const unsigned char* const base = A + line(b);
 #pragma unroll
     for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const u32x4*>(base + a_off[i]);
-  };
-  unsigned char* const cdst = s_ring + cstep * STEP + cf * 1024 + (16 * clg + (c16 ^ clg ^ (12 * cstep))) * 16;
-  auto write = [&](int b, const u32x4 (&w)[WP], const u32x4 (&x)[AP]) {
-    unsigned char* const dst = cdst + (b & 1) * SLOT;
-#pragma unroll
-    for (int i = 0; i < AP; ++i) *reinterpret_cast<u32x4*>(dst + 2 * i * 1024) = x[i];
-#pragma unroll
-    for (int i = 0; i < WP; ++i) *reinterpret_cast<u32x4*>(dst + (MFC + 2 * i) * 1024) = w[i];
   };
   // the weights need neither the row map nor GEMM-1
 #pragma unroll
@@ -2008,85 +1967,10 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
 #pragma unroll
   for (int b = 0; b < AHEAD; ++b) load_a(b, ar[b]);
 
-  // ---- K loop --------------------------------------------------------------------------
-  // Block b (steps 2 b, 2 b + 1), with its first step's fragments in registers:
-  //   write block b + 1 (in registers) to the ring, load block b + 1 + AHEAD;
-  //   step 2 b: MFMAs, each fragment refilled with step 2 b + 1's after its last use;
-  //   barrier (block b + 1 is in the ring); step 2 b + 1 likewise, refilled from
-  //   block b + 1.
-  // Block b + 1's slot held block b - 1, whose last fragments were read before
-  // block b - 1's barrier.  No load is under a run-time condition inside a
-  // round, so the compiler counts the loads in flight exactly; the first
-  // round is peeled so that the loop is entered in its steady state, and the
-  // last one loads nothing.
   f32x4 acc[MF][NF];
-#pragma unroll
-  for (int i = 0; i < MF; ++i)
-#pragma unroll
-    for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const unsigned char* const frag0 = s_ring + (16 * lg + (lr ^ lg)) * 16;
-  const unsigned char* const frag1 = s_ring + STEP + (16 * lg + (lr ^ lg ^ 12)) * 16;
-  u32x4 a[MF], w[NF];
-  auto read_a = [&](const unsigned char* at, int i) {
-    a[i] = *reinterpret_cast<const u32x4*>(at + (wm * MF + i) * 1024);
-  };
-  auto read_w = [&](const unsigned char* at, int j) {
-    w[j] = *reinterpret_cast<const u32x4*>(at + (MFC + wn * NF + j) * 1024);
-  };
-  constexpr int ROUND = AHEAD;                                // blocks per round: sets and slots are immediates
-  static_assert(ROUND == 2, "register sets and ring slots alternate together");
-  auto round = [&](int r, auto last_c) {
-    constexpr bool LAST = decltype(last_c)::value;
-#pragma unroll
-    for (int u = 0; u < ROUND; ++u) {
-      const int b = r * ROUND + u;
-      const bool more = !LAST || u + 1 < ROUND;               // block b + 1 exists
-      constexpr int S = ROUND;
-      if (more) write(b + 1, wr[(u + 1) % S], ar[(u + 1) % S]);
-      if (!LAST) {
-        // past the last block (the round before the last loads one too many) line() wraps: in bounds, unused
-        load_w(b + 1 + AHEAD, wr[(u + 1) % S]);
-        load_a(b + 1 + AHEAD, ar[(u + 1) % S]);
-      }
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const unsigned char* const next = h == 0 ? frag1 + u * SLOT : frag0 + (u ^ 1) * SLOT;
-        const bool refill = h == 0 || more;
-#pragma unroll
-        for (int j = 0; j < NF; ++j) {
-#pragma unroll
-          for (int i = 0; i < MF; ++i) {
-            mid_mfma<DT>(acc[i][j], w[j], a[i]);
-            if (refill && j == NF - 1) read_a(next, i);
-          }
-          if (refill) read_w(next, j);
-          asm volatile("" ::: "memory");
-        }
-        if (h == 0 && more) lds_barrier();
-      }
-    }
-  };
-  write(0, wr[0], ar[0]);
-  load_w(AHEAD, wr[0]);
-  load_a(AHEAD, ar[0]);
-  lds_barrier();
-#pragma unroll
-  for (int i = 0; i < MF; ++i) read_a(frag0, i);
-#pragma unroll
-  for (int j = 0; j < NF; ++j) read_w(frag0, j);
-  const int rounds = NB / ROUND;                              // NB is even and at least 4 (the host checks)
-  if (rounds > 1) {
-    round(0, std::integral_constant<bool, false>());
-    for (int r = 1; r < rounds - 1; ++r) round(r, std::integral_constant<bool, false>());
-  }
-  round(rounds - 1, std::integral_constant<bool, true>());
+  ring_loop<DT, MFC>(NB, s_ring, wr, ar, load_w, load_a, acc);
 
   // ---- epilogue: lane (lr, lg) of a fragment pair holds columns 8 lg .. 8 lg + 7 of row lr
-  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < MF; ++i)
-#pragma unroll
-    for (int j = 0; j < NF; ++j) pin_acc(acc[i][j]);
   T* const C = static_cast<T*>(p.C);
   if constexpr (!GEMM1) {
     if (__builtin_amdgcn_readfirstlane(*s_gave)) {            // the wait for act gave up
@@ -2150,7 +2034,7 @@ __device__ __forceinline__ void mid_body(const GemmParams& p, int unit, int n_cb
   // offsets[nl] < 0: the dispatch gave up; no expert has rows, the call is flagged
   {
     const int last = p.offsets[nl];
-    for (int j = tid; j <= nl; j += mid::NT) s_off[j] = last < 0 ? 0 : p.offsets[j];
+    for (int j = tid; j <= nl; j += ring::NT) s_off[j] = last < 0 ? 0 : p.offsets[j];
     if (last < 0 && unit == 0 && tid == 0 && p.flags != nullptr) atomic_or_1(p.flags, sched::kFlagInput);
   }
   __syncthreads();
@@ -2180,11 +2064,11 @@ __device__ __forceinline__ void mid_body(const GemmParams& p, int unit, int n_cb
 }
 
 template <int DT, int MFC>
-__global__ __launch_bounds__(mid::NT, 2) void moe_gemm_mid_kernel(GemmParams p1, GemmParams p2, int g1_blocks,
+__global__ __launch_bounds__(ring::NT, 2) void moe_gemm_mid_kernel(GemmParams p1, GemmParams p2, int g1_blocks,
                                                                   int* sched) {
   __shared__ int s_pre[bfk::NLMAX + 1];
   __shared__ int s_off[bfk::NLMAX + 1];
-  __shared__ __attribute__((aligned(16))) unsigned char s_ring[4 * (MFC + mid::WF) * 1024];
+  __shared__ __attribute__((aligned(16))) unsigned char s_ring[ring::lds_bytes(MFC)];
   __shared__ int s_gave;
   const int b = blockIdx.x;
   if (b < g1_blocks) mid_body<DT, MFC, true>(p1, b, 0, sched, s_pre, s_off, s_ring, &s_gave);
@@ -2196,7 +2080,7 @@ hipError_t launch_mid(const GemmParams& p1, const GemmParams& p2, int64_t max_ro
   // an XCD's range is at most ceil(chunks / 8) chunks
   const int64_t per_xcd = (mid::chunks(max_rows, p1.n_local, 16 * MFC) + 7) / 8;
   const int64_t b1 = 8 * per_xcd * (p1.N / 64), b2 = 8 * per_xcd * (p2.N / 128);
-  moe_gemm_mid_kernel<DT, MFC><<<dim3(static_cast<unsigned>(b1 + b2)), mid::NT, 0, stream>>>(
+  moe_gemm_mid_kernel<DT, MFC><<<dim3(static_cast<unsigned>(b1 + b2)), ring::NT, 0, stream>>>(
       p1, p2, static_cast<int>(b1), sched);
   return hipGetLastError();
 }

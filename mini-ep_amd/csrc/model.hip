@@ -14,6 +14,7 @@
 // the norm, a projection's output, the scaled residual term, the residual sum.
 #include "../../include/miniep_amd_model.h"
 #include "common.h"
+#include "ring_gemm.h"
 
 #include <initializer_list>
 #include <type_traits>
@@ -743,6 +744,114 @@ hipError_t launch_linear_rows(LinearParams p, int k, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// ============================================================================
+// Projections of more rows (bf16): out = x W^T for up to three weight matrices
+// in one launch.
+//
+// Tiles of 16 MFC rows by 128 columns, the experts' mid-size K loop
+// (ring_loop): q, k and v of one prompt batch fill the chip together where
+// three launches of larger tiles leave it half empty, each paying its own ramp.
+// Tiles are listed row chunk by row chunk and split into 8 contiguous ranges,
+// one per XCD: a chunk's rows are read into one L2.
+// us with q, k and v of 1024 + 512 + 512 columns, hidden 1024, three library
+// GEMMs -> this: 64 rows 24.7 -> 9.7, 512: 25 -> 10.6, 1024: 26 -> 11.4, 2048:
+// 28.5 -> 16.0, 4096: 33.6 -> 24.3, 8192: 48 -> 47; hidden 2048, 2048 + 512 +
+// 512 columns: 1024 rows 34 -> 25, 2048: 43 -> 38, 4096: 62 -> 65.  (A single
+// matrix is no faster than the library's: 2048 rows of 1024, 11.2.)  Bound by
+// the LDS (768 cycles of reads and writes for 512 of MFMAs per block of K) and,
+// with one workgroup on a CU, by the waits around a block's barrier; four
+// blocks of loads ahead instead of two change nothing.
+// ============================================================================
+struct LinearTileParams {
+  const uint16_t* x;          // (n, K)
+  const uint16_t* w[3];       // (cols[i], K)
+  uint16_t* out[3];           // (n, cols[i])
+  int cols[3];                // multiples of 128
+  int tiles[3];               // column tiles of matrices 0 .. i together
+  int n, K;
+};
+
+template <int MFC>
+__global__ __launch_bounds__(ring::NT, 2) void linear_tile_kernel(LinearTileParams p) {
+  constexpr int DT = MEP_DTYPE_BF16, CH = 16 * MFC, AP = MFC / 2, WP = ring::WP;
+  __shared__ __attribute__((aligned(16))) unsigned char s_ring[ring::lds_bytes(MFC)];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1, lr = lane & 15, lg = lane >> 4;
+  const int units = (p.n + CH - 1) / CH * p.tiles[2];
+  const int xcd = blockIdx.x & 7;
+  const int u = static_cast<int>(static_cast<int64_t>(units) * xcd / 8) + static_cast<int>(blockIdx.x >> 3);
+  if (u >= static_cast<int>(static_cast<int64_t>(units) * (xcd + 1) / 8)) return;
+  const int row0 = u / p.tiles[2] * CH, tile = u % p.tiles[2];
+  const int mat = tile < p.tiles[0] ? 0 : (tile < p.tiles[1] ? 1 : 2);
+  const int col0 = (tile - (mat == 0 ? 0 : p.tiles[mat - 1])) * 128;
+  const int row_bytes = p.K * 2, NB = row_bytes / 128;
+  const unsigned char* const W = reinterpret_cast<const unsigned char*>(p.w[mat]);
+  const unsigned char* const A = reinterpret_cast<const unsigned char*>(p.x);
+  const ring::Copy cp;
+  uint32_t w_off[WP], a_off[AP];                           // x and a matrix are below 4 GiB (the host checks)
+  // weight fragment 4 wn + j of the tile: row m of the pair's half j & 1 is
+  // column 8 (m / 4) + 4 (j & 1) + m % 4 of 32, so a lane's results across a
+  // pair are 8 consecutive columns
+#pragma unroll
+  for (int i = 0; i < WP; ++i) {
+    const int fr = 2 * i + cp.half, j = fr & 3;
+    const int row = col0 + 64 * (fr >> 2) + 32 * (j >> 1) + 8 * (cp.row16 >> 2) + 4 * (j & 1) + (cp.row16 & 3);
+    w_off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(row_bytes) + cp.chunk * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < AP; ++i)
+    a_off[i] = static_cast<uint32_t>(min(row0 + 32 * i + 16 * cp.half + cp.row16, p.n - 1)) *
+                   static_cast<uint32_t>(row_bytes) + cp.chunk * 16;
+  u32x4 wr[ring::AHEAD][WP], ar[ring::AHEAD][AP];
+  auto line = [&](int b) { return (b >= NB ? b - NB : b) * 128; };
+  auto load_w = [&](int b, u32x4 (&w)[WP]) {
+    const unsigned char* const base = W + line(b);
+#pragma unroll
+    for (int i = 0; i < WP; ++i) w[i] = *reinterpret_cast<const u32x4*>(base + w_off[i]);
+  };
+  auto load_a = [&](int b, u32x4 (&x)[AP]) {
+    const unsigned char* const base = A + line(b);
+#pragma unroll
+    for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const u32x4*>(base + a_off[i]);
+  };
+#pragma unroll
+  for (int b = 0; b < ring::AHEAD; ++b) {
+    load_w(b, wr[b]);
+    load_a(b, ar[b]);
+  }
+  f32x4 acc[MFC / 2][4];
+  ring_loop<DT, MFC>(NB, s_ring, wr, ar, load_w, load_a, acc);
+  const int N = p.cols[mat];
+#pragma unroll
+  for (int i = 0; i < MFC / 2; ++i) {
+    const int r = row0 + (wm * (MFC / 2) + i) * 16 + lr;
+    if (r >= p.n) continue;
+    const int64_t at = static_cast<int64_t>(r) * N + col0 + 64 * wn + 8 * lg;
+#pragma unroll
+    for (int jp = 0; jp < 2; ++jp) {
+      float v[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[c] = acc[i][2 * jp + (c >> 2)][c & 3];
+      *reinterpret_cast<u32x4*>(p.out[mat] + at + 32 * jp) = pack_chunk<DT>(v);
+    }
+  }
+}
+
+// Tiles of 128 rows read x and W through LDS less often, tiles of 64 rows are
+// taken while they fit the chip at once (us, hidden 1024, q + k + v of 2048
+// columns: 1024 rows 11.4 against 14.7 with 128, 2048 rows 16.5 against 16.0,
+// 4096 rows 27.8 against 24.3).
+hipError_t launch_linear_tile(const LinearTileParams& p, hipStream_t stream) {
+  auto go = [&](auto mfc) {
+    constexpr int MFC = decltype(mfc)::value;
+    const int64_t units = static_cast<int64_t>((p.n + 16 * MFC - 1) / (16 * MFC)) * p.tiles[2];
+    linear_tile_kernel<MFC><<<dim3(static_cast<unsigned>((units + 7) / 8 * 8)), ring::NT, 0, stream>>>(p);
+  };
+  if (static_cast<int64_t>((p.n + 63) / 64) * p.tiles[2] <= device_cu_count()) go(std::integral_constant<int, 4>());
+  else go(std::integral_constant<int, 8>());
+  return hipGetLastError();
+}
+
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 }  // namespace
@@ -945,6 +1054,42 @@ extern "C" int mep_norm_head(const void* h, const void* delta, float mult, const
   lin.out_mult = divisor;
   lin.n = static_cast<int>(n_rows);
   const hipError_t e = launch_linear_rows<true, kLinScaled>(lin, hidden, static_cast<hipStream_t>(stream));
+  MEP_REQUIRE(e == hipSuccess, MEP_ERR_HIP, "%s: launch failed: %s", fn, hipGetErrorString(e));
+  return MEP_OK;
+}
+
+extern "C" int mep_linear(const void* x, int64_t n_rows, int32_t k, const void* const* w, const int32_t* cols,
+                          int32_t n_mats, void* const* out, void* stream) {
+  clear_error();
+  const char* fn = "mep_linear";
+  MEP_REQUIRE(n_rows >= 0 && n_mats >= 1 && n_mats <= 3 && w && cols && out, MEP_ERR_INVALID_ARG, "%s: bad sizes", fn);
+  MEP_REQUIRE(k >= 256 && k % 128 == 0 && k <= (1 << 20), MEP_ERR_UNSUPPORTED,
+              "%s: K %d must be a multiple of 128, at least 256", fn, k);
+  MEP_REQUIRE(n_rows * k < (int64_t(1) << 31) && n_rows < (int64_t(1) << 23), MEP_ERR_UNSUPPORTED, "%s: x too large", fn);
+  LinearTileParams p{};
+  int64_t tiles = 0;
+  for (int i = 0; i < 3; ++i) {
+    p.cols[i] = i < n_mats ? cols[i] : 0;
+    MEP_REQUIRE(i >= n_mats || (p.cols[i] > 0 && p.cols[i] % 128 == 0 &&
+                                static_cast<int64_t>(p.cols[i]) * k < (int64_t(1) << 31)), MEP_ERR_UNSUPPORTED,
+                "%s: %d columns must be a multiple of 128", fn, p.cols[i]);
+    tiles += p.cols[i] / 128;
+    p.tiles[i] = static_cast<int>(tiles);
+  }
+  MEP_REQUIRE((n_rows + 63) / 64 * tiles < (int64_t(1) << 31), MEP_ERR_UNSUPPORTED, "%s: too many tiles", fn);
+  if (n_rows == 0) return MEP_OK;
+  MEP_REQUIRE(x != nullptr && aligned16(x), MEP_ERR_INVALID_ARG,
+              "%s: buffers must be present and 16-byte aligned", fn);
+  for (int i = 0; i < n_mats; ++i) {
+    MEP_REQUIRE(w[i] && out[i] && aligned16(w[i]) && aligned16(out[i]), MEP_ERR_INVALID_ARG,
+                "%s: buffers must be present and 16-byte aligned", fn);
+    p.w[i] = static_cast<const uint16_t*>(w[i]);
+    p.out[i] = static_cast<uint16_t*>(out[i]);
+  }
+  p.x = static_cast<const uint16_t*>(x);
+  p.n = static_cast<int>(n_rows);
+  p.K = k;
+  const hipError_t e = launch_linear_tile(p, static_cast<hipStream_t>(stream));
   MEP_REQUIRE(e == hipSuccess, MEP_ERR_HIP, "%s: launch failed: %s", fn, hipGetErrorString(e));
   return MEP_OK;
 }

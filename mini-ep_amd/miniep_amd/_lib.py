@@ -94,6 +94,7 @@ _SIGNATURES = {
                                            _c_void_p, _c_void_p, _size, _c_void_p, _c_void_p, _c_void_p]),
     "mep_norm_head": (ctypes.c_int, [_c_void_p, _c_void_p, ctypes.c_float, _c_void_p, ctypes.c_float, _c_void_p, _i64,
                                      _i32, _i32, ctypes.c_float, _c_void_p, _c_void_p]),
+    "mep_linear": (ctypes.c_int, [_c_void_p, _i64, _i32, _c_void_p, _c_void_p, _i32, _c_void_p, _c_void_p]),
     "mep_experts_workspace_size": (_size, [_i64, _i32, _i32]),
     "mep_experts_queue_ints": (_size, [_i64, _i32]),
     "mep_experts_check": (ctypes.c_int, [_c_void_p, _c_void_p]),

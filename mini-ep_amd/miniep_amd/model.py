@@ -289,7 +289,8 @@ class GraniteMoeModel:
                                            ws)
             else:
                 h, x = ops.add_norm(h, norm1, eps, moe_out, rm)
-                q, k, v = (F.linear(x, w[k_[m]]) for m in ("wq", "wk", "wv"))
+                proj = [w[k_[m]] for m in ("wq", "wk", "wv")]
+                q, k, v = ops.linear(x, proj) if ops.tiled_linear(x, proj) else (F.linear(x, m) for m in proj)
                 o = ops.attention(q, k, v, cos, sin, B, start, kc, vc, scale)
                 h, x = ops.add_norm(h, norm2, eps, F.linear(o, w[k_["wo"]]), rm)
             moe_out = self._moe_block(layer, x, moe_valid).contiguous()

@@ -613,6 +613,40 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tens
     return out
 
 
+def tiled_linear(x: torch.Tensor, weights) -> bool:
+    """Whether `linear` takes these operands and is faster than one library
+    GEMM per matrix: up to two 128 x 128 tiles per CU (us, hidden 1024, q + k +
+    v of 2048 columns: 2048 rows 28.5 -> 16.0, 4096 rows (two tiles) 33.6 ->
+    24.3, 8192 rows 48 -> 47; hidden 2048, 3072 columns: 2048 rows 43 -> 38,
+    3000 rows 54 -> 58)."""
+    n, k = x.shape
+    cols = [w.shape[0] for w in weights]
+    if k % 128 or k < 256 or any(c % 128 for c in cols) or max(n, *cols) * k >= 1 << 31 or \
+            any(t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16 for t in (x, *weights)):
+        return False
+    cus = torch.cuda.get_device_properties(x.device).multi_processor_count
+    return (n + 127) // 128 * (sum(cols) // 128) <= 2 * cus
+
+
+def linear(x: torch.Tensor, weights) -> list[torch.Tensor]:
+    """x (n, k) @ w^T for one to three bf16 matrices (cols, k) in one launch
+    (mep_linear); k a multiple of 128, at least 256, cols multiples of 128."""
+    dev = _require_device(x, *weights)
+    for t in (x, *weights):
+        if t.dtype != torch.bfloat16 or not t.is_contiguous():
+            raise TypeError("linear takes contiguous bf16 tensors")
+    n, k = x.shape
+    m = len(weights)
+    if any(w.dim() != 2 or w.shape[1] != k for w in weights):
+        raise ValueError("linear: shapes do not match")
+    out = [torch.empty(n, w.shape[0], dtype=x.dtype, device=dev) for w in weights]
+    rc = _lib.lib().mep_linear(x.data_ptr(), n, k, (ctypes.c_void_p * m)(*(w.data_ptr() for w in weights)),
+                               (ctypes.c_int32 * m)(*(w.shape[0] for w in weights)), m,
+                               (ctypes.c_void_p * m)(*(o.data_ptr() for o in out)), _stream(dev))
+    _lib.check(rc, "mep_linear")
+    return out
+
+
 def small_rows(n_rows: int, hidden: int, dtype: torch.dtype) -> bool:
     """Whether attention_block / norm_head take n_rows rows of this width."""
     return n_rows <= 32 and hidden in (1024, 2048) and dtype == torch.bfloat16

@@ -157,3 +157,19 @@ def test_attention_block(B, T, start, H, hq, hk):
             # one bf16 step of the element (or of the rotation's other half), seldom
             assert ((a - b).abs() <= most * b.abs() + 2.0 ** -7 * b.abs().mean()).float().mean() > 0.999
             assert float((a - b).norm() / b.norm()) <= 2e-3
+
+
+@pytest.mark.parametrize("n,K,cols", [
+    (1, 256, (128,)), (33, 1024, (1024, 512, 512)), (64, 1024, (128, 128)), (65, 384, (128, 256, 128)),
+    (130, 512, (256,)), (1024, 1024, (1024, 512, 512)), (1025, 1024, (1024, 512, 512)), (4097, 256, (512, 128))])
+def test_linear(n, K, cols):
+    """Tiles of 64 and of 128 rows, partial last tiles, one to three matrices,
+    the shortest K.  Products of bf16 are exact in fp32: K roundings at most of
+    sums below |x| |w|, then one to bf16."""
+    g = torch.Generator().manual_seed(n + K)
+    x = torch.randn(n, K, generator=g).bfloat16().to(DEV)
+    ws = [(torch.randn(c, K, generator=g) * 0.02).bfloat16().to(DEV) for c in cols]
+    for w, got in zip(ws, ops.linear(x, ws)):
+        want = x.double() @ w.double().T.contiguous()
+        tol = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T.contiguous())
+        assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + tol).all()
