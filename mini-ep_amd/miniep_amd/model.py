@@ -249,12 +249,14 @@ class GraniteMoeModel:
         if cfg.hidden_size > 4096 or cfg.hidden_size % 8 or B * T == 0 or B * hq > 65535:
             return False
         start = 0 if cache is None else cache.length
-        if start + T > self.rope.cos.shape[0]:
-            return False
+        for t in (self.rope.cos, self.rope.sin):
+            if start + T > t.shape[0] or t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16:
+                return False
         if cache is not None:
             shape = (B, hk, cache.max_len, d)
             for c in (*cache.k, *cache.v):
-                if c.dtype != torch.float32 or c.device != e.device or c.shape != shape or not c.is_contiguous():
+                if c.dtype != torch.float32 or c.device != e.device or c.shape != shape or not c.is_contiguous() or \
+                        c.data_ptr() % 16:
                     return False
             if start + T > cache.max_len:
                 return False
@@ -294,6 +296,8 @@ class GraniteMoeModel:
                 o = ops.attention(q, k, v, cos, sin, B, start, kc, vc, scale)
                 h, x = ops.add_norm(h, norm2, eps, F.linear(o, w[k_["wo"]]), rm)
             moe_out = self._moe_block(layer, x, moe_valid).contiguous()
+            if moe_out.data_ptr() % 16:                              # a backend's view into something larger
+                moe_out = moe_out.clone()
         if logits_at is not None:
             at = (torch.arange(B, device=h.device), logits_at)
             h, moe_out = (None if z is None else z.view(B, T, H)[at] for z in (h, moe_out))

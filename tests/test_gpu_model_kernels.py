@@ -101,6 +101,28 @@ def test_native_forward_equals_torch_statement(dtype):
     assert got.shape == (3, 1, cfg.vocab_size) and float((got - want).norm() / want.norm()) <= tol
 
 
+def test_native_forward_with_unaligned_tensors():
+    """A backend that returns a view off the 16-byte grid, and such a cache:
+    accepted, with the results of aligned ones (the cache goes through the torch
+    statement, so to its rounding)."""
+    cfg = ModelConfig(num_hidden_layers=2, vocab_size=997)
+    m = build_hip_model(cfg, random_weights(cfg, seed=3, dtype=torch.bfloat16, device=DEV))
+    ids = torch.randint(0, cfg.vocab_size, (2, 40), generator=torch.Generator().manual_seed(1)).to(DEV)
+    want = m(ids)
+
+    def off_grid(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.reshape(-1)
+        return flat[1:].view(t.shape)
+
+    cache = KVCache(cfg, 2, 40, DEV)
+    cache.k = [off_grid(t) for t in cache.k]
+    assert float((m(ids, cache=cache) - want).norm() / want.norm()) <= 2e-2
+    inner = m.moe[0].route_and_call
+    m.moe[0].route_and_call = lambda *a, **kw: (off_grid(inner(*a, **kw)[0]),)
+    assert torch.equal(m(ids), want)
+
+
 def _norm64(h, w):
     return w.double() * h.double() * torch.rsqrt(h.double().pow(2).mean(-1, keepdim=True) + 1e-6)
 
