@@ -1922,19 +1922,13 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
     if (kb >= NB) kb -= NB;
     return kb * 128;
   };
-  auto load_w = [&](int b, u32x4 (&w)[WP]) {
-    const unsigned char* const base = W + line(b);
-#pragma unroll
-    for (int i = 0; i < WP; ++i) w[i] = *reinterpret_cast<const u32x4*>(base + w_off[i]);
-  };
-  auto load_a = [&](int b, u32x4 (&x)[AP]) {
-    const unsigned char* const base = A + line(b);
-#pragma unroll
-    for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const u32x4*>(base + a_off[i]);
-  };
+  auto load_w = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(W + line(b) + w_off[i]); };
+  auto load_a = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(A + line(b) + a_off[i]); };
   // the weights need neither the row map nor GEMM-1
 #pragma unroll
-  for (int b = 0; b < AHEAD; ++b) load_w(b, wr[b]);
+  for (int b = 0; b < AHEAD; ++b)
+#pragma unroll
+    for (int i = 0; i < WP; ++i) wr[b][i] = load_w(b, i);
 
   int* const done1 = sched + sched::mid_word(q);
   int* const seen2 = done1 + 1;
@@ -1965,7 +1959,9 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
     a_off[i] = from * static_cast<uint32_t>(row_bytes) + cc * 16;
   }
 #pragma unroll
-  for (int b = 0; b < AHEAD; ++b) load_a(b, ar[b]);
+  for (int b = 0; b < AHEAD; ++b)
+#pragma unroll
+    for (int i = 0; i < AP; ++i) ar[b][i] = load_a(b, i);
 
   f32x4 acc[MF][NF];
   ring_loop<DT, MFC>(NB, s_ring, wr, ar, load_w, load_a, acc);
@@ -2739,7 +2735,7 @@ bool tiled_down(int dtype, int64_t max_rows, int inter) {
 //    fill whole rounds of the CUs: 1500 tokens 67 against 72, 4096 tokens 116
 //    against 143, 2500 tokens 98 against 103;
 //  - this one below (64 tokens 27 -> 23, 128: 43 -> 24, 256: 57 -> 29, 517:
-//    52 -> 37, 1024: 60 -> 50), where an expert's rows fill at most half a
+//    52 -> 36, 1024: 60 -> 48), where an expert's rows fill at most half a
 //    row tile (hidden 2048, 64 experts, 500 tokens: 216 -> 195), and where the
 //    tiled launch's second round would be nearly empty (2048 tokens: 92 -> 82).
 int mid_row_frags(int64_t max_rows, int n_local, int inter) {
@@ -2751,10 +2747,10 @@ int mid_row_frags(int64_t max_rows, int n_local, int inter) {
   if (!sparse && tiles * 4 > cu * 3 && !(tiles > cu && tiles * 20 <= cu * 27)) return 0;
   // chunks of 128 rows read the weights half as often as chunks of 64, if the
   // experts have that many rows and the chip is still full (128 tokens: even;
-  // 384 tokens: 34 -> 30, 700: 47 -> 42; 10 experts with 120 rows each: 19 with
-  // 64, 25 with 128)
+  // 384 tokens: 34 -> 30; 517: skewed routing 49 -> 42, flat 42 -> 43; 700: 47 ->
+  // 42; 10 experts with 120 rows each: 19 with 64, 25 with 128)
   const int64_t units = (max_rows / 128 + n_local / 2) * (inter / 64);
-  return max_rows >= static_cast<int64_t>(n_local) * 64 && units * 4 >= cu * (sparse ? 4 : 7) ? 8 : 4;
+  return max_rows >= static_cast<int64_t>(n_local) * 64 && units * 4 >= cu * (sparse ? 4 : 6) ? 8 : 4;
 }
 
 // fp32, every size: chunks of 64 rows, or of 32 while those of 64 are too few

@@ -754,13 +754,13 @@ hipError_t launch_linear_rows(LinearParams p, int k, hipStream_t stream) {
 // Tiles are listed row chunk by row chunk and split into 8 contiguous ranges,
 // one per XCD: a chunk's rows are read into one L2.
 // us with q, k and v of 1024 + 512 + 512 columns, hidden 1024, three library
-// GEMMs -> this: 64 rows 24.7 -> 9.7, 512: 25 -> 10.6, 1024: 26 -> 11.4, 2048:
-// 28.5 -> 16.0, 4096: 33.6 -> 24.3, 8192: 48 -> 47; hidden 2048, 2048 + 512 +
-// 512 columns: 1024 rows 34 -> 25, 2048: 43 -> 38, 4096: 62 -> 65.  (A single
-// matrix is no faster than the library's: 2048 rows of 1024, 11.2.)  Bound by
-// the LDS (768 cycles of reads and writes for 512 of MFMAs per block of K) and,
-// with one workgroup on a CU, by the waits around a block's barrier; four
-// blocks of loads ahead instead of two change nothing.
+// GEMMs -> this: 64 rows 24.7 -> 8.9, 512: 25 -> 9.9, 1024: 26 -> 11.1, 2048:
+// 28.5 -> 14.8, 4096: 33.2 -> 21.7, 8192: 45 -> 39; hidden 2048, 2048 + 512 +
+// 512 columns: 1024 rows 34 -> 22, 2048: 42 -> 34, 3000: 51 -> 53, 4096: 60 ->
+// 55.  (A single matrix is no faster than the library's: 2048 rows of 1024,
+// 11.2.)  Bound by the LDS (756 cycles of reads and writes for 512 of MFMAs per
+// block of K) and, with one workgroup on a CU, by the waits around a block's
+// barrier; four blocks of loads ahead instead of two change nothing.
 // ============================================================================
 struct LinearTileParams {
   const uint16_t* x;          // (n, K)
@@ -804,20 +804,14 @@ __global__ __launch_bounds__(ring::NT, 2) void linear_tile_kernel(LinearTilePara
                    static_cast<uint32_t>(row_bytes) + cp.chunk * 16;
   u32x4 wr[ring::AHEAD][WP], ar[ring::AHEAD][AP];
   auto line = [&](int b) { return (b >= NB ? b - NB : b) * 128; };
-  auto load_w = [&](int b, u32x4 (&w)[WP]) {
-    const unsigned char* const base = W + line(b);
-#pragma unroll
-    for (int i = 0; i < WP; ++i) w[i] = *reinterpret_cast<const u32x4*>(base + w_off[i]);
-  };
-  auto load_a = [&](int b, u32x4 (&x)[AP]) {
-    const unsigned char* const base = A + line(b);
-#pragma unroll
-    for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const u32x4*>(base + a_off[i]);
-  };
+  auto load_w = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(W + line(b) + w_off[i]); };
+  auto load_a = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(A + line(b) + a_off[i]); };
 #pragma unroll
   for (int b = 0; b < ring::AHEAD; ++b) {
-    load_w(b, wr[b]);
-    load_a(b, ar[b]);
+#pragma unroll
+    for (int i = 0; i < WP; ++i) wr[b][i] = load_w(b, i);
+#pragma unroll
+    for (int i = 0; i < AP; ++i) ar[b][i] = load_a(b, i);
   }
   f32x4 acc[MFC / 2][4];
   ring_loop<DT, MFC>(NB, s_ring, wr, ar, load_w, load_a, acc);
@@ -839,8 +833,9 @@ __global__ __launch_bounds__(ring::NT, 2) void linear_tile_kernel(LinearTilePara
 
 // Tiles of 128 rows read x and W through LDS less often, tiles of 64 rows are
 // taken while they fit the chip at once (us, hidden 1024, q + k + v of 2048
-// columns: 1024 rows 11.4 against 14.7 with 128, 2048 rows 16.5 against 16.0,
-// 4096 rows 27.8 against 24.3).
+// columns, before the writes were spread over the MFMA groups: 1024 rows 11.4
+// against 14.7 with 128, 2048 rows 16.5 against 16.0, 4096 rows 27.8 against
+// 24.3).
 hipError_t launch_linear_tile(const LinearTileParams& p, hipStream_t stream) {
   auto go = [&](auto mfc) {
     constexpr int MFC = decltype(mfc)::value;

@@ -61,20 +61,25 @@ struct Copy {
 // acc[i][j] = the products of row fragment i and weight fragment j of this
 // wave (wave 2 wm + wn: row fragments wm MFC/2 .., weight fragments 4 wn ..)
 // over NB blocks of one 128-byte line (two K-steps) per row; NB even, at least
-// 4.  load_w(b, r) / load_a(b, r) load block b of this thread's rows, pass by
-// pass; wr[b], ar[b] hold blocks 0 .. AHEAD - 1 on entry.  One load past the
-// last block is made and not used.
+// 4.  load_w(b, i) / load_a(b, i) load block b of this thread's row of pass i;
+// wr[b], ar[b] hold blocks 0 .. AHEAD - 1 on entry.  Loads up to two
+// blocks past the last one are made and not used.
 //
-// Block b (steps 2 b, 2 b + 1), with its first step's fragments in registers:
-//   write block b + 1 (in registers) to the ring, load block b + 1 + AHEAD;
-//   step 2 b: MFMAs, each fragment refilled with step 2 b + 1's after its last use;
-//   barrier (block b + 1 is in the ring); step 2 b + 1 likewise, refilled from
-//   block b + 1.
-// Block b + 1's slot held block b - 1, whose last fragments were read before
-// block b - 1's barrier.  No load is under a run-time condition inside a
-// round, so the compiler counts the loads in flight exactly; the first
-// round is peeled so that the loop is entered in its steady state, and the
-// last one loads nothing.
+// Block b (steps 2 b, 2 b + 1), with its first step's fragments and the rows of
+// block b + 1 in place:
+//   step 2 b: MFMAs; between their groups the weights of block b + 1 go from
+//   registers to the ring and step 2 b + 1's fragments come from it (rows into a
+//   second set, a weight fragment after its last use); load the weights of
+//   block b + 3; barrier: block b + 1 is in the ring, block b's slot free;
+//   step 2 b + 1 likewise, with the rows of block b + 2 into that slot, its next
+//   fragments from block b + 1; load the rows of block b + 4.
+// The writes are the slower side of the LDS (75 B/clk, reads about 200), so they
+// are spread over a block's MFMA groups: all at its start they hold up the
+// fragment reads behind them (a block of 128 x 128 with one workgroup on a CU
+// 1433 -> 1156 cycles, with two 2269 -> 1960; its MFMAs take 512 and 1024).
+// No load is under a run-time condition inside a round, so the compiler
+// counts the loads in flight exactly; the first round is peeled so that the
+// loop is entered in its steady state, and the last one loads nothing.
 //
 // The ring holds MFMA fragments of 1 KiB, lane (lr, lg)'s 16 bytes in slot
 // 16 lg + (lr ^ lg ^ 12 (step & 1)); a copying lane group takes rows 4 apart.
@@ -92,12 +97,11 @@ __device__ __forceinline__ void ring_loop(int NB, unsigned char* s_ring, u32x4 (
   const ring::Copy cp;
   const int clg = cp.chunk & 3, cstep = cp.chunk >> 2;
   unsigned char* const cdst = s_ring + cstep * STEP + cp.half * 1024 + (16 * clg + (cp.row16 ^ clg ^ (12 * cstep))) * 16;
-  auto write = [&](int b, const u32x4 (&w)[WP], const u32x4 (&x)[AP]) {
-    unsigned char* const dst = cdst + (b & 1) * SLOT;
-#pragma unroll
-    for (int i = 0; i < AP; ++i) *reinterpret_cast<u32x4*>(dst + 2 * i * 1024) = x[i];
-#pragma unroll
-    for (int i = 0; i < WP; ++i) *reinterpret_cast<u32x4*>(dst + (MFC + 2 * i) * 1024) = w[i];
+  auto write_a = [&](int slot, int i, const u32x4& v) {
+    *reinterpret_cast<u32x4*>(cdst + slot * SLOT + 2 * i * 1024) = v;
+  };
+  auto write_w = [&](int slot, int i, const u32x4& v) {
+    *reinterpret_cast<u32x4*>(cdst + slot * SLOT + (MFC + 2 * i) * 1024) = v;
   };
 #pragma unroll
   for (int i = 0; i < MF; ++i)
@@ -105,60 +109,75 @@ __device__ __forceinline__ void ring_loop(int NB, unsigned char* s_ring, u32x4 (
     for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const unsigned char* const frag0 = s_ring + (16 * lg + (lr ^ lg)) * 16;
   const unsigned char* const frag1 = s_ring + STEP + (16 * lg + (lr ^ lg ^ 12)) * 16;
-  u32x4 a[MF], w[NF];
-  auto read_a = [&](const unsigned char* at, int i) {
-    a[i] = *reinterpret_cast<const u32x4*>(at + (wm * MF + i) * 1024);
+  u32x4 a[2][MF], w[NF];
+  auto read_a = [&](const unsigned char* at, int h, int i) {
+    a[h][i] = *reinterpret_cast<const u32x4*>(at + (wm * MF + i) * 1024);
   };
   auto read_w = [&](const unsigned char* at, int j) {
     w[j] = *reinterpret_cast<const u32x4*>(at + (MFC + wn * NF + j) * 1024);
   };
-  constexpr int ROUND = ring::AHEAD;                    // blocks per round: sets and slots are immediates
-  static_assert(ROUND % 2 == 0, "a block's register set and ring slot are fixed by its place in the round");
+  constexpr int ROUND = ring::AHEAD;                          // blocks per round: sets and slots are immediates
+  static_assert(ROUND == 2, "register sets and ring slots alternate together");
+  static_assert(AP <= NF && WP == NF, "a block's writes fit one per MFMA group");
   auto round = [&](int r, auto last_c) {
     constexpr bool LAST = decltype(last_c)::value;
 #pragma unroll
     for (int u = 0; u < ROUND; ++u) {
       const int b = r * ROUND + u;
-      const bool more = !LAST || u + 1 < ROUND;               // block b + 1 exists
-      constexpr int S = ROUND;
-      if (more) write(b + 1, wr[(u + 1) % S], ar[(u + 1) % S]);
-      if (!LAST) {
-        // past the last block (the round before the last loads one too many) line() wraps: in bounds, unused
-        load_w(b + 1 + ring::AHEAD, wr[(u + 1) % S]);
-        load_a(b + 1 + ring::AHEAD, ar[(u + 1) % S]);
-      }
+      const bool more = !LAST || u == 0;                      // block b + 1 exists
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const unsigned char* const next = h == 0 ? frag1 + (u & 1) * SLOT : frag0 + (~u & 1) * SLOT;
+        const unsigned char* const next = h == 0 ? frag1 + u * SLOT : frag0 + (u ^ 1) * SLOT;
         const bool refill = h == 0 || more;
 #pragma unroll
         for (int j = 0; j < NF; ++j) {
 #pragma unroll
-          for (int i = 0; i < MF; ++i) {
-            ring_mfma<DT>(acc[i][j], w[j], a[i]);
-            if (refill && j == NF - 1) read_a(next, i);
+          for (int i = 0; i < MF; ++i) ring_mfma<DT>(acc[i][j], w[j], a[h][i]);
+          if (h == 0 && more) write_w(u ^ 1, j, wr[u ^ 1][j]);
+          if (h == 1 && !LAST && j < AP) write_a(u, j, ar[u][j]);
+          // (all of the next step's row fragments are used by its first group)
+          if (refill && 2 * j < MF) {
+            read_a(next, h ^ 1, 2 * j);
+            if (2 * j + 1 < MF) read_a(next, h ^ 1, 2 * j + 1);
           }
           if (refill) read_w(next, j);
           asm volatile("" ::: "memory");
         }
+        // past the last block (the round before the last loads two too many) the line wraps: in bounds, unused
+        if (h == 0 && !LAST)
+#pragma unroll
+          for (int i = 0; i < WP; ++i) wr[u ^ 1][i] = load_w(b + 3, i);
+        if (h == 1 && !LAST)
+#pragma unroll
+          for (int i = 0; i < AP; ++i) ar[u][i] = load_a(b + 4, i);
         if (h == 0 && more) lds_barrier();
       }
     }
   };
-  write(0, wr[0], ar[0]);
-  load_w(ring::AHEAD, wr[0]);
-  load_a(ring::AHEAD, ar[0]);
+#pragma unroll
+  for (int i = 0; i < AP; ++i) write_a(0, i, ar[0][i]);
+#pragma unroll
+  for (int i = 0; i < WP; ++i) write_w(0, i, wr[0][i]);
+#pragma unroll
+  for (int i = 0; i < WP; ++i) wr[0][i] = load_w(2, i);
+#pragma unroll
+  for (int i = 0; i < AP; ++i) ar[0][i] = load_a(2, i);
+#pragma unroll
+  for (int i = 0; i < AP; ++i) write_a(1, i, ar[1][i]);
+#pragma unroll
+  for (int i = 0; i < AP; ++i) ar[1][i] = load_a(3, i);
   lds_barrier();
 #pragma unroll
-  for (int i = 0; i < MF; ++i) read_a(frag0, i);
+  for (int i = 0; i < MF; ++i) read_a(frag0, 0, i);
 #pragma unroll
   for (int j = 0; j < NF; ++j) read_w(frag0, j);
-  const int rounds = NB / ROUND;                              // NB is even and at least 4 (the host checks)
-  if (rounds > 1) {
-    round(0, std::integral_constant<bool, false>());
-    for (int r = 1; r < rounds - 1; ++r) round(r, std::integral_constant<bool, false>());
-  }
-  round(rounds - 1, std::integral_constant<bool, true>());
+  std::integral_constant<bool, true> yes;
+  std::integral_constant<bool, false> no;
+  const int rounds = NB / ROUND;                              // at least 2
+  round(0, no);
+  for (int r = 1; r < rounds - 1; ++r) round(r, no);
+  round(rounds - 1, yes);
+
   // the MFMAs are inline asm: wait out the last ones before acc is read
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 #pragma unroll

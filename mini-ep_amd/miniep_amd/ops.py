@@ -616,9 +616,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tens
 def tiled_linear(x: torch.Tensor, weights) -> bool:
     """Whether `linear` takes these operands and is faster than one library
     GEMM per matrix: up to two 128 x 128 tiles per CU (us, hidden 1024, q + k +
-    v of 2048 columns: 2048 rows 28.5 -> 16.0, 4096 rows (two tiles) 33.6 ->
-    24.3, 8192 rows 48 -> 47; hidden 2048, 3072 columns: 2048 rows 43 -> 38,
-    3000 rows 54 -> 58)."""
+    v of 2048 columns: 2048 rows 28.5 -> 14.8, 4096 rows (two tiles) 33.2 ->
+    21.7; hidden 2048, 3072 columns: 2048 rows 42 -> 34, 3000 rows 51 -> 53)."""
     n, k = x.shape
     cols = [w.shape[0] for w in weights]
     if k % 128 or k < 256 or any(c % 128 for c in cols) or max(n, *cols) * k >= 1 << 31 or \
