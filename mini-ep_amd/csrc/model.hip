@@ -1,6 +1,6 @@
 // The transformer around the MoE block (gfx950): residual adds and RMSNorm,
-// rotary embedding with the KV cache, causal attention, and the projections of
-// small batches.
+// rotary embedding with the KV cache, causal attention, the projections of small
+// batches, and q, k and v of larger ones.
 //
 // Replaces, in the reference's model (modeling.py):
 //   RMSNorm                                      :55-63

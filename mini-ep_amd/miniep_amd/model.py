@@ -25,7 +25,8 @@ with ``fuse_router`` (``build_hip_model``) runs the norms, residual adds, RoPE,
 cache writes and attention on the HIP kernels of ``ops`` (``add_norm``,
 ``attention``: head size 64, 1, 2 or 4 query heads per kv head, fp32 cache), and
 with at most 32 rows in bf16 the projections and the head (``attention_block``,
-``norm_head``).
+``norm_head``), with more the q, k and v projections (``linear``, where
+``tiled_linear`` says so).
 Everything else, a model with other MoE backends among it, runs the torch
 statement of the same model below.
 """
