@@ -1917,11 +1917,7 @@ __device__ __forceinline__ void mid_chunk(const GemmParams& p, int e, int q, int
     w_off[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(row_bytes) + cc * 16;
   }
   u32x4 wr[AHEAD][WP], ar[AHEAD][AP];
-  auto line = [&](int b) {                                    // byte offset of block b's line of a row
-    int kb = b + rot;
-    if (kb >= NB) kb -= NB;
-    return kb * 128;
-  };
+  auto line = [&](int b) { return ring::block_at(b, rot, NB) * 128; };   // byte offset of block b's line of a row
   auto load_w = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(W + line(b) + w_off[i]); };
   auto load_a = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(A + line(b) + a_off[i]); };
   // the weights need neither the row map nor GEMM-1

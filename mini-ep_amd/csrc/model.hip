@@ -803,7 +803,7 @@ __global__ __launch_bounds__(ring::NT, 2) void linear_tile_kernel(LinearTilePara
     a_off[i] = static_cast<uint32_t>(min(row0 + 32 * i + 16 * cp.half + cp.row16, p.n - 1)) *
                    static_cast<uint32_t>(row_bytes) + cp.chunk * 16;
   u32x4 wr[ring::AHEAD][WP], ar[ring::AHEAD][AP];
-  auto line = [&](int b) { return (b >= NB ? b - NB : b) * 128; };
+  auto line = [&](int b) { return ring::block_at(b, 0, NB) * 128; };
   auto load_w = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(W + line(b) + w_off[i]); };
   auto load_a = [&](int b, int i) { return *reinterpret_cast<const u32x4*>(A + line(b) + a_off[i]); };
 #pragma unroll

@@ -4,6 +4,7 @@
 #pragma once
 
 #include "common.h"
+#include "ring_blocks.h"
 
 #include <type_traits>
 
@@ -40,7 +41,6 @@ __device__ __forceinline__ void ring_mfma(f32x4& acc, const u32x4& w, const u32x
 
 namespace ring {
 constexpr int NT = 256;
-constexpr int AHEAD = 2;                      // blocks (two K-steps) of loads in flight
 constexpr int WF = 8;                         // weight fragments of a workgroup: 128 weight rows
 constexpr int WP = WF / 2;                    // copy passes of 32 weight rows
 constexpr int lds_bytes(int mfc) { return 4 * (mfc + WF) * 1024; }
@@ -63,7 +63,8 @@ struct Copy {
 // over NB blocks of one 128-byte line (two K-steps) per row; NB even, at least
 // 4.  load_w(b, i) / load_a(b, i) load block b of this thread's row of pass i;
 // wr[b], ar[b] hold blocks 0 .. AHEAD - 1 on entry.  Loads up to two
-// blocks past the last one are made and not used.
+// blocks past the last one are made and not used (ring::block_at keeps them in
+// the row).
 //
 // Block b (steps 2 b, 2 b + 1), with its first step's fragments and the rows of
 // block b + 1 in place:
@@ -143,7 +144,7 @@ __device__ __forceinline__ void ring_loop(int NB, unsigned char* s_ring, u32x4 (
           if (refill) read_w(next, j);
           asm volatile("" ::: "memory");
         }
-        // past the last block (the round before the last loads two too many) the line wraps: in bounds, unused
+        // (the round before the last loads blocks NB and NB + 1 of the rows: unused)
         if (h == 0 && !LAST)
 #pragma unroll
           for (int i = 0; i < WP; ++i) wr[u ^ 1][i] = load_w(b + 3, i);

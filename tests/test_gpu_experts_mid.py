@@ -37,6 +37,10 @@ def _case(counts, k, H, I, seed, dtype=BF):
     # 128-row chunks: an average of 64 rows and more, enough column blocks
     ("edges128", [64, 1, 127, 128, 129, 63, 65, 16] * 4, 4, 512, 1024),
     ("k256", [40, 100, 7, 210, 11, 0, 64, 80], 2, 256, 256),       # the shortest K loops, no rotation of whole quarters
+    # the shortest K loop with every rotation of it, 64- and 128-row chunks, several chunks of an expert
+    ("k256_rot64", [130, 1, 65, 64, 200, 0, 96, 84], 2, 1024, 256),
+    ("k256_rot64_wide", [40, 100, 7, 210, 11, 0, 64, 80], 2, 2048, 256),
+    ("k256_rot128", [64, 1, 127, 128, 129, 63, 257, 16] * 8, 5, 1024, 256),
     ("one_expert", [300], 1, 1024, 512),                            # fewer chunks than XCDs
     ("e64_wide", [5] * 63 + [197], 2, 2048, 1024),
     ("hot", [1000, 8, 8, 8, 8, 8, 4, 4], 1, 1024, 512),

@@ -7,6 +7,9 @@ slots per rank (scripts/make_plan.py:24-29).
 """
 import ctypes
 import json
+import shutil
+import subprocess
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -197,3 +200,33 @@ def test_dispatch_noalloc_rejects_calls_beyond_its_scratch():
     rc = L.mep_dispatch_noalloc(fake, None, n, 8, 256, fake, fake, 1, 0, None, seg, 1, 0, fake, 256,
                                 fake, fake, fake, fake, None, None, None, None)
     assert rc == _lib.ERR_UNSUPPORTED and b"static scratch" in L.mep_last_error()
+
+
+CSRC = Path(__file__).resolve().parents[1] / "mini-ep_amd" / "csrc"
+
+
+def test_ring_loop_blocks_stay_in_the_row(tmp_path):
+    """Every block that the GEMM ring loop loads (its index runs AHEAD past the
+    last one) lies in the row, for every K of at least four blocks and every
+    rotation of the experts' GEMM-2, and the blocks used are a rotation of all:
+    a line past the row may be one that another workgroup is still writing."""
+    src = tmp_path / "blocks.cpp"
+    src.write_text('''
+#include "ring_blocks.h"
+#include <cstdio>
+int main() {
+  for (int nb = 4; nb <= 512; nb += 2)
+    for (int q = 0; q < (nb % 4 == 0 ? 4 : 1); ++q)
+      for (int b = 0; b < nb + mep::ring::AHEAD; ++b) {
+        const int rot = q * (nb / 4), at = mep::ring::block_at(b, rot, nb);
+        if (at < 0 || at >= nb || (b < nb && at != (b + rot) % nb)) {
+          std::printf("nb %d rot %d load %d: block %d\\n", nb, rot, b, at);
+          return 1;
+        }
+      }
+}
+''')
+    exe = tmp_path / "blocks"
+    subprocess.run([shutil.which("g++") or "c++", "-std=c++17", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+    res = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
