@@ -112,8 +112,19 @@ struct GiveupTest {
 };
 GiveupTest giveup_test();
 
+// Workgroup barrier behind which every wave's global stores are complete, for
+// a count or a flag that tells other workgroups about them.  __syncthreads()
+// alone does not do that on gfx950: it leaves the stores in flight.
+constexpr int kVmcnt0 = 0x0F70;     // s_waitcnt vmcnt(0) alone
+__device__ __forceinline__ void store_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(kVmcnt0);
+  __syncthreads();
+}
+
 // End of a workgroup of a one-launch dispatch exchange, called by every lane
-// of wave 0 after a barrier that follows all of the workgroup's stores.  Lane
+// of wave 0 after a store_barrier() that follows all of the workgroup's stores
+// (a store that landed after the count could overwrite the poison).  Lane
 // 0 counts the workgroup finished in its group's word (groups of at least
 // kDoneGroup consecutive blocks, at most kMaxDoneGroups of them), a workgroup
 // that gave up with kGaveUpUnit on top; the group's last workgroup returns
@@ -127,7 +138,8 @@ GiveupTest giveup_test();
 // The chain of returned atomics is the end of the launch (0.6 to 0.8 us each):
 // one up to kDoneGroup workgroups, two beyond, none for a single one (with a
 // give-up word of its own it was three: router + dispatch of 100 tokens 10.7 ->
-// 9.7 us, of 2048 11.8 -> 11.0, of 16384 16.4 -> 16.0).
+// 10.1 us, of 2048 11.8 -> 11.3, of 16384 16.4 -> 16.3; 0.3 us of each is the
+// wait for the stores).
 constexpr int kExchangeLast = 1, kExchangeGaveUp = 2;
 constexpr int kDoneGroup = 32;
 constexpr uint32_t kGaveUpUnit = 1u << 16;   // far above a group's or the groups' number
@@ -171,10 +183,11 @@ inline int dtype_bytes(int dtype) {
 }
 
 // Workgroup barrier that orders LDS only: this wave's LDS reads and writes
-// complete (lgkmcnt(0)) before it arrives.  __syncthreads() also waits for
-// every outstanding global access (vmcnt(0)): for stores nobody waits for, and
-// for loads that a pipeline keeps in flight.  The empty asm statements keep
-// the compiler from moving memory accesses across.
+// complete (lgkmcnt(0)) before it arrives, whatever global accesses it has in
+// flight.  (__syncthreads() also has the workgroup-scope fences of the language.
+// They happen to cost no wait for global accesses on gfx950, where a
+// workgroup shares one L1, but nothing promises that.)  The empty asm
+// statements keep the compiler from moving memory accesses across.
 constexpr int kLgkmcnt0 = 0xC07F;   // s_waitcnt lgkmcnt(0) alone (vmcnt 63, expcnt 7)
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");

@@ -576,7 +576,8 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(DispatchParams p) {
   }
   }
   if (FUSED && tag_bad) atomicOr(&flag, tag_bad);
-  __syncthreads();
+  if constexpr (FUSED) store_barrier();            // row_of_entry and offsets, before finish_exchange
+  else __syncthreads();
   if (tid == 0) {
     p.flags[p.nbl + b] = flag;
     if constexpr (FUSED) p.flags[b] = cflag;

@@ -57,8 +57,6 @@ namespace mep {
 namespace {
 
 constexpr int kRowBytes = 128;   // K bytes per row per LDS stage
-// s_waitcnt immediate for "vmcnt(0)" alone (gfx9 encoding: expcnt and lgkmcnt at max)
-constexpr int kVmcnt0 = 0x0F70;
 
 template <int BM_, int BN_, int WM_, int WN_>
 struct TileCfg {
@@ -2279,9 +2277,9 @@ __device__ void decode_route(const DecodeParams& p, unsigned char* lds) {
     p.ws_flags[1] = 0u;
     p.ws_header[0] = 1u;
   }
-  // every wave's stores are in this XCD's L2; write them back to memory,
+  // every wave's stores have reached this XCD's L2; write them back to memory,
   // then publish the records (device scope: written through to memory)
-  __syncthreads();
+  store_barrier();
   if (wave == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     if (lane < E) {

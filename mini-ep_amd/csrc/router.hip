@@ -521,7 +521,7 @@ __global__ __launch_bounds__(kWaves * 64) void route_dispatch32_kernel(const uin
   if (nb > 1) {
     // the last workgroup to finish poisons a call in which one gave up, and
     // advances the epoch (every workgroup has read it)
-    __syncthreads();
+    store_barrier();
     if (tid < 64) {
       const int r = finish_exchange(o.header, gave_up, nb);
       if (r & kExchangeGaveUp) poison_dispatch(o.row_of_entry, n_tokens * KC, o.offsets, E);

@@ -6,7 +6,9 @@ summed routing counts of results/bench_naive.json at world 4 with 2 replica
 slots per rank (scripts/make_plan.py:24-29).
 """
 import ctypes
+import importlib.util
 import json
+import re
 import shutil
 import subprocess
 from pathlib import Path
@@ -230,3 +232,28 @@ int main() {
     subprocess.run([shutil.which("g++") or "c++", "-std=c++17", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
     res = subprocess.run([str(exe)], capture_output=True, text=True)
     assert res.returncode == 0, res.stdout
+
+
+@pytest.mark.parametrize("source,kernel,tells", [
+    # the atomic that counts a workgroup finished; the write-back in front of the routing records
+    ("router.hip", "route_dispatch32_kernelILi1E", r"global_atomic_add .* sc0"),
+    ("dispatch.hip", "scatter_kernelILb1E", r"global_atomic_add .* sc0"),
+    ("grouped_swiglu.hip", "moe_decode_kernelILi1E", r"buffer_wbl2 sc1"),
+])
+def test_stores_complete_before_other_workgroups_are_told(source, kernel, tells, tmp_path):
+    """A workgroup's stores are waited for (vmcnt(0)) by every wave in front of
+    the barrier behind which one wave tells other workgroups that they are made:
+    the compiler's own barrier leaves them in flight."""
+    spec = importlib.util.spec_from_file_location("miniep_amd_build", CSRC.parent / "build.py")
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    asm = tmp_path / "kernel.txt"
+    subprocess.run([build.hipcc(), *build.HIPCC_FLAGS, "-w", "--cuda-device-only", "-S", str(CSRC / source), "-o",
+                    str(asm)], check=True, capture_output=True)
+    text = asm.read_text()
+    body = re.search(rf"^_Z\S*{kernel}\S*:[^\n]*$(.*?)^\.Lfunc_end", text, re.M | re.S).group(1).splitlines()
+    code = [line.split(";")[0].strip() for line in body]
+    told = next(i for i, c in enumerate(code) if re.match(tells, c))
+    barrier = max(i for i in range(told) if code[i] == "s_barrier")
+    store = max(i for i in range(barrier) if re.match(r"(global|flat|buffer)_store", code[i]))
+    assert any(c.startswith("s_waitcnt") and "vmcnt(0)" in c for c in code[store:barrier]), code[store:told + 1]
