@@ -240,6 +240,8 @@ size_t mep_experts_queue_ints(int64_t max_rows, int32_t n_local);
  * MEP_OK, or MEP_ERR_HIP with the reason in mep_last_error(). */
 int mep_experts_check(const int32_t* tile_queue, void* stream);
 
+/* Bytes of `workspace`, 16-byte aligned like every buffer (act, which the
+ * one-launch kernels put on the first 128-byte boundary, and 256 bytes). */
 size_t mep_experts_workspace_size(int64_t max_rows, int32_t inter, int32_t dtype);
 
 int mep_grouped_swiglu(const void* x, int64_t n_tokens, int32_t top_k,

@@ -2856,6 +2856,16 @@ int check_expert_args(const char* fn, int64_t n_tokens, int top_k, int n_local, 
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+// act of a one-launch call: the first whole line of the workspace (which has
+// room for it: mep_experts_workspace_size is act and 256 bytes).  GEMM-2 reads
+// act with plain loads while other chunks' rows are still being written, so a
+// line must not hold rows of two chunks: it could be read, and kept in the CU's
+// L1, for one chunk before the other's part of it is final.  An act row is
+// whole lines long.
+void* act_lines(void* workspace) {
+  return reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(workspace) + 127) / 128 * 128);
+}
+
 }  // namespace
 }  // namespace mep
 
@@ -2937,6 +2947,7 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
   const size_t need = mep_experts_workspace_size(max_rows, inter, dtype);
   MEP_REQUIRE(workspace_bytes >= need, MEP_ERR_WORKSPACE, "%s: workspace %zu B < required %zu B", fn,
               workspace_bytes, need);
+  void* const act = act_lines(workspace);
   int mid_frags = 0;
   if (dtype == MEP_DTYPE_BF16 && inter % 256 == 0) mid_frags = mid_row_frags(max_rows, n_local, inter);
   // (fp32's two launches take any schedule buffer: a smaller one keeps them)
@@ -2951,8 +2962,8 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
     auto run = [&](auto dt) {
       constexpr int DT = decltype(dt)::value;
       GemmParams g1 = gemm1_params<DT, CfgBf16>(x, n_tokens, top_k, perm, offsets, n_local, w_in, w_slot, hidden, inter,
-                                                workspace);
-      GemmParams g2 = gemm2_params<DT, CfgBf16>(workspace, top_k, perm, offsets, n_local, max_rows, w_out, w_slot,
+                                                act);
+      GemmParams g2 = gemm2_params<DT, CfgBf16>(act, top_k, perm, offsets, n_local, max_rows, w_out, w_slot,
                                                 hidden, inter, y_entries);
       set_sched(g1, tile_queue);
       set_sched(g2, tile_queue);
@@ -2974,7 +2985,7 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
     MEP_REQUIRE(aligned16(x) && aligned16(w_in) && aligned16(w_out) && aligned16(workspace) && aligned16(y_entries),
                 MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
     const MoeParams p = moe_params(x, n_tokens, top_k, perm, offsets, n_local, max_rows, w_in, w_out, w_slot,
-                                   hidden, inter, workspace, y_entries, tile_queue);
+                                   hidden, inter, act, y_entries, tile_queue);
     const hipError_t e = launch_tiled<kModeBoth>(p, max_rows, static_cast<hipStream_t>(stream));
     MEP_REQUIRE(e == hipSuccess, MEP_ERR_HIP, "%s: %s", fn, hipGetErrorString(e));
     return MEP_OK;
@@ -2988,8 +2999,8 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
     MEP_REQUIRE(aligned16(x) && aligned16(w_in) && aligned16(w_out) && aligned16(workspace) && aligned16(y_entries),
                 MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
     GemmParams g1 = gemm1_params<MEP_DTYPE_BF16, CfgBf16>(x, n_tokens, top_k, perm, offsets, n_local, w_in, w_slot,
-                                                          hidden, inter, workspace);
-    GemmParams g2 = gemm2_params<MEP_DTYPE_BF16, CfgBf16>(workspace, top_k, perm, offsets, n_local, max_rows, w_out,
+                                                          hidden, inter, act);
+    GemmParams g2 = gemm2_params<MEP_DTYPE_BF16, CfgBf16>(act, top_k, perm, offsets, n_local, max_rows, w_out,
                                                           w_slot, hidden, inter, y_entries);
     set_sched(g1, tile_queue);
     set_sched(g2, tile_queue);
@@ -3218,8 +3229,8 @@ extern "C" int mep_moe_layer(const void* x, const void* w_router, const uint8_t*
                 MEP_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", fn);
     const hipError_t e = launch_decode(x, w_router, valid_mask, n_tokens, hidden, n_experts, top_k, dtype, w_in, w_out,
                                        inter, topk_idx, topk_gate, logits, counts, offsets, perm, row_of_entry,
-                                       route_counts, y_entries, dispatch_ws, experts_ws, tile_queue, tile_queue_ints,
-                                       out, static_cast<hipStream_t>(stream));
+                                       route_counts, y_entries, dispatch_ws, act_lines(experts_ws), tile_queue,
+                                       tile_queue_ints, out, static_cast<hipStream_t>(stream));
     if (e == hipSuccess) return MEP_OK;
     MEP_REQUIRE(e == hipErrorNotSupported, MEP_ERR_HIP, "%s: launch failed: %s", fn, hipGetErrorString(e));
   }

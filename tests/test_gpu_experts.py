@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from helpers import TOL_BF16, TOL_F32, banner, rel_err, to_np
-from miniep_amd import ops, workloads
+from miniep_amd import _lib, ops, workloads
 from oracle import moe_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -463,3 +463,63 @@ def test_decode_layer_graph_replay():
     ops.experts_check()
     for q in ops._QUEUES.values():
         assert int(q.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("n,k,I,dtype", [
+    (40, 1, 128, torch.float32), (40, 2, 256, torch.bfloat16), (320, 2, 256, torch.bfloat16),
+    (4000, 4, 512, torch.bfloat16)])
+def test_act_starts_on_a_line(n, k, I, dtype):
+    """A workspace off the 128-byte grid (each one-launch kernel: fp32, at most
+    256 rows, mid-size, tiled): act starts on the first whole line of it, so no
+    line holds rows of two chunks, nothing outside the workspace is written,
+    and the results are those of an aligned one."""
+    banner(f"experts, workspace at +16 bytes: {n} x {k} rows, I {I}, {dtype}")
+    E, H = 4, 256
+    g = torch.Generator().manual_seed(n)
+    topk = torch.rand(n, E, generator=g).topk(k, -1).indices
+    x = torch.randn(n, H, generator=g).to(dtype).to(DEV)
+    w_in, w_out = (w.to(dtype).to(DEV) for w in workloads.expert_weights(g, E, H, I))
+    table, n_rep, g2l = _world1(E)
+    d = ops.dispatch(topk.to(DEV), None, E, table, n_rep, False, None, 0, g2l, E)
+    want = ops.grouped_swiglu(x, d, w_in, w_out)
+    L = _lib.lib()
+    code = _lib.DTYPE_F32 if dtype == torch.float32 else _lib.DTYPE_BF16
+    need = L.mep_experts_workspace_size(n * k, I, code)
+    ws = torch.full((16 + need + 512,), 0xAB, dtype=torch.uint8, device=DEV)
+    assert ws.data_ptr() % 128 == 0
+    got = torch.empty_like(want)
+    tq = torch.zeros(L.mep_experts_queue_ints(n * k, E), dtype=torch.int32, device=DEV)
+    rc = L.mep_grouped_swiglu(x.data_ptr(), n, k, d.perm.data_ptr(), d.offsets.data_ptr(), E, n * k, w_in.data_ptr(),
+                              w_out.data_ptr(), H, I, code, got.data_ptr(), ws.data_ptr() + 16, need, tq.data_ptr(),
+                              tq.numel(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, L.mep_last_error()
+    assert torch.equal(got, want)
+    size = n * k * I * x.element_size()
+    assert bool((ws[:128] == 0xAB).all()) and bool((ws[128 + size:] == 0xAB).all())
+    assert bool((ws[128:128 + size].view(-1, 16) != 0xAB).any(1).all())
+
+
+def test_act_starts_on_a_line_decode_layer():
+    """The same for mep_moe_layer's one launch."""
+    banner("decode layer, workspace at +16 bytes")
+    n, E, k, H, I = 9, 32, 8, 1024, 256
+    g = torch.Generator().manual_seed(4)
+    x, w_r = (torch.randn(r, H, generator=g).bfloat16().to(DEV) for r in (n, E))
+    w_in, w_out = (w.bfloat16().to(DEV) for w in workloads.expert_weights(g, E, H, I))
+    want, idx, gate, d = ops.moe_layer(x, w_r, k, w_in, w_out)
+    L = _lib.lib()
+    need = L.mep_experts_workspace_size(n * k, I, _lib.DTYPE_BF16)
+    ws = torch.full((16 + need + 512,), 0xAB, dtype=torch.uint8, device=DEV)
+    dws = torch.zeros(L.mep_route_dispatch_workspace_size(n, E), dtype=torch.uint8, device=DEV)
+    tq = torch.zeros(L.mep_moe_layer_queue_ints(n, E, H), dtype=torch.int32, device=DEV)
+    y, out = torch.empty(n * k, H, dtype=x.dtype, device=DEV), torch.empty_like(want)
+    i32 = [torch.empty(s, dtype=torch.int32, device=DEV) for s in (E, E + 1, n * k, n * k)]
+    rc = L.mep_moe_layer(x.data_ptr(), w_r.data_ptr(), None, n, H, E, k, _lib.DTYPE_BF16, w_in.data_ptr(),
+                         w_out.data_ptr(), I, idx.data_ptr(), gate.data_ptr(), None, *(t.data_ptr() for t in i32), None,
+                         y.data_ptr(), dws.data_ptr(), dws.numel(), ws.data_ptr() + 16, need, tq.data_ptr(), tq.numel(),
+                         out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, L.mep_last_error()
+    assert torch.equal(out, want)
+    size = n * k * I * 2
+    assert bool((ws[:128] == 0xAB).all()) and bool((ws[128 + size:] == 0xAB).all())
+    assert bool((ws[128:128 + size].view(-1, 16) != 0xAB).any(1).all())
