@@ -181,6 +181,11 @@ __device__ __forceinline__ f32x4 load4(const typename Elem<DT>::T* src) {
   }
 }
 
+// What a running softmax subtracts from its scores: their maximum, 0 while every
+// score so far is -inf (an overflow, or -inf in a key), so that such keys weigh 0
+// once a finite score follows.  (-inf - -inf would be NaN for good.)
+__device__ __forceinline__ float finite_top(float m) { return m == -__builtin_inff() ? 0.0f : m; }
+
 // Keys (rotated) and values of the call's tokens into the cache: one thread
 // per 4 elements of a (token, kv head).
 template <int DT>
@@ -327,8 +332,9 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
         mb = fmaxf(mb, s[kt][i]);
       }
     mb = fmaxf(mb, __shfl_xor(mb, 16, 64));
-    mb = fmaxf(mb, __shfl_xor(mb, 32, 64));               // finite: key 0 is in the first block and seen by all
-    const float alpha = __builtin_amdgcn_exp2f(m - mb);
+    mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
+    const float top = finite_top(mb);
+    const float alpha = __builtin_amdgcn_exp2f(m - top);
     m = mb;
     l *= alpha;
 #pragma unroll
@@ -339,7 +345,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - m);
+        s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - top);
         l += s[kt][i];
       }
 #pragma unroll
@@ -485,12 +491,14 @@ __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnPa
       if (lane == 0) s_red[wave][h] = v;
     }
     lds_barrier();                                         // the values' loads stay in flight
+    float top[G];
 #pragma unroll
     for (int h = 0; h < G; ++h) {
       float v = s_red[0][h];
 #pragma unroll
       for (int w = 1; w < kDecWaves; ++w) v = fmaxf(v, s_red[w][h]);
-      const float alpha = __builtin_amdgcn_exp2f(m[h] - v);   // 0 in the first chunk
+      top[h] = finite_top(v);
+      const float alpha = __builtin_amdgcn_exp2f(m[h] - top[h]);   // 0 in the first chunk
       m[h] = mx[h] = v;
       l[h] *= alpha;
 #pragma unroll
@@ -505,7 +513,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnPa
         const f32x4 v = c0 + s == pos ? fresh[1] : vr[u];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-          const float e = __builtin_amdgcn_exp2f(s_p[h][s] - m[h]);
+          const float e = __builtin_amdgcn_exp2f(s_p[h][s] - top[h]);
           l[h] += e;
 #pragma unroll
           for (int i = 0; i < 4; ++i) o[h][i] += e * v[i];

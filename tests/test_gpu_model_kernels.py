@@ -75,6 +75,36 @@ def test_attention(B, T, start, hq, hk, dtype):
     assert float(err.max()) <= tol
 
 
+@pytest.mark.parametrize("T,dead", [(1, 2048), (1, 2100), (1, 3), (70, 64), (70, 130), (70, 1)])
+def test_attention_scores_of_minus_infinity(T, dead):
+    """Cached keys whose scores are -inf weigh 0, also where they fill the first
+    chunk (decode) or block (prefill) of keys."""
+    B, hq, hk, d, start = 2, 8, 4, 64, dead + 5
+    cfg = ModelConfig(num_attention_heads=hq, num_key_value_heads=hk, hidden_size=64 * hq)
+    rope = RotaryTable(cfg, DEV)
+    g = torch.Generator().manual_seed(dead + T)
+    q = torch.full((B * T, hq * d), 1.0, device=DEV)
+    k, v = (torch.randn(B * T, hk * d, generator=g).to(DEV) for _ in range(2))
+    cache = torch.randn(2, B, hk, start + T, d, generator=g).to(DEV)
+    pos = torch.arange(start, start + T, device=DEV)
+    # a dead key is 0 but for its element 63, where every rotated query is positive
+    turned = _rope64(q.double().view(B, T, hq, d).transpose(1, 2), rope, pos)
+    cache[0][:, :, :dead] = 0.0
+    cache[0][:, :, :dead, 63] = -torch.inf
+    assert bool((turned[..., 63] > 0).all())
+    out = ops.attention(q, k, v, rope.cos, rope.sin, B, start, cache[0].clone(), cache[1].clone(), 0.05)
+    kc, vc = cache[0].double(), cache[1].double()
+    kc[:, :, start:] = _rope64(k.double().view(B, T, hk, d).transpose(1, 2), rope, pos)
+    vc[:, :, start:] = v.double().view(B, T, hk, d).transpose(1, 2)
+    kk, vv = (t.repeat_interleave(hq // hk, 1) for t in (kc, vc))
+    s = (turned @ kk.transpose(2, 3).contiguous()) * 0.05
+    s = s.masked_fill(torch.arange(start + T, device=DEV) > pos[:, None], -torch.inf)
+    assert bool((s[..., :dead] == -torch.inf).all())
+    want = (torch.softmax(s, -1) @ vv).transpose(1, 2).reshape(B * T, hq * d)
+    tol = (64 * float(s[s.isfinite()].abs().max()) + (start + T) / 64 + 32) * 2.0 ** -24 * float(vv.abs().max())
+    assert float((out.double() - want).abs().max()) <= tol         # (NaN fails it)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_native_forward_equals_torch_statement(dtype):
     """Prefill, a decode step and a second chunk through one cache, and the
