@@ -21,7 +21,8 @@ is computed in fp32 for the positions asked for; router logits are fp32 (the
 router hook decides, see ``backend.route``).
 
 On the GPU a causal forward (no ``positions`` or ``attn_mask`` given) of a model
-with ``fuse_router`` (``build_hip_model``) runs the norms, residual adds, RoPE,
+with ``fuse_router`` (``build_hip_model``), its block, attention, rotation and
+cache write not overridden, runs the norms, residual adds, RoPE,
 cache writes and attention on the HIP kernels of ``ops`` (``add_norm``,
 ``attention``: head size 64, 1, 2 or 4 query heads per kv head, fp32 cache), and
 with at most 32 rows in bf16 the projections and the head (``attention_block``,
@@ -241,6 +242,11 @@ class GraniteMoeModel:
         cfg, e = self.cfg, self.embed
         if not self.fuse_router or positions is not None or attn_mask is not None:
             return False
+        # a program's own block, attention, rotation or cache write is called as ever
+        if not _own(self, "_block") or not _own(self, "_attention") or not _own(self.rope, "rotate"):
+            return False
+        if cache is not None and not _own(cache, "write"):
+            return False
         if not e.is_cuda or not input_ids.is_cuda:
             return False
         B, T = input_ids.shape
@@ -341,6 +347,17 @@ class GraniteMoeModel:
         return F.linear(h.float(), self._head) / self.cfg.logits_scaling
 
     __call__ = forward
+
+
+# the methods whose work the HIP kernels do
+_COVERED = {"_block": GraniteMoeModel._block, "_attention": GraniteMoeModel._attention,
+            "rotate": RotaryTable.rotate, "write": KVCache.write}
+
+
+def _own(obj, name: str) -> bool:
+    """Whether obj's method is the one of this file (not a subclass's, nor one set on the object or class)."""
+    m = getattr(obj, name, None)
+    return getattr(m, "__func__", None) is _COVERED[name] and m.__self__ is obj
 
 
 def greedy_generate(model: GraniteMoeModel, prompts: torch.Tensor, new_tokens: int,

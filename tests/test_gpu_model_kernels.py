@@ -5,7 +5,8 @@ import pytest
 import torch
 
 from miniep_amd import ops
-from miniep_amd.model import KVCache, ModelConfig, RotaryTable, build_hip_model, random_weights
+from miniep_amd.model import (GraniteMoeModel, KVCache, ModelConfig, RotaryTable, build_hip_model,
+                              random_weights)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -129,6 +130,43 @@ def test_native_forward_equals_torch_statement(dtype):
     at = torch.tensor([3, -1, 44], device=DEV)
     got, want = m(ids, logits_at=at), m(ids, logits_at=at, attn_mask=causal(45, 45))
     assert got.shape == (3, 1, cfg.vocab_size) and float((got - want).norm() / want.norm()) <= tol
+
+
+@pytest.mark.parametrize("what", ["KVCache.write", "RotaryTable.rotate", "_block", "_attention", "set on the object",
+                                  "set on the class"])
+def test_overridden_parts_are_called(what, monkeypatch):
+    """A program's own cache write, rotation, block or attention (a subclass's,
+    or one put in place of ours) is called for every layer of a prefill and of a
+    decode step, with the results of the native forward up to rounding."""
+    cfg = ModelConfig(num_hidden_layers=2, vocab_size=997)
+    m = build_hip_model(cfg, random_weights(cfg, seed=3, dtype=torch.bfloat16, device=DEV))
+    ids = torch.randint(0, cfg.vocab_size, (2, 41), generator=torch.Generator().manual_seed(1)).to(DEV)
+    plain = KVCache(cfg, 2, 50, DEV)
+    want = [m(ids[:, :40], cache=plain), m(ids[:, 40:], cache=plain)]
+    calls = []
+
+    def counted(fn):
+        def call(*a, **kw):
+            calls.append(fn)
+            return fn(*a, **kw)
+        return call
+
+    cache, per_layer = KVCache(cfg, 2, 50, DEV), 1
+    if what == "KVCache.write":
+        cache = type("Cache", (KVCache,), {"write": counted(KVCache.write)})(cfg, 2, 50, DEV)
+    elif what == "RotaryTable.rotate":
+        m.rope, per_layer = type("Rope", (RotaryTable,), {"rotate": counted(RotaryTable.rotate)})(cfg, DEV), 2
+    elif what == "set on the object":
+        cache.write = counted(cache.write)
+    elif what == "set on the class":
+        monkeypatch.setattr(KVCache, "write", counted(KVCache.write))
+    else:
+        m = type("Model", (GraniteMoeModel,), {what: counted(getattr(GraniteMoeModel, what))})(
+            cfg, m.w, m.router, m.moe, fuse_router=True)
+    got = [m(ids[:, :40], cache=cache), m(ids[:, 40:], cache=cache)]
+    assert len(calls) == 2 * cfg.num_hidden_layers * per_layer
+    for a, b in zip(got, want):
+        assert float((a - b).norm() / b.norm()) <= 2e-2
 
 
 def test_native_forward_with_unaligned_tensors():
