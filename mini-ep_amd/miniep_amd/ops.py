@@ -183,29 +183,20 @@ class Dispatch:
 
 
 _PARTS = {"counts": 0, "offsets": 1, "perm": 2, "row_of_entry": 3}
-
-
-def _part_ptr(disp: Dispatch, name: str) -> int:
-    t = disp.__dict__.get(name)
-    return disp.ptrs[_PARTS[name]] if t is None else t.data_ptr()
+# Largest block of index tensors in one allocation: what any one of them that
+# outlives the others keeps alive.  16 tokens to 2000 tokens top-8 are a few KiB
+# to this; above, a call is bound by the GPU and four allocations cost nothing.
+_PACKED_INTS = 32768
 
 
 class _PackedDispatch(Dispatch):
     """A Dispatch whose index tensors are parts of one allocation, made into
     tensors of their own when they are first asked for (a decode call asks for
-    none of them; four allocations are 5 us of host time)."""
+    none of them; four allocations are 5 us of host time).  Made by
+    _new_dispatch; its constructor, copies and pickles are a Dispatch's."""
 
-    def __init__(self, n_tokens: int, top_k: int, n_local: int, dev: torch.device, dest: torch.Tensor | None = None):
-        nk = max(n_tokens * top_k, 1)
-        size = [max(n_local, 1), n_local + 1, nk, nk]
-        start = [0]
-        for v in size:                                      # each part on a 256-byte boundary
-            start.append(start[-1] + (v + 63) // 64 * 64)
-        size[0] = n_local
-        buf = torch.empty(start[-1], dtype=torch.int32, device=dev)
-        base = buf.data_ptr()
-        self.__dict__.update(n_tokens=n_tokens, top_k=top_k, n_local=n_local, dest=dest, _buf=buf, _at=start,
-                             _size=size, ptrs=[base + 4 * v for v in start[:4]])   # counts, offsets, perm, row_of_entry
+    def part_ptr(self, part: int) -> int:
+        return self._buf.data_ptr() + 4 * self._at[part]
 
     def __getattr__(self, name):
         part = _PARTS.get(name)
@@ -214,6 +205,33 @@ class _PackedDispatch(Dispatch):
         t = self._buf[self._at[part]:self._at[part] + self._size[part]]
         self.__dict__[name] = t
         return t
+
+
+def _new_dispatch(n_tokens: int, top_k: int, n_local: int, dev: torch.device,
+                  dest: torch.Tensor | None = None) -> tuple[Dispatch, list[int]]:
+    """A Dispatch with uninitialised index tensors, and the addresses of its
+    counts, offsets, perm and row_of_entry."""
+    nk = max(n_tokens * top_k, 1)
+    size = [max(n_local, 1), n_local + 1, nk, nk]
+    at = [0]
+    for v in size:                                          # each part on a 256-byte boundary
+        at.append(at[-1] + (v + 63) // 64 * 64)
+    if at[-1] > _PACKED_INTS:
+        parts = [torch.empty(v, dtype=torch.int32, device=dev) for v in size]
+        return (Dispatch(parts[0][:n_local], *parts[1:], dest, n_tokens, top_k, n_local),
+                [t.data_ptr() for t in parts])
+    size[0] = n_local
+    buf = torch.empty(at[-1], dtype=torch.int32, device=dev)
+    d = _PackedDispatch.__new__(_PackedDispatch)
+    d.__dict__.update(n_tokens=n_tokens, top_k=top_k, n_local=n_local, dest=dest, _buf=buf, _at=at, _size=size)
+    base = buf.data_ptr()
+    return d, [base + 4 * v for v in at[:4]]
+
+
+def _part_ptr(disp: Dispatch, name: str) -> int:
+    if type(disp) is _PackedDispatch and name not in disp.__dict__:
+        return disp.part_ptr(_PARTS[name])
+    return getattr(disp, name).data_ptr()
 
 
 def dispatch(topk_idx: torch.Tensor, valid_mask: torch.Tensor | None, n_experts: int,
@@ -246,11 +264,11 @@ def dispatch(topk_idx: torch.Tensor, valid_mask: torch.Tensor | None, n_experts:
     ws = _dispatch_workspace(dev, int(L.mep_dispatch_workspace_size(n, k, n_experts, n_seg, seg_arr)))
     nk = max(n * k, 1)
     dest = torch.empty(nk, dtype=torch.int32, device=dev) if want_dest else None
-    d = _PackedDispatch(n, k, n_local, dev, dest)
+    d, parts = _new_dispatch(n, k, n_local, dev, dest)
     st = _stream(dev)
     rc = L.mep_dispatch(_ptr(idx), _ptr(vm), n, k, n_experts, table.data_ptr(), n_rep.data_ptr(),
                         table.shape[1], 1 if has_replicas else 0, _ptr(rr), seg_arr, n_seg,
-                        my_rank, g2l.data_ptr(), n_local, *d.ptrs, _ptr(dest), _ptr(route_counts),
+                        my_rank, g2l.data_ptr(), n_local, *parts, _ptr(dest), _ptr(route_counts),
                         ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "mep_dispatch")
     if check:
@@ -287,10 +305,10 @@ def route_dispatch(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, valid_m
     gate = torch.empty((n, k), dtype=x.dtype, device=dev)
     logits = torch.empty((n, e), dtype=torch.float32, device=dev) if return_logits else None
     ws = _dispatch_workspace(dev, int(L.mep_route_dispatch_workspace_size(n, e)))
-    d = _PackedDispatch(n, k, e, dev)
+    d, parts = _new_dispatch(n, k, e, dev)
     st = _stream(dev)
     rc = L.mep_route_dispatch(x.data_ptr(), w.data_ptr(), _ptr(vm), n, h, e, k, _dtype_code(x), idx.data_ptr(),
-                              gate.data_ptr(), _ptr(logits), *d.ptrs, _ptr(route_counts), ws.data_ptr(), ws.numel(), st)
+                              gate.data_ptr(), _ptr(logits), *parts, _ptr(route_counts), ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "mep_route_dispatch")
     if check:
         _lib.check(L.mep_dispatch_check(ws.data_ptr(), st), "mep_route_dispatch")
@@ -417,7 +435,7 @@ def moe_layer(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, w_in: torch.
     idx = torch.empty((n, k), dtype=torch.int64, device=dev)
     gate = torch.empty((n, k), dtype=x.dtype, device=dev)
     logits = torch.empty((n, e), dtype=torch.float32, device=dev) if return_logits else None
-    d = _PackedDispatch(n, k, e, dev)
+    d, parts = _new_dispatch(n, k, e, dev)
     out = torch.empty((n, h), dtype=x.dtype, device=dev)
     st = _stream(dev)
     dws = _dispatch_workspace(dev, int(L.mep_route_dispatch_workspace_size(n, e)))
@@ -433,7 +451,7 @@ def moe_layer(x_flat: torch.Tensor, w_router: torch.Tensor, k: int, w_in: torch.
     if tq is None or tq.numel() < need:
         tq = _QUEUES[key] = torch.zeros(max(need, 64), dtype=torch.int32, device=dev)
     rc = L.mep_moe_layer(x.data_ptr(), w.data_ptr(), _ptr(vm), n, h, e, k, code, wi.data_ptr(), wo.data_ptr(), inter,
-                         idx.data_ptr(), gate.data_ptr(), _ptr(logits), *d.ptrs, _ptr(route_counts), y, dws.data_ptr(),
+                         idx.data_ptr(), gate.data_ptr(), _ptr(logits), *parts, _ptr(route_counts), y, dws.data_ptr(),
                          dws.numel(), y + y_bytes, ews_bytes, tq.data_ptr(), tq.numel(), out.data_ptr(), st)
     _lib.check(rc, "mep_moe_layer")
     return (out, idx, gate, d) + ((logits,) if return_logits else ())

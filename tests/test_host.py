@@ -5,9 +5,12 @@ results/plan_balanced.json is the reference's plan_balanced() output for the
 summed routing counts of results/bench_naive.json at world 4 with 2 replica
 slots per rank (scripts/make_plan.py:24-29).
 """
+import copy
 import ctypes
+import dataclasses
 import importlib.util
 import json
+import pickle
 import re
 import shutil
 import subprocess
@@ -17,7 +20,7 @@ import numpy as np
 import pytest
 import torch
 
-from miniep_amd import Placement, _lib, plan_balanced
+from miniep_amd import Placement, _lib, ops, plan_balanced
 from oracle import moe_oracle as O
 
 
@@ -257,3 +260,32 @@ def test_stores_complete_before_other_workgroups_are_told(source, kernel, tells,
     barrier = max(i for i in range(told) if code[i] == "s_barrier")
     store = max(i for i in range(barrier) if re.match(r"(global|flat|buffer)_store", code[i]))
     assert any(c.startswith("s_waitcnt") and "vmcnt(0)" in c for c in code[store:barrier]), code[store:told + 1]
+
+
+@pytest.mark.parametrize("n,k,n_local", [(1, 8, 32), (0, 8, 32), (100, 8, 0), (1000, 8, 32), (2100, 8, 32), (16384, 8, 64)])
+def test_dispatch_is_an_ordinary_dataclass(n, k, n_local):
+    """A Dispatch as the calls make it, its index tensors in one allocation or
+    in four: replace, copies and pickles of it stand on their own (the addresses
+    that the launches get are those of their tensors), and an index tensor that
+    outlives the others keeps at most 128 KiB besides itself."""
+    d, parts = ops._new_dispatch(n, k, n_local, torch.device("cpu"))
+    nk = max(n * k, 1)
+    names = ["counts", "offsets", "perm", "row_of_entry"]
+    ptr = {m: ops._part_ptr(d, m) for m in names}                     # before a part is made into a tensor
+    assert list(ptr.values()) == parts and isinstance(d, ops.Dispatch)
+    made = [copy.deepcopy(d), pickle.loads(pickle.dumps(d)), copy.copy(d), dataclasses.replace(d, top_k=k)]
+    for m, v in zip(names, (n_local, n_local + 1, nk, nk)):
+        t = getattr(d, m)
+        assert t.shape == (v,) and t.dtype == torch.int32 and t.is_contiguous()
+        assert v == 0 or ops._part_ptr(d, m) == t.data_ptr() == ptr[m]
+        assert t.untyped_storage().nbytes() <= max(4 * max(v, 1), 128 << 10)
+        for e in made:
+            assert v == 0 or ops._part_ptr(e, m) == getattr(e, m).data_ptr()
+            assert torch.equal(getattr(e, m), t) and (e.n_tokens, e.top_k, e.max_rows) == (n, k, n * k)
+        for e in made[:2]:                                            # deep ones
+            assert v == 0 or getattr(e, m).data_ptr() != t.data_ptr()
+    other = torch.arange(nk, dtype=torch.int32)
+    e = dataclasses.replace(d, perm=other, dest=other)
+    assert e.perm is other and e.dest is other and ops._part_ptr(e, "perm") == other.data_ptr() and d.dest is None
+    d.offsets = torch.zeros(n_local + 1, dtype=torch.int32)
+    assert ops._part_ptr(d, "offsets") == d.offsets.data_ptr()
