@@ -181,10 +181,10 @@ __device__ __forceinline__ f32x4 load4(const typename Elem<DT>::T* src) {
   }
 }
 
-// What a running softmax subtracts from its scores: their maximum, 0 while every
-// score so far is -inf (an overflow, or -inf in a key), so that such keys weigh 0
-// once a finite score follows.  (-inf - -inf would be NaN for good.)
-__device__ __forceinline__ float finite_top(float m) { return m == -__builtin_inff() ? 0.0f : m; }
+// Start of a running softmax's maximum: finite, so that keys whose scores are
+// -inf (an overflow, or -inf in a key) weigh 0 also while no other score has been
+// seen (-inf - -inf would be NaN for good).
+constexpr float kLowest = -3.402823466e38f;
 
 // Keys (rotated) and values of the call's tokens into the cache: one thread
 // per 4 elements of a (token, kv head).
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
     }
   };
   const int k_end = min(S, p.start + q0 + kFlashQ);       // keys the workgroup's last query sees
-  float m = -__builtin_inff(), l = 0.0f;
+  float m = kLowest, l = 0.0f;
   f32x4 o[4];
 #pragma unroll
   for (int d = 0; d < 4; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -333,8 +333,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
       }
     mb = fmaxf(mb, __shfl_xor(mb, 16, 64));
     mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
-    const float top = finite_top(mb);
-    const float alpha = __builtin_amdgcn_exp2f(m - top);
+    const float alpha = __builtin_amdgcn_exp2f(m - mb);
     m = mb;
     l *= alpha;
 #pragma unroll
@@ -345,7 +344,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - top);
+        s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - m);
         l += s[kt][i];
       }
 #pragma unroll
@@ -452,7 +451,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnPa
   f32x4 o[G];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
-    m[h] = mx[h] = -__builtin_inff();
+    m[h] = mx[h] = kLowest;
     l[h] = 0.0f;
     o[h] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -491,14 +490,12 @@ __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnPa
       if (lane == 0) s_red[wave][h] = v;
     }
     lds_barrier();                                         // the values' loads stay in flight
-    float top[G];
 #pragma unroll
     for (int h = 0; h < G; ++h) {
       float v = s_red[0][h];
 #pragma unroll
       for (int w = 1; w < kDecWaves; ++w) v = fmaxf(v, s_red[w][h]);
-      top[h] = finite_top(v);
-      const float alpha = __builtin_amdgcn_exp2f(m[h] - top[h]);   // 0 in the first chunk
+      const float alpha = __builtin_amdgcn_exp2f(m[h] - v);   // (in the first chunk l and o are 0)
       m[h] = mx[h] = v;
       l[h] *= alpha;
 #pragma unroll
@@ -513,7 +510,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void attention_decode_kernel(AttnPa
         const f32x4 v = c0 + s == pos ? fresh[1] : vr[u];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-          const float e = __builtin_amdgcn_exp2f(s_p[h][s] - top[h]);
+          const float e = __builtin_amdgcn_exp2f(s_p[h][s] - m[h]);
           l[h] += e;
 #pragma unroll
           for (int i = 0; i < 4; ++i) o[h][i] += e * v[i];
