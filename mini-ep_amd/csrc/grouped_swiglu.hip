@@ -2726,25 +2726,37 @@ bool tiled_down(int dtype, int64_t max_rows, int inter) {
 //  - at most 256 rows: the small-batch launch, which may end with the combine
 //    (32 tokens: 26 with it, 23 + 4 without);
 //  - the tiled kernel where its row tiles are mostly full and its GEMM-1 tiles
-//    fill whole rounds of the CUs: 1500 tokens 67 against 72, 4096 tokens 116
-//    against 143, 2500 tokens 98 against 103;
+//    fill whole rounds of the CUs: 1500 tokens flat 58 against 64, 4096 tokens
+//    132 against 148, 2500 tokens 95 against 98;
 //  - this one below (64 tokens 27 -> 23, 128: 43 -> 24, 256: 57 -> 29, 517:
-//    52 -> 36, 1024: 60 -> 48), where an expert's rows fill at most half a
-//    row tile (hidden 2048, 64 experts, 500 tokens: 216 -> 195), and where the
-//    tiled launch's second round would be nearly empty (2048 tokens: 92 -> 82).
-int mid_row_frags(int64_t max_rows, int n_local, int inter) {
+//    52 -> 36, 1024: 60 -> 54; 8 experts, 5500 rows of top-2: 51.1 -> 50.7),
+//    where an expert's rows fill at most half a row tile (hidden 2048, 64
+//    experts, 500 tokens: 216 -> 195, 1000: 240 -> 230), and where the tiled
+//    launch begins a second round and this one still ends sooner, which is
+//    decided by the chunks (a hot expert's row tiles are full, so tiles alone
+//    say too little).  us against chunks of 128 rows x 128 act columns, two a
+//    CU counting 1.0: hidden 1024: 1.01 78 -> 69 (8 experts), 1.13 95 -> 83
+//    (2048 tokens), 1.13 79.6 -> 77.6, 1.19 78.7 -> 79.2, 1.25 78.6 -> 83.3;
+//    hidden 512: 1.13 53 -> 51, 1.25 53.5 -> 54.3; hidden 2048: 0.93 158 -> 135
+//    (32 experts), 0.94 144 -> 131, 1.04 150 -> 143 and 125 -> 134 (intermediate
+//    1024), 1.09 148 -> 152.  A longer K takes more of the ring's LDS time and
+//    less of the tiles' fixed one; at hidden 4096 that moves the first line too
+//    (0.59 of a round of tiles 153 -> 147, 0.72 165 -> 174, 1.09 241 -> 263).
+int mid_row_frags(int64_t max_rows, int n_local, int hidden, int inter) {
   if (max_rows <= 256) return 0;
   const int64_t cu = device_cu_count();
   // row tiles and chunks: an expert's last one is half empty on average
   const int64_t tiles = (max_rows / bfk::BM + n_local / 2) * (inter / (bfk::BN / 2));
+  const int64_t blocks = (max_rows / 128 + n_local / 2) * (inter / 128);
   const bool sparse = max_rows <= static_cast<int64_t>(n_local) * (bfk::BM / 2);
-  if (!sparse && tiles * 4 > cu * 3 && !(tiles > cu && tiles * 20 <= cu * 27)) return 0;
+  const bool part = tiles * 20 <= cu * (hidden <= 2048 ? 15 : 12);      // of a round
+  const bool spill = tiles > cu && blocks * 10 <= cu * (hidden <= 1024 ? 23 : hidden <= 2048 ? 19 : 0);
+  if (!sparse && !part && !spill) return 0;
   // chunks of 128 rows read the weights half as often as chunks of 64, if the
   // experts have that many rows and the chip is still full (128 tokens: even;
   // 384 tokens: 34 -> 30; 517: skewed routing 49 -> 42, flat 42 -> 43; 700: 47 ->
   // 42; 10 experts with 120 rows each: 19 with 64, 25 with 128)
-  const int64_t units = (max_rows / 128 + n_local / 2) * (inter / 64);
-  return max_rows >= static_cast<int64_t>(n_local) * 64 && units * 4 >= cu * (sparse ? 4 : 6) ? 8 : 4;
+  return max_rows >= static_cast<int64_t>(n_local) * 64 && blocks * 4 >= cu * (sparse ? 2 : 3) ? 8 : 4;
 }
 
 // fp32, every size: chunks of 64 rows, or of 32 while those of 64 are too few
@@ -2752,7 +2764,10 @@ int mid_row_frags(int64_t max_rows, int n_local, int inter) {
 // padding rows cost more than reading the weights again).  us of one call
 // against the two launches of 128 x 128 tiles, GraniteMoE's experts: 1 token
 // 109 -> 40, 32: 116 -> 53, 128: 114 -> 70 (64-row chunks: 107), 256: 217 ->
-// 91, 512: 216 -> 140, 1500: 424 -> 325 (32-row chunks: 350), 4096: 946 -> 802.
+// 91, 512: 216 -> 140, 1500: 423 -> 314 (32-row chunks: 339), 4096: 942 -> 792,
+// 8192: 1783 -> 1561, 16384: 3450 -> 3083; 8 experts, 32768 rows: 940 -> 770;
+// hidden 2048, 64 experts: 100 tokens 813 -> 313, 4096: 3859 -> 3313; hidden 512,
+// 16 experts, 65536 rows: 500 -> 402.
 int mid_row_frags_f32(int64_t max_rows, int n_local, int inter) {
   const int64_t units = (max_rows / 64 + n_local / 2) * (inter / 64);
   return units >= 2 * device_cu_count() ? 4 : 2;
@@ -2949,7 +2964,7 @@ int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k,
               workspace_bytes, need);
   void* const act = act_lines(workspace);
   int mid_frags = 0;
-  if (dtype == MEP_DTYPE_BF16 && inter % 256 == 0) mid_frags = mid_row_frags(max_rows, n_local, inter);
+  if (dtype == MEP_DTYPE_BF16 && inter % 256 == 0) mid_frags = mid_row_frags(max_rows, n_local, hidden, inter);
   // (fp32's two launches take any schedule buffer: a smaller one keeps them)
   else if (dtype == MEP_DTYPE_F32 && static_cast<int64_t>(tile_queue_ints) >= sched::words(max_rows, n_local))
     mid_frags = mid_row_frags_f32(max_rows, n_local, inter);

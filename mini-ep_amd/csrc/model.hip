@@ -837,10 +837,11 @@ __global__ __launch_bounds__(ring::NT, 2) void linear_tile_kernel(LinearTilePara
 }
 
 // Tiles of 128 rows read x and W through LDS less often, tiles of 64 rows are
-// taken while they fit the chip at once (us, hidden 1024, q + k + v of 2048
-// columns, before the writes were spread over the MFMA groups: 1024 rows 11.4
-// against 14.7 with 128, 2048 rows 16.5 against 16.0, 4096 rows 27.8 against
-// 24.3).
+// taken while they fit the chip at once (us, 64 against 128 rows a tile, by
+// tiles of 64 per CU; hidden 1024, q + k + v of 2048 columns: 1.0 10.3 against
+// 13.0, 1.12 14.5 against 13.2, 2.0 15.6 against 14.9, 4.0 27.5 against 23.3;
+// hidden 2048, 3072 columns: 0.75 18.0 against 21.4, 1.12 25.5 against 22.1; hidden
+// 512, 1024 columns: 1.0 7.0 against 8.8, 1.47 9.7 against 9.1).
 hipError_t launch_linear_tile(const LinearTileParams& p, hipStream_t stream) {
   auto go = [&](auto mfc) {
     constexpr int MFC = decltype(mfc)::value;
