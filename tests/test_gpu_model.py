@@ -19,7 +19,11 @@ teacher-forced decisions: its logits are about 0.5 in size, top-2 gaps about
 0.02, and the step's logit error about 0.1.)
 
 fp32: the HIP fp32 kernels against the fp32 restatement; the 8 x 32
-continuations must be identical.
+continuations must be identical.  With the HIP model's routing replayed into
+the reference every step's logits agree to the order of fp32 sums (3.1e-6 on
+a scale of 0.55), and a routing that the reference would have decided
+otherwise (2 of 104256; such a token's logits then differ by up to 2.2e-1) is
+a tie within the two models' difference of the router's logits.
 
 bf16: the two paths legitimately round differently (one bf16 ulp in some
 expert outputs: their fp32 sums run in different orders), and a random
@@ -84,9 +88,48 @@ def _sensitivity(ref, prompts, ref_free):
     return int((ptoks != ref_free).sum())
 
 
+class _Recorded:
+    """A HIP backend that keeps, call by call, its routing and the router logits
+    of its input (fp32, torch)."""
+
+    def __init__(self, inner, log):
+        self.inner, self.log = inner, log
+
+    def route_and_call(self, x_flat, w_router, k, valid_mask=None):
+        out, idx, gate = self.inner.route_and_call(x_flat, w_router, k, valid_mask)
+        self.log.append((idx, gate, x_flat.float() @ w_router.float().T))
+        return out, idx, gate
+
+
+class _CheckedReplay:
+    """Router that returns the recorded routing in order and compares it with
+    its own logits: the largest difference of the two models' router logits, and
+    of each decision that its own logits would have made otherwise, the gap
+    between the best logit left out and the worst one taken, and the difference
+    of the token's logits in the two models."""
+
+    def __init__(self, log):
+        self.log, self.i, self.err, self.scale, self.flips = log, 0, 0.0, 0.0, []
+
+    def __call__(self, x_flat, w_router, k):
+        idx, gate, theirs = self.log[self.i]
+        self.i += 1
+        own = x_flat.float() @ w_router.float().T
+        err = (own - theirs).abs().amax(-1)
+        self.err, self.scale = max(self.err, float(err.max())), max(self.scale, float(own.abs().max()))
+        taken = own.gather(1, idx).amin(-1)
+        left = own.scatter(1, idx, -torch.inf).amax(-1)
+        flip = left > taken
+        if bool(flip.any()):
+            self.flips += list(zip((left - taken)[flip].tolist(), err[flip].tolist()))
+        return idx, gate
+
+
 def test_config3_fp32_greedy_identity():
     banner("config 3 fp32: 24 layers, prefill 8x512, 32 greedy steps, identity")
     cfg, w, hip, ref, prompts = _setup(torch.float32)
+    log = []
+    hip.moe = [_Recorded(be, log) for be in hip.moe]
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     toks, _, hip_logits = greedy_generate(hip, prompts, 32, return_logits=True)
@@ -96,6 +139,12 @@ def test_config3_fp32_greedy_identity():
     # the same steps teacher-forced on the HIP tokens: the logit error of the fp32 path
     _, _, ref_logits = greedy_generate(ref, prompts, 32, forced=toks, return_logits=True)
     err = (hip_logits - ref_logits).abs().amax(-1)
+    # ... and with the HIP model's routing replayed: no choice of experts can fall the other way
+    replay = _CheckedReplay(log)
+    forced_ref = GraniteMoeModel(cfg, w, replay, ref.moe)
+    _, _, fr_logits = greedy_generate(forced_ref, prompts, 32, forced=toks, return_logits=True)
+    assert replay.i == len(log) == 32 * cfg.num_hidden_layers
+    ferr = (hip_logits - fr_logits).abs().amax(-1)
     # the reference's gate B fingerprint (worker.py:165-173,189-191): the first
     # LOGIT_FP_SIZE = 64 logits of the last prefill position, max abs diff
     # below GATE_LOGIT_TOL = 2e-3 (miniep/__init__.py:4-6); here also over the
@@ -110,7 +159,19 @@ def test_config3_fp32_greedy_identity():
           f"smallest reference top-2 gap {float(rmargins.min()):.3e}; layer-12 MoE x0.9 moves "
           f"{moved}/{toks.numel()}", flush=True)
     print("  per step, max over sequences: " + " ".join(f"{v:.1e}" for v in err.amax(0).tolist()), flush=True)
+    print("  with the HIP routing replayed: " + " ".join(f"{v:.1e}" for v in ferr.amax(0).tolist()), flush=True)
+    print(f"  logit scale {float(ref_logits.abs().max()):.2f}; router logits of the two models differ by {replay.err:.2e} "
+          f"at most; {len(replay.flips)} of {sum(len(i) for i, _, _ in log)} routings fall the other way: "
+          + ", ".join(f"gap {a:.1e} (logits differ by {b:.1e})" for a, b in replay.flips[:8]), flush=True)
     assert moved > toks.numel() // 5, "the decoded tokens do not depend on the MoE blocks"
+    # two models with the same routing differ by the order of their fp32 sums: 24 layers of two sums each into
+    # the residual stream, of at most 1024 products (about sqrt(1024) roundings each), relative to the scale
+    order = 24 * 2 * 32 * 2.0 ** -24
+    assert float(ferr.max()) <= order * float(fr_logits.abs().max()), "a step's logits differ with the routing replayed"
+    assert replay.err <= order * replay.scale
+    # a routing that falls the other way does so at a tie: the gap is within the logits' difference at that token
+    # (both sides of it, and the router kernel's own sum)
+    assert all(gap <= 2 * diff + 2 * 32 * 2.0 ** -24 * replay.scale for gap, diff in replay.flips)
     assert fp_diff < GATE_LOGIT_TOL and prefill_diff < GATE_LOGIT_TOL, "prefill logits beyond the gate tolerance"
     assert torch.equal(toks, rtoks), "fp32 greedy continuations differ from the reference"
 
