@@ -106,6 +106,17 @@ def test_attention_scores_of_minus_infinity(T, dead):
     assert float((out.double() - want).abs().max()) <= tol         # (NaN fails it)
 
 
+def _count_native(m):
+    """The calls of m's forward on the HIP kernels, appended as they are made."""
+    calls, inner = [], m._forward_native
+
+    def forward(*a, **kw):
+        calls.append(a[0].shape)
+        return inner(*a, **kw)
+    m._forward_native = forward
+    return calls
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_native_forward_equals_torch_statement(dtype):
     """Prefill, a decode step and a second chunk through one cache, and the
@@ -121,14 +132,17 @@ def test_native_forward_equals_torch_statement(dtype):
         return torch.arange(s, device=DEV) <= torch.arange(s - t, s, device=DEV)[:, None]
 
     tol = 2e-2 if dtype == torch.bfloat16 else 2e-5
+    native = _count_native(m)
     a, b = (KVCache(cfg, 3, 50, DEV) for _ in range(2))
     for lo, hi in ((0, 30), (30, 31), (31, 45)):
         got = m(ids[:, lo:hi], cache=a)
         want = m(ids[:, lo:hi], cache=b, attn_mask=causal(hi - lo, hi))
         assert a.length == b.length == hi and got.shape == want.shape
+        assert native.pop() == (3, hi - lo) and not native           # the first call ran on them, the second did not
         assert float((got - want).norm() / want.norm()) <= tol
     at = torch.tensor([3, -1, 44], device=DEV)
     got, want = m(ids, logits_at=at), m(ids, logits_at=at, attn_mask=causal(45, 45))
+    assert native == [(3, 45)]
     assert got.shape == (3, 1, cfg.vocab_size) and float((got - want).norm() / want.norm()) <= tol
 
 
@@ -163,8 +177,9 @@ def test_overridden_parts_are_called(what, monkeypatch):
     else:
         m = type("Model", (GraniteMoeModel,), {what: counted(getattr(GraniteMoeModel, what))})(
             cfg, m.w, m.router, m.moe, fuse_router=True)
+    native = _count_native(m)
     got = [m(ids[:, :40], cache=cache), m(ids[:, 40:], cache=cache)]
-    assert len(calls) == 2 * cfg.num_hidden_layers * per_layer
+    assert not native and len(calls) == 2 * cfg.num_hidden_layers * per_layer
     for a, b in zip(got, want):
         assert float((a - b).norm() / b.norm()) <= 2e-2
 
@@ -183,12 +198,14 @@ def test_native_forward_with_unaligned_tensors():
         flat[1:] = t.reshape(-1)
         return flat[1:].view(t.shape)
 
+    native = _count_native(m)
     cache = KVCache(cfg, 2, 40, DEV)
     cache.k = [off_grid(t) for t in cache.k]
     assert float((m(ids, cache=cache) - want).norm() / want.norm()) <= 2e-2
+    assert not native
     inner = m.moe[0].route_and_call
     m.moe[0].route_and_call = lambda *a, **kw: (off_grid(inner(*a, **kw)[0]),)
-    assert torch.equal(m(ids), want)
+    assert torch.equal(m(ids), want) and native == [(2, 40)]
 
 
 def _norm64(h, w):
