@@ -127,6 +127,7 @@ class HipEPShareBackend:
         self.stats = stats
         self.check = check
         self.w_slot = None
+        self._const: dict = {}
         if store is not None:
             self.use_store(placement, store)
         else:
@@ -145,11 +146,21 @@ class HipEPShareBackend:
         for i, e in enumerate(local_experts):
             g2l[e] = i
         self.g2l = g2l.to(self.w_in.device)
-        # constant tables of the send and receive halves, laid out with the placement
-        dev, E = self.w_in.device, self.placement.num_experts
-        self._nobody = torch.full((E,), -1, dtype=torch.int32, device=dev)
-        self._by_rank = _world1_tables(self.placement.world, dev)
-        self._by_expert = _world1_tables(E, dev)
+        # laid out with the placement, so that a captured call makes none
+        self._constants(self.placement.world)
+        self._constants(self.placement.num_experts)
+
+    def _constants(self, size: int):
+        """(table, n_rep, identity, nobody) for `size` keys, all on rank 0 (or, by
+        `nobody`, resident nowhere).  Copied from the host, so they are complete
+        for every stream that a call may run on, and, being constant, kept as
+        long as this backend whatever the placement."""
+        dev = self.w_in.device
+        t = self._const.get((size, dev))
+        if t is None:
+            nobody = torch.full((size,), -1, dtype=torch.int32)
+            t = self._const[size, dev] = tuple(v.to(dev) for v in (*_world1_tables(size, "cpu"), nobody))
+        return t
 
     def apply_placement(self, placement: Placement, w_in: torch.Tensor, w_out: torch.Tensor):
         """Swap in a new placement and this rank's re-sliced weights
@@ -203,10 +214,10 @@ class HipEPShareBackend:
             rr = torch.zeros(1, E, dtype=torch.long, device=dev)
         rc = self.stats.route_counts[self.layer] if self.stats is not None else None
         d = ops.dispatch(topk_idx, valid_mask, E, table, n_rep, has_rep, rr if has_rep else None, -1,
-                         self._nobody, 0, route_counts=rc, want_dest=True, check=self.check)
+                         self._constants(E)[3], 0, route_counts=rc, want_dest=True, check=self.check)
         # the destination-sorted order is the dispatch itself keyed by destination
         key = d.dest[: n * k].clamp(min=0).view(n, k).to(torch.int64)   # masked entries stay masked
-        t1, r1, ident = self._by_rank if self._by_rank[0].shape[0] == world else _world1_tables(world, dev)
+        t1, r1, ident, _ = self._constants(world)
         srt = ops.dispatch(key, valid_mask, world, t1, r1, False, None, 0, ident, world, check=False)
         m = int(srt.offsets[-1])
         send_x, send_ids = ops.gather_rows(x_flat.to(self.w_in.dtype), srt.perm, m, k, topk_idx)
@@ -221,7 +232,7 @@ class HipEPShareBackend:
         if n == 0:
             return torch.empty(0, recv_x.shape[1], dtype=self.w_in.dtype, device=dev)
         E = self.placement.num_experts
-        t1, r1, _ = self._by_expert
+        t1, r1, _, _ = self._constants(E)
         d = ops.dispatch(recv_experts.view(n, 1), None, E, t1, r1, False, None, 0, self.g2l,
                          len(self.local_experts), check=self.check)
         if self.stats is not None:

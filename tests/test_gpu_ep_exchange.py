@@ -114,3 +114,37 @@ def test_gather_rows_and_combine_rows_direct():
     a = ops.combine_rows(y[order.to(DEV)], gate, inv_p)
     b = ops.combine(y, gate, present.to(DEV))
     assert torch.equal(a, b)
+
+
+def test_send_and_receive_on_another_stream():
+    """A backend made (and given another placement) on one stream, behind work
+    that is still running there, and called on another at once: its tables are
+    complete, and those of the placement before stay while a call uses them."""
+    banner("ep backend made on one stream, called on another")
+    L = workloads.make_layer(512, seed=12, zipf_s=1.1)
+    x, wi, wo = (t.bfloat16().to(DEV) for t in (L.x, L.w_in, L.w_out))
+    idx, _ = route(x, L.w_router.bfloat16().to(DEV), 8)
+    naive, other = (Placement([[[(e // 8 + shift) % 4] for e in range(32)]], device=DEV) for shift in (0, 1))
+    for p in (naive, other):
+        p.tables(0, DEV + ":0")
+    weights = [(wi[m].contiguous(), wo[m].contiguous()) for m in (p.experts_of_rank(1)[0] for p in (naive, other))]
+
+    def steps(be):
+        sent = be.send(x, idx)
+        mine = sent.experts.new_tensor(be.local_experts)
+        y = be.receive(sent.x[: len(mine) * 8], mine.repeat(8))
+        return sent.x, sent.experts, sent.send_counts, sent.inv, y
+
+    want = [steps(HipEPShareBackend(0, p, 1, *w)) for p, w in zip((naive, other), weights)]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)                                   # some ms of the first stream's time
+    be = HipEPShareBackend(0, naive, 1, *weights[0])
+    with torch.cuda.stream(side):
+        got = [steps(be)]
+    be.apply_placement(other, *weights[1])
+    with torch.cuda.stream(side):
+        got.append(steps(be))
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert all(torch.equal(s, t) for s, t in zip(a, b))
