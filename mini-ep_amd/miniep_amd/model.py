@@ -242,6 +242,8 @@ class GraniteMoeModel:
         cfg, e = self.cfg, self.embed
         if not self.fuse_router or positions is not None or attn_mask is not None:
             return False
+        if torch.is_autocast_enabled("cuda"):
+            return False
         # a program's own block, attention, rotation or cache write is called as ever
         if not _own(self, "_block") or not _own(self, "_attention") or not _own(self.rope, "rotate"):
             return False

@@ -184,6 +184,19 @@ def test_overridden_parts_are_called(what, monkeypatch):
         assert float((a - b).norm() / b.norm()) <= 2e-2
 
 
+def test_forward_under_autocast():
+    """An fp32 model under autocast, whose products are then bf16: accepted, the
+    result that of the torch statement."""
+    cfg = ModelConfig(num_hidden_layers=2, vocab_size=997)
+    m = build_hip_model(cfg, random_weights(cfg, seed=3, dtype=torch.float32, device=DEV))
+    ids = torch.randint(0, cfg.vocab_size, (2, 40), generator=torch.Generator().manual_seed(1)).to(DEV)
+    mask = torch.arange(40, device=DEV) <= torch.arange(40, device=DEV)[:, None]
+    native = _count_native(m)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        got, want = m(ids), m(ids, attn_mask=mask)
+    assert torch.equal(got, want) and not native
+
+
 def test_native_forward_with_unaligned_tensors():
     """A backend that returns a view off the 16-byte grid, and such a cache:
     accepted, with the results of aligned ones (the cache goes through the torch
