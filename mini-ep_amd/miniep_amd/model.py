@@ -304,15 +304,17 @@ class GraniteMoeModel:
                 q, k, v = ops.linear(x, proj) if ops.tiled_linear(x, proj) else (F.linear(x, m) for m in proj)
                 o = ops.attention(q, k, v, cos, sin, B, start, kc, vc, scale)
                 h, x = ops.add_norm(h, norm2, eps, F.linear(o, w[k_["wo"]]), rm)
-            moe_out = self._moe_block(layer, x, moe_valid).contiguous()
+            moe_out = self._moe_block(layer, x, moe_valid).view(n, H).contiguous()
             if moe_out.data_ptr() % 16:                              # a backend's view into something larger
                 moe_out = moe_out.clone()
+            if moe_out.dtype != h.dtype:                             # a backend of another dtype: the sum is promoted
+                h, moe_out = h + moe_out * rm, None
         if logits_at is not None:
             at = (torch.arange(B, device=h.device), logits_at)
             h, moe_out = (None if z is None else z.view(B, T, H)[at] for z in (h, moe_out))
         norm = w["model.norm.weight"]
-        if moe_out is not None and moe_out.dtype != h.dtype:      # a last backend of another dtype
-            return self._logits(rms_norm(h + moe_out * rm, norm, eps).view(B, -1, H))
+        if h.dtype != norm.dtype:                                    # promoted by the last layer's backend
+            return self._logits(rms_norm(h, norm, eps).view(B, -1, H))
         if ops.small_rows(h.shape[0], H, h.dtype):
             logits = ops.norm_head(h, moe_out, rm, norm, eps, self.embed, cfg.logits_scaling)
             return logits.view(B, -1, self.embed.shape[0])

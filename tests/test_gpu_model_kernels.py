@@ -4,7 +4,7 @@ statement."""
 import pytest
 import torch
 
-from miniep_amd import ops
+from miniep_amd import HipMoEBackend, ops
 from miniep_amd.model import (GraniteMoeModel, KVCache, ModelConfig, RotaryTable, build_hip_model,
                               random_weights)
 
@@ -195,6 +195,30 @@ def test_forward_under_autocast():
     with torch.autocast("cuda", dtype=torch.bfloat16):
         got, want = m(ids), m(ids, attn_mask=mask)
     assert torch.equal(got, want) and not native
+
+
+@pytest.mark.parametrize("model,backend,layers", [(torch.float32, torch.bfloat16, (0, 1)),
+                                                  (torch.float32, torch.bfloat16, (0,)), (torch.bfloat16, torch.float32, (1,))])
+def test_backends_of_another_dtype_and_shape(model, backend, layers):
+    """Backends whose experts (and output) are of another dtype than the model,
+    in the last layer only where the sum outgrows the weights' dtype, and one
+    that returns (batch, tokens, hidden): as the torch statement has them."""
+    cfg = ModelConfig(num_hidden_layers=2, vocab_size=997)
+    w = random_weights(cfg, seed=3, dtype=model, device=DEV)
+    m = build_hip_model(cfg, w)
+    for i in layers:
+        be = m.moe[i]
+        m.moe[i] = HipMoEBackend(be.w_in.to(backend), be.w_out.to(backend))
+    inner = m.moe[1].route_and_call
+    m.moe[1].route_and_call = lambda *a, **kw: (inner(*a, **kw)[0].view(2, -1, cfg.hidden_size),)
+    ids = torch.randint(0, cfg.vocab_size, (2, 41), generator=torch.Generator().manual_seed(1)).to(DEV)
+    native = _count_native(m)
+    a, b = KVCache(cfg, 2, 50, DEV), KVCache(cfg, 2, 50, DEV)
+    for lo, hi in ((0, 40), (40, 41)):
+        mask = torch.arange(hi, device=DEV) <= torch.arange(lo, hi, device=DEV)[:, None]
+        got, want = m(ids[:, lo:hi], cache=a), m(ids[:, lo:hi], cache=b, attn_mask=mask)
+        assert got.shape == want.shape and native.pop() == (2, hi - lo) and not native
+        assert float((got - want).norm() / want.norm()) <= 2e-2
 
 
 def test_native_forward_with_unaligned_tensors():
