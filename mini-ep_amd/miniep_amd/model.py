@@ -304,7 +304,7 @@ class GraniteMoeModel:
                 q, k, v = ops.linear(x, proj) if ops.tiled_linear(x, proj) else (F.linear(x, m) for m in proj)
                 o = ops.attention(q, k, v, cos, sin, B, start, kc, vc, scale)
                 h, x = ops.add_norm(h, norm2, eps, F.linear(o, w[k_["wo"]]), rm)
-            moe_out = self._moe_block(layer, x, moe_valid).view(n, H).contiguous()
+            moe_out = self._moe_block(layer, x, moe_valid).view(B, T, H).reshape(n, H).contiguous()
             if moe_out.data_ptr() % 16:                              # a backend's view into something larger
                 moe_out = moe_out.clone()
             if moe_out.dtype != h.dtype:                             # a backend of another dtype: the sum is promoted

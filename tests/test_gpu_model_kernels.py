@@ -221,6 +221,22 @@ def test_backends_of_another_dtype_and_shape(model, backend, layers):
         assert float((got - want).norm() / want.norm()) <= 2e-2
 
 
+def test_backend_with_strided_output():
+    """A backend whose (batch, tokens, hidden) lies tokens first in memory."""
+    cfg = ModelConfig(num_hidden_layers=2, vocab_size=997)
+    m = build_hip_model(cfg, random_weights(cfg, seed=3, dtype=torch.bfloat16, device=DEV))
+    ids = torch.randint(0, cfg.vocab_size, (2, 40), generator=torch.Generator().manual_seed(1)).to(DEV)
+    want = m(ids)
+    inner = m.moe[0].route_and_call
+
+    def tokens_first(*a, **kw):
+        out = inner(*a, **kw)[0].view(2, 40, cfg.hidden_size)
+        return (out.transpose(0, 1).contiguous().transpose(0, 1),)
+    m.moe[0].route_and_call = tokens_first
+    native = _count_native(m)
+    assert torch.equal(m(ids), want) and native == [(2, 40)]
+
+
 def test_native_forward_with_unaligned_tensors():
     """A backend that returns a view off the 16-byte grid, and such a cache:
     accepted, with the results of aligned ones (the cache goes through the torch
