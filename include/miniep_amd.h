@@ -213,15 +213,18 @@ int mep_route_dispatch(const void* x, const void* w_router, const uint8_t* valid
  *   x (N, H)   w_in (n_local, 2I, H)   w_out (n_local, H, I)   y_entries (N*k, H)
  * max_rows >= offsets[n_local] (e.g. N*k) bounds the launch.
  * Supported: H % 256 == 0, I % 128 == 0.
- * With bf16 and I % 256 == 0 both GEMMs run as ONE launch at every size.  At
- * most 256 rows (decode): GEMM-2's workgroups load their weights while GEMM-1
- * runs and start on a 32-row chunk once its GEMM-1 workgroups are done.  Some
- * tens to a few hundred rows per expert: the same by chunks of 64 or 128 rows,
- * the column blocks of a chunk on one XCD.  More: a persistent launch, each
- * XCD works through its share of the row tiles, and a row tile's GEMM-2 tiles
- * start once its GEMM-1 tiles are done.  (I % 256 != 0: one launch up to 1024
- * rows, two above.)  fp32 runs one launch by chunks of 32 or 64 rows if
- * tile_queue is given and large enough, else two.
+ * With bf16 and I % 256 == 0 both GEMMs run as ONE launch.  At most 256 rows
+ * (decode): GEMM-2's workgroups load their weights while GEMM-1 runs and start
+ * on a 32-row chunk once its GEMM-1 workgroups are done.  Some tens to a few
+ * hundred rows per expert: the same by chunks of 64 or 128 rows, the column
+ * blocks of a chunk on one XCD.  More: a persistent launch, each XCD works
+ * through its share of the row tiles, and a row tile's GEMM-2 tiles start once
+ * its GEMM-1 tiles are done.  (Very few experts with a large I, such as one
+ * expert with I 4096 and 2047 rows, fill the chip with row tiles earlier: they
+ * run the first kind up to 1024 rows, and two launches from 1025 to 2048.)
+ * bf16 with I % 256 != 0 runs two launches at every size.  fp32 runs one
+ * launch by chunks of 32 or 64 rows if tile_queue is given and large enough,
+ * else two.
  * tile_queue: tile_queue_ints >= mep_experts_queue_ints(max_rows, n_local)
  * int32 of device memory, zero before the first call; the one-launch kernels
  * keep their schedule there (per-XCD tile counters, per-row-tile or
@@ -295,10 +298,10 @@ int mep_grouped_swiglu_slots(const void* x, int64_t n_tokens, int32_t top_k,
  * :120-128 scatter_combine, :144 the gate multiply) in one call.  Arguments
  * are those of the two calls; max_rows must be n_tokens * top_k (every
  * (token, slot) cell of y_entries), out is (n_tokens, H) like mep_combine's.
- * For bf16, top-8 and at most 256 rows (decode; 1024 if I % 256 != 0) the
- * small-batch launch of both GEMMs ends with the combine: extra workgroups wait (bounded) until
- * every GEMM-2 workgroup's y stores are complete, then sum in slot order, so
- * the results equal the two calls' bit for bit with one launch fewer.  Other
+ * For bf16, I % 256 == 0, top-8 and at most 256 rows (decode) the small-batch
+ * launch of both GEMMs ends with the combine: extra workgroups wait (bounded)
+ * until every GEMM-2 workgroup's y stores are complete, then sum in slot order,
+ * so the results equal the two calls' bit for bit with one launch fewer.  Other
  * sizes and dtypes make the two calls.  Schedule words 12 and 13 of
  * `tile_queue` serve the combine and are left at zero.
  */

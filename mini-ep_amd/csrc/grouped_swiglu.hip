@@ -1845,9 +1845,9 @@ hipError_t launch_skinny_both(const GemmParams& p1, const GemmParams& p2, int64_
 
 // ============================================================================
 // Some tens to a few hundred rows per expert in bf16 (a prompt or a large
-// decode batch), every size in fp32: one workgroup per (chunk of 16 MFC rows of one local
-// expert, column block of 64 act / 128 output columns), both GEMMs in one
-// launch.
+// decode batch), every size in fp32: one workgroup per (chunk of 16 MFC rows of
+// one local expert, column block of 64 act / 128 output columns), both GEMMs in
+// one launch.
 //
 // The tiled kernel's 256 x 256 tiles leave most of the chip idle there (a few
 // row tiles times 4 column tiles on 256 CUs, each a serial chain of a GEMM-1
@@ -1862,9 +1862,9 @@ hipError_t launch_skinny_both(const GemmParams& p1, const GemmParams& p2, int64_
 // the MFMA layout, as the small-batch kernel does, put 16 rows under 16
 // neighbouring lanes: 64 L1 lookups per KiB instead of 8 to 16, which bound
 // the loop once a weight row met more than some 64 rows: 171 us at 4096
-// tokens of the GraniteMoE layer in bf16, 143 so.)  Plain loads and LDS writes, not LDS DMA: the
-// compiler waits for every load in flight before reading LDS that a DMA may
-// have written.)  The K loop is ring_loop (ring_gemm.h).
+// tokens of the GraniteMoE layer in bf16, 143 so.)  Plain loads and LDS writes,
+// not LDS DMA: the compiler waits for every load in flight before reading LDS
+// that a DMA may have written.  The K loop is ring_loop (ring_gemm.h).
 //
 // Chunks are listed by expert and split into 8 contiguous ranges, one per XCD
 // (workgroup b runs on XCD b mod 8): the column blocks of a chunk share its
@@ -2742,6 +2742,10 @@ bool tiled_down(int dtype, int64_t max_rows, int inter) {
 //    1024), 1.09 148 -> 152.  A longer K takes more of the ring's LDS time and
 //    less of the tiles' fixed one; at hidden 4096 that moves the first line too
 //    (0.59 of a round of tiles 153 -> 147, 0.72 165 -> 174, 1.09 241 -> 263).
+// The experts' own rows are not known here, so a line is drawn for skewed and
+// flat routing together: 1700 tokens are 87 -> 68 skewed, but 59 -> 67 with 425
+// rows for every expert (64 row tiles, exactly one round); 128 experts, 2000
+// tokens 115 -> 113 and, with 125 rows each, 108 -> 117.
 int mid_row_frags(int64_t max_rows, int n_local, int hidden, int inter) {
   if (max_rows <= 256) return 0;
   const int64_t cu = device_cu_count();
@@ -2945,8 +2949,9 @@ int down_impl(const char* fn, const void* act, int64_t n_tokens, int32_t top_k, 
                                          inter, y_entries, tile_queue, s);
 }
 
-// Both GEMMs: one launch of the tiled kernel when both would run tiled, else
-// the two launches.
+// Both GEMMs: one launch of the mid-size kernel where its rule takes the rows,
+// of the tiled or the small-batch kernel where both GEMMs would run it, else the
+// two launches.
 // comb: NULL, or a combine that the small-batch launch may end with; then
 // *combined tells whether it did (otherwise the caller runs the combine).
 int grouped_impl(const char* fn, const void* x, int64_t n_tokens, int32_t top_k, const int32_t* perm,

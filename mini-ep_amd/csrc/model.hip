@@ -77,8 +77,13 @@ __device__ __forceinline__ float residual(float h, float delta, float mult) {
 // weight * (h_out / sqrt(mean(h_out^2) + eps)).  One wave per row, the row in
 // registers (NCH 16-byte chunks per lane), so h and delta are read once and
 // h_out and x written once.  Bound by those bytes for many rows (2048 rows of
-// 1024 in bf16: 16.8 MB in 5.8 us), by the launch for a few (8 rows: 3.8 us);
-// as torch operations the same step was nine launches.
+// 1024 in bf16: 16.8 MB in 5.6 us; 16384 rows of 1024, 2048 and 4096: 21, 43 and
+// 102 us, 5.3 to 6.3 TB/s), by the launch for a few (8 rows: 2.4 to 3.8 us);
+// as torch operations the same step was nine launches.  fp32 rows of 1028 to
+// 2048 elements are the slow width: their instance (<F32, 8>) holds part of the
+// row in accumulator registers, moves it back and forth and runs one wave per
+// SIMD (16384 rows of 2048 in 163 us, 3.3 TB/s; of 1024 47 us and 5.7, of 4096
+// 190 us and 5.6).
 // ============================================================================
 constexpr int kNormWaves = 4;
 
@@ -379,9 +384,11 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnParams p) {
 // lane layout.  The sums of the 64 key groups meet in LDS in a fixed order.
 // Two batches of loads are kept in flight, from the first keys (before the
 // rotation) through the softmax's barrier to the last values.  Bound by one
-// CU's loads: 8 sequences of 513 positions, 8 kv heads (16.8 MB of cache):
-// 11.0 us (14.1 with one batch at a time and the sums of 16 lanes through
-// LDS), against 46 us for torch's fp32 attention alone.
+// CU's loads: 8 sequences of 513 positions, 8 kv heads (16.8 MB of cache), two
+// query heads each: 11.0 us (14.1 with one batch at a time and the sums of 16
+// lanes through LDS), against 46 us for torch's fp32 attention alone.  With one
+// and four query heads each (back to back, where two take 9.2): 7.7 and 12.0;
+// one sequence of 4000 positions 25, 30 and 47.
 constexpr int kDecWaves = 16, kDecKeys = 2048;
 
 // The sum over a row of 16 lanes, in every lane: the tree of xor 1, 2, 4, 8 (a
