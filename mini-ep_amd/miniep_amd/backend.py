@@ -158,8 +158,9 @@ class HipEPShareBackend:
         dev = self.w_in.device
         t = self._const.get((size, dev))
         if t is None:
-            nobody = torch.full((size,), -1, dtype=torch.int32)
-            t = self._const[size, dev] = tuple(v.to(dev) for v in (*_world1_tables(size, "cpu"), nobody))
+            table, n_rep, g2l = _world1_tables(size, "cpu")
+            rows = torch.stack([table[:, 0], n_rep, g2l, torch.full_like(n_rep, -1)]).to(dev)    # one copy
+            t = self._const[size, dev] = (rows[0][:, None], *rows[1:])
         return t
 
     def apply_placement(self, placement: Placement, w_in: torch.Tensor, w_out: torch.Tensor):
